@@ -348,7 +348,7 @@ def ring_tick_rate(torch, rows=352, iters=50, seed=5):
     us = t0.elapsed_time(t1) * 1e3 / iters
     multi = lens_h[lens_h >= 2]
     alg = int(len(multi) * hkv * (W * D * 2 * 2 + W * 8) + int(multi.sum()) * hkv * (2 * 512 + 12 * 512))
-    return {"kernel": "ring_attn_mfma_kernel (hsg_ring_attention, min_len 2)", "rows": int(len(multi)),
+    return {"kernel": "ring_attn_kernel (hsg_ring_attention, min_len 2)", "rows": int(len(multi)),
             "tokens": int(multi.sum()), "avg_us": round(us, 2), "alg_bytes_per_launch": alg,
             "achieved_gbs": round(alg / (us * 1e-6) / 1e9, 1), "hbm_frac": round(alg / (us * 1e-6) / 8e12, 3)}
 

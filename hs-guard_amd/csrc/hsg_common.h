@@ -235,6 +235,12 @@ __device__ __forceinline__ int tid_per_site() {
   return t;
 }
 
+// A lane index (or anything derived from it) through an empty asm, for the same use inside a loop
+__device__ __forceinline__ int lane_per_site(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
 // A loaded value through an empty asm: the load then runs where it stands. Without it the compiler sinks a load
 // whose value only one side of a select uses into a branch, with its own wait, at every such select.
 __device__ __forceinline__ float loaded_here(float x) {

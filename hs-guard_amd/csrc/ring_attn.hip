@@ -1,4 +1,5 @@
-// Window-W GQA ring attention (decode, short ticks and 64-token window fills) for gfx950 on MFMA.
+// Window-W GQA attention over a slot's ring and a row's own new keys (short ticks, 64-token window fills), or over
+// the row's own keys alone (whole sequences), for gfx950 on MFMA.
 //
 // Contract: src/hs_guard/engine/ring_attention_kernel.py:7-26 (torch reference) with the v8 kernel's
 // numerics and epilogue (src/hs_guard/engine/fused_kernels.py:288-356): keys in blocks of 32 (the W ring
@@ -6,22 +7,31 @@
 // in the P.V product and summed in fp32, output / sum rounded to bf16, times bf16(sigmoid(gate)); the
 // tick's keys/values are written into the ring in place after every read.
 //
-// Mapping: query rows r = l*G + g (token l, q group g) of one (row, kv head) form 16-row tiles; one
-// workgroup (4 waves) per (row, kv head, query group qg), wave w taking tile 4*qg + w, so a 64-step row
-// spreads over several workgroups that stream the same ring in parallel. The in-place ring write is a second
-// launch (ring_write_kernel) after all reads. All key positions of the ring and the tick go to LDS first, and
-// fills (64 keys) whose positions are outside every query's window of the workgroup are skipped. Per fill the
-// workgroup stages K and V row-major in LDS from registers loaded during the previous fill (each load
-// instruction of a wave reads two whole 512-byte key rows); then each wave runs on v_mfma_f32_16x16x32_bf16
-//   S^T[key, m] = K . Q^T   (A = K rows from LDS, B = Q from registers; 2 key tiles x 8 d-steps)
-// for both of the fill's 32-key softmax blocks first (four independent accumulation chains instead of two:
-// the fill's critical path is this chain, then the softmax, then P.V), and then, block by block,
-//   O^T[d, m] += V^T . P^T  (A = V^T by LDS transpose reads of the row-major V, B = P straight from the S^T
-//                            accumulators: the k order of the product is the lane's own key order, so P
-//                            never leaves registers)
-// The S^T accumulator layout puts one query row per lane column, so the running max / sum and the O^T
-// rescale are per-lane scalars plus a 2-step butterfly (lane xor 16, 32).
+// Query rows r = l*G + g (token l, q group g) of one (row, kv head) form 16-row tiles, and a workgroup of 4 waves takes
+// a group of 4 tiles. Both paths below run, per 32 keys, on v_mfma_f32_16x16x32_bf16,
+//   S^T[key, m] = K . Q^T
+//   O^T[d, m] += V^T . P^T   (A = V^T by LDS transpose reads of row-major V, B = P straight from the S^T accumulators:
+//                             the k order of the product is the lane's own key order, so P never leaves registers)
+// The S^T accumulator layout puts one query row per lane column, so maxima, sums and the O^T rescale are per-lane
+// scalars. The in-place ring write is a second launch (ring_write_kernel) after all reads.
+//
+// attend_group (2 to 4 tiles): wave w takes tile w, and the keys pass through LDS 64 at a time for all waves, loaded
+// into registers a fill ahead. The LDS reads of every wave's whole fill (256 KB per fill of a full group) bound it.
+// attend_tile (one tile: a row of up to 16 / G tokens, or a longer row's last tile): one wave would do all the work, so
+// the waves split the KEYS instead: of the tile's key blocks (the ring's in column order, then the new keys' from the
+// first one it sees), wave w takes blocks w, w + 4, ..., at most SLOTS of them, its keys going straight from global
+// memory into operand registers. Two phases, as in the decode kernel: every score and block maximum first; then, the
+// reference's running max after block b being the prefix maximum m_b of the block maxima, each block's probabilities
+// exp(s - m_b) in bf16 times its values, a wave chaining its blocks by exp(m_prev - m_b) and the waves' partial sums
+// meeting in LDS with weights exp(m_last - m_final). No workgroup barrier inside the phases, and unconditional loads (a
+// block the tile does not see reads the row's own first new keys): under branches they were waited for at once.
+// Measured (W = 512, 16 q / 4 kv heads), with every tile on attend_group before and now:
+// 72 padded rows of 2 to 64 steps 147 -> 92 us (49 us of it whole groups past their rows' lengths, which ran their
+// keys), 64 rows of 4 steps 41.6 -> 28.0 us, one such row 34.9 -> 21.6 us. Splitting the keys of longer rows' tiles too
+// reads K and V once per tile instead of once per group: 72 rows of 64 steps 264 us against 165.
 #include <math.h>
+
+#include <type_traits>
 
 #include "hsg_common.h"
 
@@ -29,20 +39,23 @@ namespace hsg {
 namespace {
 
 constexpr int D = 256;
-constexpr int NW = 4;
+constexpr int NW = 4;                  // waves per workgroup
+constexpr int TQ = 16;                 // query rows of a tile
 constexpr int KB = 32;                 // keys per softmax block (the reference's BN)
-constexpr int SB = 2;                  // softmax blocks staged per LDS fill
-constexpr int KF = KB * SB;            // keys per LDS fill
 constexpr int W_MAX = 512;
 constexpr int LB_MAX = 64;
-constexpr int KS_STRIDE = D + 8;       // bf16 per K or V row in LDS (16-byte pad)
+constexpr int SLOTS = 5;               // attend_tile: key blocks of a wave: W / 32 ring blocks and 2 of new keys, or the 18 that the
+                                       // window of a tile's up to 16 tokens can touch, over 4 waves
+constexpr int KV_LOADS = 2 * D / KB;   // 16-byte K loads of a wave per block (and V loads)
+constexpr int KF = 2 * KB;             // attend_group: keys per LDS fill
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) int i32x4;
 
 struct RingParams {
   const uint16_t* q; int64_t q_sn, q_sl, q_sh, q_sg;
-  uint16_t* ring_k; uint16_t* ring_v; int64_t ring_rows; int W;
+  uint16_t* ring_k; uint16_t* ring_v; int64_t ring_rows; int W;   // ring_k NULL: the row's own keys only
   const uint16_t* new_k; int64_t nk_sn, nk_sl, nk_sh;
   const uint16_t* new_v; int64_t nv_sn, nv_sl, nv_sh;
   const uint16_t* gate; int64_t g_sn, g_sl, g_sh, g_sg, g_off;
@@ -52,286 +65,592 @@ struct RingParams {
   float scale;
   int write_ring;
   int min_len;
-  int qgroups;      // workgroups per (row, kv head): groups of NW 16-row query tiles
+  int pairs;        // rows x kv heads
+  int qgroups;      // workgroups (groups of NW tiles) per (row, kv head)
   uint16_t* out; int64_t o_sn, o_sl, o_sh, o_sg;
 };
 
-__device__ __forceinline__ bf16x8 as_bf16x8(uint4 w) { return __builtin_bit_cast(bf16x8, w); }
+__device__ __forceinline__ bf16x8 as_bf16x8(u32x4 w) { return __builtin_bit_cast(bf16x8, w); }
 
-constexpr int KP_NONE = -(1 << 30);
+constexpr int KP_NONE = -(1 << 30);    // an empty ring column
+constexpr int KP_FAR = 1 << 29;        // clamp of a position relative to the row's start
 
 // exp of the softmax argument on the hardware exp2 (v_exp_f32): exp(x) = 2^(x log2 e). The reference kernel
 // takes tl.exp, Triton's fast exponential, here too (src/hs_guard/engine/fused_kernels.py:318-319,335-336).
 __device__ __forceinline__ float exp_fast(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
 
-typedef __attribute__((ext_vector_type(4))) short s16x4_;
-
 // LDS transpose read (ds_read_b64_tr_b16): within each group of 16 lanes, lane 4q + e receives element e of
 // the 4-element (8-byte) vectors addressed by lanes q, q + 4, q + 8, q + 12 of its group. With V row-major
 // ([key][dim]), lane s of a group addressing key row r0 + (s >> 2), dims c0 + 4 (s & 3) .. +3 receives dim
 // c0 + s of keys r0 .. r0 + 3: the A operand of O^T += V^T . P^T.
-__device__ __forceinline__ uint2 ld_tr4(const uint16_t* p) {
-  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_*)(p)));
+typedef __attribute__((ext_vector_type(4))) short s16x4_;
+__device__ __forceinline__ u32x2 ld_tr4(const uint16_t* p) {
+  return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4_*)(p)));
 }
 
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+// Eight of them, of four dim tiles (LDS byte addresses a0 .. a3) and key rows 0 and 16, with one wait: the compiler
+// issues its builtin one product ahead, an LDS round trip per product.
+__device__ __forceinline__ void ld_tr_4x2(u32x2 (&v)[4][2], uint32_t a0, uint32_t a1, uint32_t a2, uint32_t a3) {
+  static_assert(16 * D * 2 == 8192, "the offset below is 16 rows");
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:8192\n\t"
+      "ds_read_b64_tr_b16 %2, %9\n\t"
+      "ds_read_b64_tr_b16 %3, %9 offset:8192\n\t"
+      "ds_read_b64_tr_b16 %4, %10\n\t"
+      "ds_read_b64_tr_b16 %5, %10 offset:8192\n\t"
+      "ds_read_b64_tr_b16 %6, %11\n\t"
+      "ds_read_b64_tr_b16 %7, %11 offset:8192\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0][0]), "=&v"(v[0][1]), "=&v"(v[1][0]), "=&v"(v[1][1]), "=&v"(v[2][0]), "=&v"(v[2][1]), "=&v"(v[3][0]),
+        "=&v"(v[3][1])
+      : "v"(a0), "v"(a1), "v"(a2), "v"(a3)
+      : "memory");
 }
 
-__global__ __launch_bounds__(NW * 64, 2) void ring_attn_mfma_kernel(const RingParams p) {
-  __shared__ __align__(16) uint16_t Ks[KF * KS_STRIDE];
-  __shared__ __align__(16) uint16_t Vs[KF * KS_STRIDE];
-  // key position - start (the row's first new position), clamped to [-2W-1, 2W+1]; KP_NONE for an empty
-  // column: ring columns [0, W), then the tick's new keys
-  __shared__ int kp_all[W_MAX + LB_MAX];
-  __shared__ uint32_t wave_mask[NW];           // per wave: bit f set if fill f has a key visible to the group
+// byte offset of an LDS pointer
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
 
+// Row pieces of 16 bytes in LDS: rows of 512 bytes whose 32-byte pairs of pieces are permuted, pair c of row r at
+// c ^ (r & 15). A transpose read (16 rows x 32 bytes) and a row read of 16 rows (16 bytes at each of 4 offsets) then
+// spread over all banks evenly. Element offset of piece `pc` of row r:
+__device__ __forceinline__ int piece_at(int r, int pc) { return r * D + 8 * (2 * ((pc >> 1) ^ (r & 15)) + (pc & 1)); }
+
+// The (row, kv head) of a workgroup: element pointers of its first token's query, new key, new value, gate and output
+struct Row {
+  const uint16_t* qrow;
+  const uint16_t* krow;
+  const uint16_t* vrow;
+  const uint16_t* grow;   // NULL: no gate
+  uint16_t* orow;
+  const int64_t* ring_pos;
+  int64_t slot, start, ring_base;
+  int len, steps;         // valid tokens and output steps (padded rows: up to lb, the rest zeros)
+  int RB;                 // ring blocks
+};
+
+struct SplitLds {
+  uint16_t Vs[NW][KB * D];       // per wave: one block of V (piece_at), then the wave's O
+  int kp_s[NW][W_MAX / NW];      // key position - start of the wave's ring columns; KP_NONE for an empty one
+  float bm_s[TQ][NW * SLOTS];    // block maxima of each query row, -inf where nothing is seen
+  float l_s[NW][TQ];             // per wave: weighted sum of each query row
+};
+
+struct GroupLds {
+  uint16_t Ks[KF * D], Vs[KF * D];   // the fill's keys and values (piece_at)
+  int kp[W_MAX];                     // key position - start of the ring columns; KP_NONE for an empty one
+  uint32_t mask[NW];                 // per wave: bit f set if the ring's fill f has a key visible to the group
+};
+
+// ---------------------------------------------------------------------------------------------------------
+// A group of up to NW tiles: wave w takes tile w, keys in fills of KF through LDS.
+// ---------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ void attend_group(const RingParams& p, const Row& ro, int r_lo, GroupLds& lds, int lane, int wave) {
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  // query group slowest: consecutive workgroups (which the dispatcher deals round-robin over the 8 XCDs)
-  // take consecutive (row, kv head) pairs, so the live workgroups of a short-row tick spread over all XCDs
-  const int n_pairs = gridDim.x / p.qgroups;
-  const int qg = blockIdx.x / n_pairs;
-  const int nh = blockIdx.x - qg * n_pairs;
-  const int n = nh / p.hkv;
-  const int h = nh - n * p.hkv;
-  const int64_t slot = p.slots[n];
-  const int64_t start = p.starts[n];
-  int64_t len = p.lens[n];
-  const bool padded = p.offsets == nullptr;
-  if (slot < 0 || slot >= p.ring_rows || len < 0 || len > (padded ? LB_MAX : p.lb)) len = 0;  // rejected row
-  if (padded && len > p.lb) len = p.lb;
-  if (!padded && len < p.min_len) return;              // left to another kernel (single-step rows: split-K)
-  const int steps = padded ? p.lb : (int)len;          // output steps written for this row
-  const int64_t base_tok = padded ? 0 : p.offsets[n];
-  const int64_t q_row = padded ? n * p.q_sn : base_tok * p.q_sl;
-  const int64_t nk_row = padded ? n * p.nk_sn : base_tok * p.nk_sl;
-  const int64_t nv_row = padded ? n * p.nv_sn : base_tok * p.nv_sl;
-  const int64_t g_row = padded ? n * p.g_sn : base_tok * p.g_sl;
-  const int64_t o_row = padded ? n * p.o_sn : base_tok * p.o_sl;
-  const int W = p.W;
-  const int G = p.G;
-  const int64_t ring_base = ((slot * p.hkv + h) * (int64_t)(W + 1)) * D;
-  const int64_t* rpos = p.ring_pos + slot * (int64_t)(W + 1);
-  const int M = G * steps;                              // query rows of this (row, kv head)
-  const int QT = (M + 15) >> 4;                         // 16-row tiles
-  const int q4 = lane >> 4;                             // lane group: keys 4*q4 .., dims 8*q4 ..
-  const int mcol = lane & 15;                           // the lane's query row within its tile
-  const int n_ring_blocks = len > 0 ? W / KB : 0;
-  const int n_new_blocks = (int)((len + KB - 1) / KB);
-
-  if (qg * NW < QT) {
-    const int tile = qg * NW + wave;
-    const bool has_tile = tile < QT;
-    // ---- this lane's query row ----
-    const int r = tile * 16 + mcol;
-    const int l_tok = r / G;
-    const int gq = r - l_tok * G;
-    const bool row_ok = has_tile && r < M;
-    const bool q_valid = row_ok && l_tok < len;
-    bf16x8 qb[D / 32];
+  const int q4 = lane >> 4;                            // lane group: keys 4*q4 .., dims 8*q4 ..
+  const int mcol = lane & 15;                          // the lane's query row within its tile
+  const int W = p.W, G = p.G, RB = ro.RB, len = ro.len;
+  const int M = G * ro.steps, Mv = G * len;
+  const int r = r_lo + TQ * wave + mcol;
+  const bool has_tile = r_lo + TQ * wave < Mv;
+  const int rq = min(r, Mv - 1);                       // past the valid rows: the last one again, stored as zeros
+  const int l_tok = rq / G;
+  const int gq = rq - l_tok * G;
+  bf16x8 qb[D / 32];
 #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      uint4 w = make_uint4(0u, 0u, 0u, 0u);
-      if (q_valid)
-        w = *reinterpret_cast<const uint4*>(p.q + q_row + l_tok * p.q_sl + h * p.q_sh + gq * p.q_sg + 32 * ks + 8 * q4);
-      qb[ks] = as_bf16x8(w);
+  for (int ks = 0; ks < D / 32; ++ks)
+    qb[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(ro.qrow + l_tok * p.q_sl + gq * p.q_sg + 32 * ks + 8 * q4));
+  // tokens of the group (all waves)
+  const int l_lo = r_lo / G;
+  const int l_hi = (min(r_lo + NW * TQ, Mv) - 1) / G;
+  // Fills: the ring's, then those of the new keys the group sees (from new key j_lo). Every ring position goes to
+  // LDS in one round trip, and the ring's fills that no query of the group sees are skipped.
+  const int n_ring = (RB + 1) / 2;
+  const int j_lo = max(0, l_lo - W + 1) / KF * KF;
+  const int n_fills = n_ring + (l_hi - j_lo) / KF + 1;
+  uint32_t my_mask = 0u;
+  for (int c = tid; c < RB * KB; c += NW * 64) {
+    const int64_t kpos = ro.ring_pos[c];
+    const int64_t d = kpos - ro.start;
+    int rel = (int)(d < -KP_FAR ? -KP_FAR : d > KP_FAR ? KP_FAR : d);
+    if (kpos < 0) rel = KP_NONE;
+    lds.kp[c] = rel;
+    if (rel <= l_hi && rel > l_lo - W) my_mask |= 1u << (c / KF);
+  }
+  for (int o = 1; o < 64; o <<= 1) my_mask |= (uint32_t)__shfl_xor((int)my_mask, o, 64);
+  if (lane == 0) lds.mask[wave] = my_mask;
+  __syncthreads();
+  const uint32_t ring_mask =
+      __builtin_amdgcn_readfirstlane(lds.mask[0] | lds.mask[1] | lds.mask[2] | lds.mask[3]);
+  auto next_fill = [&](int f) {   // first fill after f with a visible key (n_fills if none)
+    ++f;
+    if (f < n_ring) {
+      const uint32_t rest = ring_mask >> f;
+      f = rest ? f + __builtin_ctz(rest) : n_ring;
     }
-    // positions covered by this query group (all waves), for skipping whole key blocks
-    const int r_lo = qg * NW * 16;
-    const int r_hi = min(M, (qg + 1) * NW * 16) - 1;
-    const int64_t qpos_lo = start + r_lo / G;
-    const int64_t qpos_hi = start + min((int64_t)(r_hi / G), len - 1);
-    float m_run = -INFINITY, l_run = 0.f;
-    f32x4 O[D / 16];
+    return f;
+  };
+  // Thread t holds piece t % 32 of keys t / 32 + 8 i (i < 8) of K and of V: every load instruction of a wave reads
+  // two whole 512-byte key rows. Keys past the fill's valid ones repeat the last one and are zeroed when staged.
+  u32x4 kr[8], vr[8];
+  auto prefetch = [&](int f) __attribute__((always_inline)) {
+    const bool ring = f < n_ring;
+    const int c0 = ring ? f * KF : j_lo + (f - n_ring) * KF;
+    const int last = ring ? min(KF, RB * KB - c0) - 1 : min(KF, len - c0) - 1;
+    const uint16_t* kb = (ring ? p.ring_k + ro.ring_base + c0 * D : ro.krow + c0 * p.nk_sl);
+    const uint16_t* vb = (ring ? p.ring_v + ro.ring_base + c0 * D : ro.vrow + c0 * p.nv_sl);
+    const int64_t kst = ring ? D : p.nk_sl, vst = ring ? D : p.nv_sl;
+    const int tl = lane_per_site(tid);
 #pragma unroll
-    for (int t = 0; t < D / 16; ++t) O[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-    // Fills: n_ring_fills of up to SB ring blocks, then the new-key blocks in fills of up to SB. Every key
-    // position goes to LDS in one round trip and the fills no query of this group sees are skipped; the
-    // next visible fill's K and V are loaded into registers while the current one is computed.
-    const int n_ring_fills = (n_ring_blocks + SB - 1) / SB;
-    const int n_fills = n_ring_fills + (n_new_blocks + SB - 1) / SB;
-    uint32_t my_mask = 0u;
-    for (int c = tid; c < W + n_new_blocks * KB; c += NW * 64) {
-      int64_t kpos;
-      int f;
-      if (c < W) {
-        kpos = c < n_ring_blocks * KB ? rpos[c] : -1;
-        f = c / KF;
-      } else {
-        const int j = c - W;
-        kpos = j < len ? start + j : -1;
-        f = n_ring_fills + j / KF;
+    for (int i = 0; i < 8; ++i) {
+      const int key = min((tl >> 5) + 8 * i, last);
+      // nontemporal, as the decode kernel's ring reads: a step's mixed tick ran 0.35 % faster (two A/B pairs
+      // on MI355X), the rings no longer displacing what the neighbouring kernels reuse
+      kr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(kb + key * kst + 8 * (tl & 31)));
+      vr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vb + key * vst + 8 * (tl & 31)));
+    }
+  };
+  float m_run = -INFINITY, l_run = 0.f;   // l_run: this lane's keys only
+  f32x4 O[D / 16];
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t) O[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+  const int rx = 4 * q4 + (mcol >> 2);    // the lane's key row of a transpose read (and + 16)
+  int fcur = next_fill(-1);
+  prefetch(fcur);
+  for (; fcur < n_fills; fcur = next_fill(fcur)) {
+    const bool ring = fcur < n_ring;
+    const int c0 = ring ? fcur * KF : j_lo + (fcur - n_ring) * KF;
+    const int nkeys = ring ? min(KF, RB * KB - c0) : min(KF, len - c0);
+    __syncthreads();  // the previous fill's LDS reads are done
+    {
+      const int tl = lane_per_site(tid);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = (tl >> 5) + 8 * i;
+        const bool live = key < nkeys;
+        const int o = piece_at(key, tl & 31);
+        *reinterpret_cast<u32x4*>(&lds.Ks[o]) = live ? kr[i] : (u32x4){0u, 0u, 0u, 0u};
+        *reinterpret_cast<u32x4*>(&lds.Vs[o]) = live ? vr[i] : (u32x4){0u, 0u, 0u, 0u};
       }
-      const int64_t rel = kpos - start;
-      kp_all[c] = kpos < 0 ? KP_NONE : (int)(rel < -2 * W - 1 ? -2 * W - 1 : rel > 2 * W + 1 ? 2 * W + 1 : rel);
-      if (kpos >= 0 && kpos <= qpos_hi && kpos > qpos_lo - W) my_mask |= 1u << f;
     }
-    // OR over the workgroup: wave butterfly, then one word per wave through LDS
-    for (int o = 1; o < 64; o <<= 1) my_mask |= (uint32_t)__shfl_xor((int)my_mask, o, 64);
-    if (lane == 0) wave_mask[wave] = my_mask;
+    const int fnext = next_fill(fcur);
+    if (fnext < n_fills) prefetch(fnext);
     __syncthreads();
-    const uint32_t fmask = wave_mask[0] | wave_mask[1] | wave_mask[2] | wave_mask[3];
-    auto fill_geom = [&](int f, bool& is_ring, int& c0, int& nb) {
-      is_ring = f < n_ring_fills;
-      const int b0 = is_ring ? f * SB : (f - n_ring_fills) * SB;
-      nb = is_ring ? min(SB, n_ring_blocks - b0) : min(SB, n_new_blocks - b0);
-      c0 = b0 * KB;   // ring column or new-key index of the fill's first key
-    };
-    // Thread t holds dims 8 (t % 32) .. +7 of keys t / 32 + 8 i (i < 8) of K and of V: every load instruction
-    // of a wave reads two whole 512-byte key rows. Keys past the fill's valid ones load a clamped valid row
-    // and are zeroed when staged.
-    u32x4 kr[8], vr[8];
-    auto prefetch = [&](int f) {
-      bool is_ring; int c0, nb;
-      fill_geom(f, is_ring, c0, nb);
-      const int nkeys = nb * KB;
-      const int dcol = 8 * (tid & 31);
+    if (!has_tile) continue;
+    // ---- S^T = K . Q^T for both softmax blocks of the fill first ----
+    f32x4 S[2][2];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int key = (tid >> 5) + 8 * i;
-        const uint16_t* ksrc;
-        const uint16_t* vsrc;
-        if (is_ring) {
-          const int64_t off = ring_base + (int64_t)(c0 + min(key, nkeys - 1)) * D + dcol;
-          ksrc = p.ring_k + off;
-          vsrc = p.ring_v + off;
-        } else {
-          const int64_t j = min(c0 + key, (int)len - 1);
-          ksrc = p.new_k + nk_row + j * p.nk_sl + h * p.nk_sh + dcol;
-          vsrc = p.new_v + nv_row + j * p.nv_sl + h * p.nv_sh + dcol;
-        }
-        // nontemporal, as the decode kernel's ring reads: a step's mixed tick ran 0.35 % faster (two A/B pairs
-        // on MI355X), the rings no longer displacing what the neighbouring kernels reuse
-        kr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(ksrc));
-        vr[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(vsrc));
-      }
-    };
-    auto next_fill = [&](int f) {   // first visible fill after f (n_fills if none)
-      const uint32_t rest = f + 1 < 32 ? (fmask >> (f + 1)) : 0u;
-      return rest ? f + 1 + __builtin_ctz(rest) : n_fills;
-    };
-    int fcur = next_fill(-1);
-    if (fcur < n_fills) prefetch(fcur);
-    for (; fcur < n_fills; fcur = next_fill(fcur)) {
-      bool is_ring; int c0, nb;
-      fill_geom(fcur, is_ring, c0, nb);
-      const int nkeys = nb * KB;
-      const int kbase = is_ring ? c0 : W + c0;   // the fill's first key in kp_all
-      __syncthreads();  // the previous fill's LDS reads are done
+    for (int sb = 0; sb < 2; ++sb) {
+      S[sb][0] = S[sb][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int key = (tid >> 5) + 8 * i;
-        const bool live = key < nkeys && (is_ring || c0 + key < len);
-        const int o = key * KS_STRIDE + 8 * (tid & 31);
-        *reinterpret_cast<u32x4*>(&Ks[o]) = live ? kr[i] : (u32x4){0u, 0u, 0u, 0u};
-        *reinterpret_cast<u32x4*>(&Vs[o]) = live ? vr[i] : (u32x4){0u, 0u, 0u, 0u};
-      }
-      const int fnext = next_fill(fcur);
-      if (fnext < n_fills) prefetch(fnext);
-      __syncthreads();
-      if (!has_tile) continue;
-      // ---- S^T = K . Q^T for both softmax blocks of the fill first (four independent accumulation chains) ----
-      f32x4 Sall[SB][2];
+      for (int ks = 0; ks < D / 32; ++ks)
 #pragma unroll
-      for (int sb = 0; sb < SB; ++sb) {
-        if (sb < nb) {
-#pragma unroll
-          for (int kt = 0; kt < 2; ++kt) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            const uint16_t* krow = &Ks[(sb * KB + 16 * kt + mcol) * KS_STRIDE + 8 * q4];
-#pragma unroll
-            for (int ks = 0; ks < D / 32; ++ks) {
-              const bf16x8 a = as_bf16x8(*reinterpret_cast<const uint4*>(krow + 32 * ks));
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qb[ks], acc, 0, 0, 0);
-            }
-            Sall[sb][kt] = acc;
-          }
-        }
-      }
-#pragma unroll
-      for (int sb = 0; sb < SB; ++sb) {
-        if (sb >= nb) break;
-        const int kb = sb * KB;   // softmax block within the fill
-        const f32x4 S[2] = {Sall[sb][0], Sall[sb][1]};
-        // ---- mask, online softmax over the block (the lane's 8 keys: 4 q4 + i and 16 + 4 q4 + i) ----
-        float s[8];
-        float bmax = -INFINITY;
-#pragma unroll
-        for (int kt = 0; kt < 2; ++kt) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int rel = kp_all[kbase + kb + 16 * kt + 4 * q4 + i];
-            const bool ok = q_valid && rel <= l_tok && rel > l_tok - W;   // KP_NONE fails the second
-            const float v = ok ? S[kt][i] * p.scale : -INFINITY;
-            s[4 * kt + i] = v;
-            bmax = fmaxf(bmax, v);
-          }
-        }
-        bmax = max_pair32(max_pair16(bmax));   // over q4 (lane xor 16, 32)
-        const float m_new = fmaxf(m_run, bmax);
-        const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-        const float alpha = exp_fast(m_run - m_safe);   // exp(-inf) = 0 before the first visible key
-        float psum = 0.f;
-        uint32_t pk[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float p0 = exp_fast(s[2 * i] - m_safe);
-          const float p1 = exp_fast(s[2 * i + 1] - m_safe);
-          psum += p0 + p1;
-          pk[i] = pack_bf16(p0, p1);
-        }
-        psum = add_xor32(add_xor16(psum));
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        const bf16x8 pb = as_bf16x8(make_uint4(pk[0], pk[1], pk[2], pk[3]));
-        // ---- O^T += V^T . P^T over the block's 32 keys, in the lane's key order ----
-#pragma unroll
-        for (int t = 0; t < D / 16; ++t) {
-          // dim 16 t + mcol of keys kb + 4 q4 .. +3 and kb + 16 + 4 q4 .. +3 (the lane's key order of P)
-          const uint16_t* vsrc = &Vs[(kb + 4 * q4 + (mcol >> 2)) * KS_STRIDE + 16 * t + 4 * (mcol & 3)];
-          const uint2 lo = ld_tr4(vsrc);
-          const uint2 hi = ld_tr4(vsrc + 16 * KS_STRIDE);
-          const bf16x8 a = as_bf16x8(make_uint4(lo.x, lo.y, hi.x, hi.y));
-          f32x4 o = O[t];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] *= alpha;
-          O[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, o, 0, 0, 0);
-        }
-      }
+        for (int kt = 0; kt < 2; ++kt)
+          S[sb][kt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              as_bf16x8(*reinterpret_cast<const u32x4*>(&lds.Ks[piece_at(sb * KB + 16 * kt + mcol, 4 * ks + q4)])), qb[ks],
+              S[sb][kt], 0, 0, 0);
     }
-    // ---- normalise, gate, store this lane's row: dims 16 t + 4 q4 + i ----
-    if (row_ok) {
-      uint16_t* dst = p.out + o_row + l_tok * p.o_sl + h * p.o_sh + gq * p.o_sg;
-      const uint16_t* gsrc = p.gate ? p.gate + g_row + l_tok * p.g_sl + h * p.g_sh + gq * p.g_sg + p.g_off : nullptr;
-      // every gate piece is loaded before the first store: out may alias gate as far as the compiler knows, so a
-      // load after a store waits for it, and the 16 pieces were 16 serial memory round trips at the end of each
-      // workgroup
-      uint2 gw[D / 16];
-      if (gsrc) {
 #pragma unroll
-        for (int t = 0; t < D / 16; ++t) gw[t] = *reinterpret_cast<const uint2*>(gsrc + 16 * t + 4 * q4);
+    for (int sb = 0; sb < 2; ++sb) {
+      if (sb * KB >= nkeys) break;
+      // ---- mask, online softmax over the block (the lane's 8 keys: 4 q4 + i and 16 + 4 q4 + i) ----
+      float s[8];
+      float bmax = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt) {
+        i32x4 rel;
+        const int at = c0 + sb * KB + 16 * kt + 4 * q4;
+        if (ring) {
+          rel = *reinterpret_cast<const i32x4*>(&lds.kp[at]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) rel[i] = at + i;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {   // KP_NONE fails the second test, a new key past the row's end the first
+          const bool ok = (rel[i] <= l_tok) & (rel[i] > l_tok - W);
+          const float v = ok ? S[sb][kt][i] * p.scale : -INFINITY;
+          s[4 * kt + i] = v;
+          bmax = fmaxf(bmax, v);
+        }
       }
+      bmax = max_pair32(max_pair16(bmax));   // over q4 (lane xor 16, 32)
+      const float m_new = fmaxf(m_run, bmax);
+      const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = exp_fast(m_run - m_safe);   // exp(-inf) = 0 before the first visible key
+      l_run *= alpha;
+      m_run = m_new;
+      u32x4 pk;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float p0 = exp_fast(s[2 * i] - m_safe);
+        const float p1 = exp_fast(s[2 * i + 1] - m_safe);
+        l_run += p0 + p1;
+        pk[i] = pack_bf16x2(p0, p1);
+      }
+      const bf16x8 pb = as_bf16x8(pk);
+      // ---- O^T += V^T . P^T over the block's 32 keys, in the lane's key order ----
 #pragma unroll
       for (int t = 0; t < D / 16; ++t) {
-        const int d = 16 * t + 4 * q4;
-        float y[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) y[i] = l_run > 0.f ? rbf(O[t][i] / l_run) : 0.f;
-        if (gsrc) {
-          float gt[4];
-          unpack2(gw[t].x, gt[0], gt[1]);
-          unpack2(gw[t].y, gt[2], gt[3]);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) y[i] = y[i] * rbf(1.0f / (1.0f + expf(-gt[i])));
-        }
-        store4_bf16(dst + d, y);
+        const uint16_t* vsrc = &lds.Vs[(sb * KB + rx) * D + 4 * (mcol & 3) + 16 * (t ^ rx)];
+        const u32x2 lo = ld_tr4(vsrc);
+        const u32x2 hi = ld_tr4(vsrc + 16 * D);
+        O[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8((u32x4){lo[0], lo[1], hi[0], hi[1]}), pb, O[t] * alpha, 0,
+                                                       0, 0);
       }
     }
   }
+  // ---- normalise, gate, store this lane's row: dims 16 t + 4 q4 + i ----
+  if (r < M) {
+    l_run = add_xor32(add_xor16(l_run));
+    const bool valid = r < Mv && l_run > 0.f;
+    const int l_out = r / G;
+    const int g_out = r - l_out * G;
+    uint16_t* dst = ro.orow + l_out * p.o_sl + g_out * p.o_sg + 4 * q4;
+    const uint16_t* gsrc = ro.grow ? ro.grow + l_out * p.g_sl + g_out * p.g_sg + 4 * q4 : nullptr;
+    // every gate piece is loaded before the first store: out may alias gate as far as the compiler knows, so a
+    // load after a store waits for it, and the 16 pieces were 16 serial memory round trips at the end of each
+    // workgroup
+    u32x2 gw[D / 16];
+    if (gsrc) {
+#pragma unroll
+      for (int t = 0; t < D / 16; ++t) gw[t] = *reinterpret_cast<const u32x2*>(gsrc + 16 * t);
+    }
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(O[t][i] / l_run) : 0.f;
+      if (gsrc) {
+        float gt[4];
+        unpack2(gw[t][0], gt[0], gt[1]);
+        unpack2(gw[t][1], gt[2], gt[3]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = y[i] * rbf(1.0f / (1.0f + expf(-gt[i])));
+      }
+      store4_bf16(dst + 16 * t, y);
+    }
+  }
+}
 
+// ---------------------------------------------------------------------------------------------------------
+// One tile (16 query rows): the four waves split its keys.
+// ---------------------------------------------------------------------------------------------------------
+__device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, int r_lo, SplitLds& lds, int lane, int wave) {
+  auto& Vs = lds.Vs;
+  auto& kp_s = lds.kp_s;
+  auto& bm_s = lds.bm_s;
+  auto& l_s = lds.l_s;
+  const int tid = threadIdx.x;
+  const int q4 = lane >> 4;                            // lane group: keys 4*q4 .., dims 8*q4 ..
+  const int mcol = lane & 15;                          // the lane's query row within its tile
+  const int W = p.W, G = p.G, RB = ro.RB, len = ro.len;
+  const int M = G * ro.steps, Mv = G * len;
+  uint16_t* const vlds = Vs[wave];
+  // ---- this lane's query row and the tile's token range ----
+  const int rq = min(r_lo + mcol, Mv - 1);   // past the valid rows: the last one again, never stored
+  const int l_tok = rq / G;
+  const int gq = rq - l_tok * G;
+  const int l_lo = r_lo / G;
+  const int l_hi = (min(r_lo + TQ, Mv) - 1) / G;
+  bf16x8 qb[D / 32];
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks)
+    qb[ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(ro.qrow + l_tok * p.q_sl + gq * p.q_sg + 32 * ks + 8 * q4));
+
+  // ---- positions of the wave's ring blocks w + 4 i; bit i: a key of block i is visible / all are to all ----
+  uint32_t any = 0u, full = 0u;
+  if (RB) {
+    int64_t kpos[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      kpos[u] = ro.ring_pos[min(wave + NW * (2 * u + (lane >> 5)), RB - 1) * KB + (lane & 31)];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t d = kpos[u] - ro.start;
+      int rel = (int)(d < -KP_FAR ? -KP_FAR : d > KP_FAR ? KP_FAR : d);
+      if (kpos[u] < 0 || wave + NW * (2 * u + (lane >> 5)) >= RB) rel = KP_NONE;
+      kp_s[wave][64 * u + lane] = rel;
+      const uint64_t va = __ballot(rel <= l_hi && rel > l_lo - W);
+      const uint64_t vf = __ballot(rel <= l_lo && rel > l_hi - W);
+      any |= ((uint32_t)va ? 1u : 0u) << (2 * u) | ((uint32_t)(va >> 32) ? 1u : 0u) << (2 * u + 1);
+      full |= ((uint32_t)vf == ~0u ? 1u : 0u) << (2 * u) | ((uint32_t)(vf >> 32) == ~0u ? 1u : 0u) << (2 * u + 1);
+    }
+    any = __builtin_amdgcn_readfirstlane(any);
+    full = __builtin_amdgcn_readfirstlane(full);
+  }
+  // the new-key blocks the tile sees: cb0 .. cb1
+  const int cb0 = max(0, l_lo - W + 1) / KB;
+  const int cb1 = l_hi / KB;
+  // the wave's blocks (ordinals wave + 4 i): bit i of seen / full as of any / full, over ring and new blocks
+  uint32_t seen = any;
+#pragma unroll
+  for (int i = 0; i < SLOTS; ++i) {
+    const int c = cb0 + wave + NW * i - RB;
+    if (wave + NW * i >= RB) {
+      seen |= (c <= cb1 ? 1u : 0u) << i;
+      full |= (c * KB + KB - 1 <= l_lo && c * KB > l_hi - W ? 1u : 0u) << i;
+    }
+  }
+  // first row, row stride and last valid row of block i's keys or values; a block nobody sees reads the row's
+  // first new keys
+  auto rows_of = [&](int i, const uint16_t* ring, const uint16_t* fresh, int64_t stride, int64_t& st, int& last) {
+    const int o = wave + NW * i;
+    const bool live = (seen >> i & 1u) != 0;
+    const bool from_ring = live && o < RB;
+    const int j0 = live && !from_ring ? (cb0 + o - RB) * KB : 0;
+    st = from_ring ? D : stride;
+    last = from_ring ? KB - 1 : min(KB - 1, len - 1 - j0);
+    return from_ring ? ring + ro.ring_base + o * (KB * D) : fresh + j0 * stride;
+  };
+  auto load_keys = [&](int i, u32x4 (&ka)[2][D / 32]) __attribute__((always_inline)) {
+    int64_t st;
+    int last;
+    const uint16_t* base = rows_of(i, p.ring_k, ro.krow, p.nk_sl, st, last);
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+      const uint16_t* src = base + min(16 * kt + mcol, last) * st + 8 * q4;
+#pragma unroll
+      for (int ks = 0; ks < D / 32; ++ks) ka[kt][ks] = *reinterpret_cast<const u32x4*>(src + 32 * ks);
+    }
+  };
+  // V: load u covers rows 2 u, 2 u + 1 whole (a key past the last valid one repeats it; its probability is zero)
+  auto load_values = [&](int i, u32x4 (&va)[KV_LOADS]) __attribute__((always_inline)) {
+    int64_t st;
+    int last;
+    const uint16_t* base = rows_of(i, p.ring_v, ro.vrow, p.nv_sl, st, last);
+    const int lv = lane_per_site(lane);
+#pragma unroll
+    for (int u = 0; u < KV_LOADS; ++u)
+      va[u] = *reinterpret_cast<const u32x4*>(base + min(2 * u + (lv >> 5), last) * st + 8 * (lv & 31));
+  };
+  for (int e = tid; e < TQ * NW * SLOTS; e += NW * 64) (&bm_s[0][0])[e] = -INFINITY;
+  lds_barrier();   // kp_s and the empty block maxima are in LDS
+
+  // ---- phase 1: scores of blocks FIRST .. SLOTS - 1 and their maxima; phase 2: probabilities and P.V ----
+  float m_last = -INFINITY, m_fin = -INFINITY, l_run = 0.f;   // l_run: this lane's keys only
+  f32x4 O[D / 16];
+  auto attend = [&](auto first) __attribute__((always_inline)) {
+    constexpr int FIRST = decltype(first)::value;
+    float s[SLOTS][8];
+    u32x4 va[KV_LOADS];
+    {
+      u32x4 ka[2][2][D / 32];
+      load_keys(FIRST, ka[FIRST & 1]);
+#pragma unroll
+      for (int i = FIRST; i < SLOTS; ++i) {
+        if (i + 1 < SLOTS) load_keys(i + 1, ka[(i + 1) & 1]);
+        else load_values(FIRST, va);
+        if (seen >> i & 1u) {
+          f32x4 S[2];
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < D / 32; ++ks)
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[i & 1][kt][ks]), qb[ks], acc, 0, 0, 0);
+            S[kt] = acc;
+          }
+          // scale and mask the lane's 8 keys 4 q4 + e and 16 + 4 q4 + e
+#pragma unroll
+          for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[i][4 * kt + e] = S[kt][e] * p.scale;
+          if (!(full >> i & 1u)) {
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+              i32x4 rel;
+              if (wave + NW * i < RB) {
+                rel = *reinterpret_cast<const i32x4*>(&kp_s[wave][KB * min(i, W_MAX / NW / KB - 1) + 16 * kt + 4 * q4]);
+              } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rel[e] = (cb0 + wave + NW * i - RB) * KB + 16 * kt + 4 * q4 + e;
+              }
+#pragma unroll
+              for (int e = 0; e < 4; ++e)   // KP_NONE fails the second
+                s[i][4 * kt + e] = ((rel[e] <= l_tok) & (rel[e] > l_tok - W)) ? s[i][4 * kt + e] : -INFINITY;
+            }
+          }
+          float bmax = -INFINITY;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) bmax = fmaxf(bmax, s[i][e]);
+          bmax = max_pair32(max_pair16(bmax));   // over q4 (lane xor 16, 32)
+          if (q4 == 0) bm_s[mcol][wave + NW * i] = bmax;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) s[i][e] = -INFINITY;
+        }
+      }
+    }
+    lds_barrier();   // every block maximum is in LDS
+    // running max through each of the wave's blocks and over all of them
+    float mb[SLOTS];
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      const f32x4 g = *reinterpret_cast<const f32x4*>(&bm_s[mcol][NW * i]);
+      float own = m_fin;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        own = fmaxf(own, w <= wave ? g[w] : -INFINITY);
+        m_fin = fmaxf(m_fin, g[w]);
+      }
+      mb[i] = own;
+    }
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) O[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = FIRST; i < SLOTS; ++i) {
+      // V of block i from registers into LDS, the next block's loads behind it
+      const int lv = lane_per_site(lane);
+#pragma unroll
+      for (int u = 0; u < KV_LOADS; ++u)
+        *reinterpret_cast<u32x4*>(vlds + piece_at(2 * u + (lv >> 5), lv & 31)) = va[u];
+      if (i + 1 < SLOTS) load_values(i + 1, va);
+      if (!(seen >> i & 1u)) continue;
+      const float m = mb[i] == -INFINITY ? 0.f : mb[i];
+      const float alpha = m_last == mb[i] ? 1.f : exp_fast(m_last - m);   // exp(-inf) = 0: nothing added so far
+      m_last = mb[i];
+      if (__ballot(alpha != 1.f)) {
+        l_run *= alpha;
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) O[t] *= alpha;
+      }
+      u32x4 pk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float p0 = exp_fast(s[i][2 * e] - m);
+        const float p1 = exp_fast(s[i][2 * e + 1] - m);
+        l_run += p0 + p1;
+        pk[e] = pack_bf16x2(p0, p1);
+      }
+      const bf16x8 pb = as_bf16x8(pk);
+      // O^T += V^T . P^T over the block's 32 keys, in the lane's key order
+      const int lt = lane_per_site(lane);
+      const int rx = 4 * (lt >> 4) + ((lt & 15) >> 2);   // the lane's key row of a transpose read (and + 16)
+      const uint32_t vbase = lds_offset(vlds) + 2 * (rx * D + 4 * (lt & 3));
+#pragma unroll
+      for (int t = 0; t < D / 16; t += 4) {
+        u32x2 v[4][2];
+        ld_tr_4x2(v, vbase + 32 * (t ^ rx), vbase + 32 * ((t + 1) ^ rx), vbase + 32 * ((t + 2) ^ rx),
+                  vbase + 32 * ((t + 3) ^ rx));
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          O[t + u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              as_bf16x8((u32x4){v[u][0][0], v[u][0][1], v[u][1][0], v[u][1][1]}), pb, O[t + u], 0, 0, 0);
+      }
+    }
+  };
+  // a wave that sees none of its first SLOTS - 1 blocks (a row without history) skips their loads. The barrier count
+  // is the same either way.
+  if (seen & ((1u << (SLOTS - 1)) - 1)) attend(std::integral_constant<int, 0>{});
+  else attend(std::integral_constant<int, SLOTS - 1>{});
+
+  // ---- combine the waves: each leaves its weighted O (lane-linear 16-byte pieces) in its own Vs and takes dims
+  // 64 w + 16 t + 4 q4 + i (t < 4) of every row ----
+  const float wgt = m_last == -INFINITY ? 0.f : exp_fast(m_last - m_fin);
+  const int lw = lane_per_site(lane);
+  l_run = add_xor32(add_xor16(l_run)) * wgt;
+  if (lw < TQ) l_s[wave][lw] = l_run;
+  f32x4* const os = reinterpret_cast<f32x4*>(vlds) + lw;
+#pragma unroll
+  for (int t = 0; t < D / 16; ++t) os[t * 64] = O[t] * wgt;
+  u32x2 gw[4];
+  const int r = r_lo + (lw & 15);
+  const int d0 = 64 * wave + 4 * (lw >> 4);
+  const int l_out = min(r, M - 1) / G;
+  const int g_out = min(r, M - 1) - l_out * G;
+  if (ro.grow) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      gw[t] = *reinterpret_cast<const u32x2*>(ro.grow + l_out * p.g_sl + g_out * p.g_sg + d0 + 16 * t);
+  }
+  lds_barrier();
+  float l_tot = 0.f;
+  f32x4 o[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) o[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    l_tot += l_s[w][lw & 15];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] += reinterpret_cast<const f32x4*>(Vs[w])[(4 * wave + t) * 64 + lw];
+  }
+  if (r < M) {
+    uint16_t* dst = ro.orow + l_out * p.o_sl + g_out * p.o_sg + d0;
+    const bool valid = r < Mv && l_tot > 0.f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(o[t][i] / l_tot) : 0.f;
+      if (ro.grow) {
+        float gt[4];
+        unpack2(gw[t][0], gt[0], gt[1]);
+        unpack2(gw[t][1], gt[2], gt[3]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = y[i] * rbf(1.0f / (1.0f + expf(-gt[i])));
+      }
+      store4_bf16(dst + 16 * t, y);
+    }
+  }
+}
+__global__ __launch_bounds__(NW * 64, 2) void ring_attn_kernel(const RingParams p) {
+  __shared__ union __align__(16) Lds {
+    SplitLds split;
+    GroupLds group;
+    __device__ Lds() {}
+  } lds;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Workgroups are dealt round-robin over the 8 XCDs. Ticks: query group slowest, so that consecutive workgroups take
+  // consecutive (row, kv head) pairs (the live workgroups of a short-row tick spread over all XCDs, and a pair's
+  // groups share one XCD's L2 when the pairs are a multiple of 8). Sequences (no ring): each XCD takes a
+  // contiguous eighth of the groups, whose windows overlap.
+  int pair, qg;
+  if (p.ring_k) {
+    qg = blockIdx.x / p.pairs;
+    pair = blockIdx.x - qg * p.pairs;
+  } else {
+    const int i = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    pair = i / p.qgroups;
+    qg = i - pair * p.qgroups;
+    if (pair >= p.pairs) return;
+  }
+  const int n = pair / p.hkv;
+  const int h = pair - n * p.hkv;
+  const bool padded = p.offsets == nullptr;
+  Row ro;
+  ro.slot = p.ring_k ? p.slots[n] : 0;
+  ro.start = p.ring_k ? p.starts[n] : 0;
+  int64_t len = p.lens[n];
+  if (len < 0 || len > (padded ? LB_MAX : p.lb) || (p.ring_k && (ro.slot < 0 || ro.slot >= p.ring_rows))) len = 0;  // rejected
+  if (padded && len > p.lb) len = p.lb;
+  if (!padded && len < p.min_len) return;              // left to another kernel (single-step rows: decode)
+  ro.len = (int)len;
+  ro.steps = padded ? p.lb : ro.len;
+  const int64_t base_tok = padded ? 0 : p.offsets[n];
+  ro.qrow = p.q + (padded ? n * p.q_sn : base_tok * p.q_sl) + h * p.q_sh;
+  ro.krow = p.new_k + (padded ? n * p.nk_sn : base_tok * p.nk_sl) + h * p.nk_sh;
+  ro.vrow = p.new_v + (padded ? n * p.nv_sn : base_tok * p.nv_sl) + h * p.nv_sh;
+  ro.grow = p.gate ? p.gate + (padded ? n * p.g_sn : base_tok * p.g_sl) + h * p.g_sh + p.g_off : nullptr;
+  ro.orow = p.out + (padded ? n * p.o_sn : base_tok * p.o_sl) + h * p.o_sh;
+  ro.RB = p.ring_k && len > 0 ? p.W / KB : 0;
+  ro.ring_base = ((ro.slot * p.hkv + h) * (int64_t)(p.W + 1)) * D;
+  ro.ring_pos = p.ring_pos + ro.slot * (int64_t)(p.W + 1);
+  const int r_lo = qg * (NW * TQ);
+  const int M = p.G * ro.steps, Mv = p.G * ro.len;      // query rows of this (row, kv head), and the valid ones
+  // rows past the length of a padded row are zeros; attend_group and attend_tile store those of the tiles they take
+  const int tiles = r_lo >= Mv ? 0 : min((Mv - r_lo + TQ - 1) / TQ, NW);
+  const int z_lo = tiles > 1 ? M : r_lo + tiles * TQ;
+  for (int e = threadIdx.x; e < (min(r_lo + NW * TQ, M) - z_lo) * (D / 4); e += NW * 64) {
+    const int r = z_lo + e / (D / 4);
+    const int l = r / p.G;
+    *reinterpret_cast<u32x2*>(ro.orow + l * p.o_sl + (r - l * p.G) * p.o_sg + 4 * (e % (D / 4))) = (u32x2){0u, 0u};
+  }
+  if (tiles == 1) attend_tile(p, ro, r_lo, lds.split, lane, wave);
+  else if (tiles > 1) attend_group(p, ro, r_lo, lds.group, lane, wave);
 }
 
 // In-place ring write of the tick's valid keys/values, launched after the attention kernel (whose query
@@ -424,9 +743,10 @@ extern "C" int hsg_ring_attention(const void* q, int64_t q_sn, int64_t q_sl, int
   p.ring_pos = ring_pos; p.slots = slots; p.starts = starts; p.lens = lens; p.offsets = offsets;
   p.lb = lb; p.hkv = hkv; p.G = groups; p.scale = scale; p.write_ring = write_ring; p.min_len = min_len;
   p.out = static_cast<uint16_t*>(out); p.o_sn = o_sn; p.o_sl = o_sl; p.o_sh = o_sh; p.o_sg = o_sg;
-  p.qgroups = ((groups * lb + 15) / 16 + NW - 1) / NW;
+  p.pairs = n_rows * hkv;
+  p.qgroups = (groups * lb + NW * TQ - 1) / (NW * TQ);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(ring_attn_mfma_kernel, dim3((unsigned)(n_rows * hkv * p.qgroups)), dim3(NW * 64), 0, st, p);
+  hipLaunchKernelGGL(ring_attn_kernel, dim3((unsigned)(p.pairs * p.qgroups)), dim3(NW * 64), 0, st, p);
   if (write_ring) hipLaunchKernelGGL(ring_write_kernel, dim3((unsigned)(n_rows * hkv)), dim3(256), 0, st, p);
   return launch_status();
 }

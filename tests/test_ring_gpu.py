@@ -405,3 +405,36 @@ def test_decode_rope_equals_norm_rope_then_decode(hq):
     assert torch.equal(k0[live], k1[live])
     assert torch.equal(rk0, rk1) and torch.equal(rv0, rv1)
     assert not torch.equal(rk1, ring_k)                 # the steps' keys were written
+
+
+@pytest.mark.parametrize("G,W", [(4, 512), (8, 64), (3, 96)])
+def test_query_tiles_match_oracle(G, W):
+    """hsg_ring_attention at the edges of its 16-row query tiles and 4-tile groups (rows = steps x G): rows of one
+    tile (keys split over the waves), of several, of a group and one tile more, up to the 64 steps of a padded tick;
+    rings full, partly filled and empty; zeros past each row's length."""
+    from hs_guard.engine.kernels import ring_attention_v8
+    print(f"[ring] query tiles G={G} W={W}", flush=True)
+    gen = torch.Generator().manual_seed(40 + G)
+    lens = [1, 16 // G, 16 // G + 1, 0, 32 // G + 1, 64 // G, 64 // G + 1, min(64, W), 3]
+    N, Hkv, D = len(lens), 2, 256
+    Lb = max(lens)
+    q = torch.randn(N, Hkv, G * Lb, D, generator=gen).to(torch.bfloat16)
+    ring_k, ring_v = (torch.randn(N + 1, Hkv, W + 1, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    new_k = torch.randn(N, Hkv, Lb, D, generator=gen).to(torch.bfloat16)
+    value = torch.randn(N, Lb, Hkv * D, generator=gen).to(torch.bfloat16)
+    gate = torch.randn(N, Lb, Hkv * G * 2 * D, generator=gen).to(torch.bfloat16)
+    slots, starts = torch.randperm(N, generator=gen), torch.tensor([3 * W + 5, W, 7, 2, 0, 5 * W - 1, W // 2, W + 40, 0])
+    ring_pos = torch.full((N + 1, W + 1), -1, dtype=torch.long)
+    for s, st in zip(slots.tolist(), starts.tolist()):
+        for p_ in range(max(0, st - W), st):
+            ring_pos[s, p_ % W] = p_
+    lens_t = torch.tensor(lens, dtype=torch.long)
+    dev = torch.device("cuda:0")
+    out = ring_attention_v8(q.to(dev), ring_k.to(dev), ring_v.to(dev), new_k.to(dev), value.to(dev), gate.to(dev),
+                            ring_pos.to(dev), slots.to(dev), starts.to(dev), lens_t.to(dev), D ** -0.5, W, False)
+    ref, _, _, _ = oring.ring_attention_v8(_np(q), _np(ring_k), _np(ring_v), _np(new_k), _np(value), _np(gate),
+                                           ring_pos.numpy(), slots.numpy(), starts.numpy(), lens_t.numpy(),
+                                           D ** -0.5, W, False)
+    _check(_np(out), ref)
+    for n, k in enumerate(lens):
+        assert torch.count_nonzero(out[n, k:]).item() == 0
