@@ -57,90 +57,159 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* hidden, const ui
 // Causal depthwise conv (KS = 4) + SiLU with the conv-history pool update.
 // _conv_silu_kernel (src/hs_guard/engine/fused_kernels.py:94-136): acc = sum_k w[c,k] * ext[t+k] in fp32,
 // out = bf16(silu(bf16(acc))); when len > 0, pool[slot, i] = ext[len + i] for i < KS-1, where
-// ext = [pool rows ; new tokens]. One thread per channel; the 3-row window slides in registers.
+// ext = [pool rows ; new tokens]. A thread takes VEC adjacent channels (2 where every row is 4-byte aligned) over
+// blocks of CONV_TB tokens, the 3-row window sliding in registers; block z of a row starts from the 3 raw rows before
+// it, so a row's blocks run in parallel workgroups. The threads of block 0 own the pool row: they read it first and
+// write the row's last 3 raw rows back, so no other block reads or writes it. The SiLU (exp and an IEEE divide per
+// value) and the 4 bytes per value bound it about equally: one 8,000-token row of 6,144 channels 49.6 us (3.96 TB/s; 54.8
+// as 64-token segments of one channel per thread), one of 311 tokens 6.5 us (12.0).
 // ---------------------------------------------------------------------------------------------------
 constexpr int KS = 4;
+constexpr int CONV_TB = 16;
 
+template <int VEC>
+struct ChannelVec {
+  uint16_t x[VEC];
+};
+
+template <int VEC>
+__device__ __forceinline__ ChannelVec<VEC> load_ch(const uint16_t* p) {
+  ChannelVec<VEC> v;
+  if constexpr (VEC == 2) {
+    const uint32_t w = *reinterpret_cast<const uint32_t*>(p);
+    v.x[0] = (uint16_t)w;
+    v.x[1] = (uint16_t)(w >> 16);
+  } else {
+    v.x[0] = *p;
+  }
+  return v;
+}
+
+template <int VEC>
+__device__ __forceinline__ void store_ch(uint16_t* p, const ChannelVec<VEC>& v) {
+  if constexpr (VEC == 2) *reinterpret_cast<uint32_t*>(p) = (uint32_t)v.x[0] | ((uint32_t)v.x[1] << 16);
+  else *p = v.x[0];
+}
+
+template <int VEC>
 __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int64_t qkv_stride, uint16_t* pool,
                                                         int64_t pool_rows, const uint16_t* weight,
                                                         const int64_t* slots, const int64_t* lens,
                                                         const int64_t* offsets, int L, int C, uint16_t* out,
                                                         int64_t out_stride) {
   const int n = blockIdx.y;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * VEC;
   if (c >= C) return;
-  const int64_t slot = slots[n];
+  const int64_t slot = pool ? slots[n] : 0;
   int64_t len = lens[n];
   const bool padded = offsets == nullptr;
-  const bool slot_ok = slot >= 0 && slot < pool_rows;
+  const bool slot_ok = !pool || (slot >= 0 && slot < pool_rows);
   if (!slot_ok || len < 0) len = 0;
   if (padded && len > L) len = L;
-  const int steps = padded ? L : (int)len;
-  if (!padded && len == 0) return;
+  const int64_t steps = padded ? L : len;
   const int64_t tok0 = padded ? (int64_t)n * L : offsets[n];
-  float w[KS];
-  for (int k = 0; k < KS; ++k) w[k] = bf2f(weight[c * KS + k]);
-  uint16_t e[KS - 1], keep[KS - 1];
-  for (int i = 0; i < KS - 1; ++i) {
-    e[i] = slot_ok ? pool[(slot * (KS - 1) + i) * (int64_t)C + c] : (uint16_t)0;
-    keep[i] = e[i];
-  }
-  auto step = [&](int t, uint16_t x) {
-    float acc = 0.f;
-    acc = fmaf(w[0], bf2f(e[0]), acc);
-    acc = fmaf(w[1], bf2f(e[1]), acc);
-    acc = fmaf(w[2], bf2f(e[2]), acc);
-    acc = fmaf(w[3], bf2f(x), acc);
-    out[(tok0 + t) * out_stride + c] = f2bf(siluf_(rbf(acc)));
-    e[0] = e[1];
-    e[1] = e[2];
-    e[2] = x;
-    if (t == len - 1) {  // window after the last real token = ext[len .. len+2]
-      keep[0] = e[0];
-      keep[1] = e[1];
-      keep[2] = e[2];
+  if ((int64_t)blockIdx.z * CONV_TB >= steps) return;
+  float w[VEC][KS];
+#pragma unroll
+  for (int v = 0; v < VEC; ++v)
+#pragma unroll
+    for (int k = 0; k < KS; ++k) w[v][k] = bf2f(weight[(c + v) * KS + k]);
+  const uint16_t* const row = qkv + tok0 * qkv_stride + c;
+  const bool history = pool && slot_ok;
+  uint16_t* const prow = history ? pool + slot * (KS - 1) * (int64_t)C + c : nullptr;
+  ChannelVec<VEC> e[KS - 1], first[KS - 1];
+  for (int64_t t0 = (int64_t)blockIdx.z * CONV_TB; t0 < steps; t0 += (int64_t)gridDim.z * CONV_TB) {
+#pragma unroll
+    for (int i = 0; i < KS - 1; ++i) {
+      if (t0 > 0) e[i] = load_ch<VEC>(row + (t0 + i - (KS - 1)) * qkv_stride);
+      else if (history) e[i] = load_ch<VEC>(prow + i * (int64_t)C);
+      else e[i] = ChannelVec<VEC>{};
+      if (t0 == 0) first[i] = e[i];
     }
-  };
-  // Whole batches of TB tokens load together (one memory round trip per batch instead of per token); the
-  // remainder, which is all of a single-token row, goes one load at a time.
-  constexpr int TB = 8;
-  int t = 0;
-  for (; t + TB <= steps; t += TB) {
-    uint16_t xs[TB];
+    auto step = [&](int64_t t, ChannelVec<VEC> x) {
+      ChannelVec<VEC> y;
 #pragma unroll
-    for (int i = 0; i < TB; ++i) xs[i] = qkv[(tok0 + t + i) * qkv_stride + c];
+      for (int v = 0; v < VEC; ++v) {
+        float acc = 0.f;
+        acc = fmaf(w[v][0], bf2f(e[0].x[v]), acc);
+        acc = fmaf(w[v][1], bf2f(e[1].x[v]), acc);
+        acc = fmaf(w[v][2], bf2f(e[2].x[v]), acc);
+        acc = fmaf(w[v][3], bf2f(x.x[v]), acc);
+        y.x[v] = f2bf(siluf_(rbf(acc)));
+      }
+      store_ch<VEC>(out + (tok0 + t) * out_stride + c, y);
+      e[0] = e[1];
+      e[1] = e[2];
+      e[2] = x;
+    };
+    // Whole batches of TB tokens load together (one memory round trip per batch instead of per token); the
+    // remainder, which is all of a single-token row, goes one load at a time.
+    constexpr int TB = 8;
+    const int64_t t1 = min(t0 + CONV_TB, steps);
+    int64_t t = t0;
+    for (; t + TB <= t1; t += TB) {
+      ChannelVec<VEC> xs[TB];
 #pragma unroll
-    for (int i = 0; i < TB; ++i) step(t + i, xs[i]);
+      for (int i = 0; i < TB; ++i) xs[i] = load_ch<VEC>(row + (t + i) * qkv_stride);
+#pragma unroll
+      for (int i = 0; i < TB; ++i) step(t + i, xs[i]);
+    }
+    for (; t < t1; ++t) step(t, load_ch<VEC>(row + t * qkv_stride));
   }
-  for (; t < steps; ++t) step(t, qkv[(tok0 + t) * qkv_stride + c]);
-  if (len > 0) {
-    for (int i = 0; i < KS - 1; ++i) pool[(slot * (KS - 1) + i) * (int64_t)C + c] = keep[i];
+  if (blockIdx.z == 0 && history && len > 0) {
+    ChannelVec<VEC> keep[KS - 1];   // the window after the last real token = ext[len .. len+2]
+#pragma unroll
+    for (int i = 0; i < KS - 1; ++i) {
+      const int64_t t = len - (KS - 1) + i;
+      if (t >= 0) keep[i] = load_ch<VEC>(row + t * qkv_stride);
+      else keep[i] = t == -3 ? first[0] : t == -2 ? first[1] : first[2];
+    }
+#pragma unroll
+    for (int i = 0; i < KS - 1; ++i) store_ch<VEC>(prow + i * (int64_t)C, keep[i]);
   }
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Gated RMSNorm of the GDN output, one wave per (token, head) of width 128 (2 values per lane).
+// Gated RMSNorm of the GDN output, per (token, head) of width 128.
 // gated_finish (src/hs_guard/engine/fused_kernels.py:215-233), as the slot step's fused epilogue computes it:
 // r = rsqrt(mean(o^2) + eps) over the head, out = bf16(bf16(w * bf16(o * r)) * silu(z)), o already bf16.
+// A lane holds VEC values: 8 (16 lanes a head, 16-byte pieces, four heads per wave) where every row is 16-byte aligned,
+// else 2 (a wave per head). HBM-bound: 8,000 tokens of 16 heads 23.0 us (4.3 TB/s; 31.9 with
+// 2 values per lane).
 // ---------------------------------------------------------------------------------------------------
+template <int VEC>
 __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const uint16_t* x, int64_t x_stride, const uint16_t* z,
                                                             int64_t z_stride, const uint16_t* w, float eps,
-                                                            uint16_t* out, int64_t out_stride, int tokens,
+                                                            uint16_t* out, int64_t out_stride, int64_t tokens,
                                                             int heads) {
-  const int lane = threadIdx.x & 63;
-  const int item = blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int LANES = 128 / VEC;   // lanes of a head
+  const int lane = threadIdx.x % LANES;
+  const int64_t item = (int64_t)blockIdx.x * (256 / LANES) + threadIdx.x / LANES;
   if (item >= tokens * heads) return;
-  const int t = item / heads;
-  const int c = (item - t * heads) * 128 + 2 * lane;
-  float x0, x1, z0, z1, w0, w1;
-  unpack2(*reinterpret_cast<const uint32_t*>(x + t * x_stride + c), x0, x1);
-  unpack2(*reinterpret_cast<const uint32_t*>(z + t * z_stride + c), z0, z1);
-  unpack2(*reinterpret_cast<const uint32_t*>(w + 2 * lane), w0, w1);
-  const float ss = wave_sum(x0 * x0 + x1 * x1);
+  const int64_t t = item / heads;
+  const int c = (int)(item - t * heads) * 128 + VEC * lane;
+  float xv[VEC], zv[VEC], wv[VEC];
+  if constexpr (VEC == 8) {
+    load8_bf16(x + t * x_stride + c, xv);
+    load8_bf16(z + t * z_stride + c, zv);
+    load8_bf16(w + VEC * lane, wv);
+  } else {
+    unpack2(*reinterpret_cast<const uint32_t*>(x + t * x_stride + c), xv[0], xv[1]);
+    unpack2(*reinterpret_cast<const uint32_t*>(z + t * z_stride + c), zv[0], zv[1]);
+    unpack2(*reinterpret_cast<const uint32_t*>(w + VEC * lane), wv[0], wv[1]);
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) ss += xv[i] * xv[i];
+  ss = VEC == 8 ? sum16_dpp(ss) : wave_sum(ss);
   const float r = rsqrtf(ss * (1.0f / 128) + eps);
-  const float y0 = rbf(w0 * rbf(x0 * r)) * siluf_(z0);
-  const float y1 = rbf(w1 * rbf(x1 * r)) * siluf_(z1);
-  *reinterpret_cast<uint32_t*>(out + t * out_stride + c) = (uint32_t)f2bf(y0) | ((uint32_t)f2bf(y1) << 16);
+  uint32_t y[VEC / 2];
+#pragma unroll
+  for (int i = 0; i < VEC; i += 2)
+    y[i / 2] = pack_bf16x2(rbf(wv[i] * rbf(xv[i] * r)) * siluf_(zv[i]),
+                           rbf(wv[i + 1] * rbf(xv[i + 1] * r)) * siluf_(zv[i + 1]));
+  if constexpr (VEC == 8) *reinterpret_cast<u32x4*>(out + t * out_stride + c) = (u32x4){y[0], y[1], y[2], y[3]};
+  else *reinterpret_cast<uint32_t*>(out + t * out_stride + c) = y[0];
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -355,15 +424,24 @@ extern "C" int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* p
                                     const void* weight, int32_t kernel_size, const int64_t* slots, const int64_t* lens,
                                     const int64_t* offsets, int32_t n_rows, int32_t L, int32_t channels, void* out,
                                     int64_t out_stride, void* stream) {
-  if (n_rows < 0 || channels <= 0 || pool_rows <= 0 || L < 0) return HSG_ERR_ARG;
+  if (n_rows < 0 || channels <= 0 || (pool && pool_rows <= 0) || L < 0) return HSG_ERR_ARG;
   if (kernel_size != KS) return HSG_ERR_SHAPE;
   if (n_rows == 0) return HSG_OK;
-  if (!qkv || !pool || !weight || !slots || !lens || !out || (!offsets && L <= 0)) return HSG_ERR_ARG;
-  const dim3 grid((channels + 255) / 256, n_rows);
-  hipLaunchKernelGGL(conv_silu_kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
-                     static_cast<const uint16_t*>(qkv), qkv_stride, static_cast<uint16_t*>(pool), pool_rows,
-                     static_cast<const uint16_t*>(weight), slots, lens, offsets, L, channels,
-                     static_cast<uint16_t*>(out), out_stride);
+  if (!qkv || !weight || (pool && !slots) || !lens || !out || (!offsets && L <= 0)) return HSG_ERR_ARG;
+  const bool pairs = channels % 2 == 0 && qkv_stride % 2 == 0 && out_stride % 2 == 0 && aligned(qkv, 4) &&
+                     aligned(out, 4) && (!pool || aligned(pool, 4));
+  // token blocks of a row in parallel, up to the grid's z limit (a row with more walks them)
+  const int blocks = L > 0 ? min((L - 1) / CONV_TB + 1, 65535) : 1;
+  const int cols = pairs ? channels / 2 : channels;
+  const dim3 grid((cols + 255) / 256, n_rows, blocks);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(qkv), qkv_stride, static_cast<uint16_t*>(pool), pool_rows,
+                       static_cast<const uint16_t*>(weight), slots, lens, offsets, L, channels,
+                       static_cast<uint16_t*>(out), out_stride);
+  };
+  if (pairs) launch(conv_silu_kernel<2>);
+  else launch(conv_silu_kernel<1>);
   return launch_status();
 }
 
@@ -378,10 +456,16 @@ extern "C" int hsg_gated_rmsnorm(const void* x, int64_t x_stride, const void* z,
       !aligned(out, 4))
     return HSG_ERR_ALIGN;
   const int64_t items = (int64_t)tokens * heads;
-  hipLaunchKernelGGL(gated_rmsnorm_kernel, dim3((unsigned)((items + 3) / 4)), dim3(256), 0,
-                     reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), x_stride,
-                     static_cast<const uint16_t*>(z), z_stride, static_cast<const uint16_t*>(w), eps,
-                     static_cast<uint16_t*>(out), out_stride, tokens, heads);
+  const bool wide = x_stride % 8 == 0 && z_stride % 8 == 0 && out_stride % 8 == 0 && aligned(x, 16) && aligned(z, 16) &&
+                    aligned(w, 16) && aligned(out, 16);
+  const auto launch = [&](auto kernel, int per_block) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)((items + per_block - 1) / per_block)), dim3(256), 0,
+                       reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), x_stride,
+                       static_cast<const uint16_t*>(z), z_stride, static_cast<const uint16_t*>(w), eps,
+                       static_cast<uint16_t*>(out), out_stride, (int64_t)tokens, heads);
+  };
+  if (wide) launch(gated_rmsnorm_kernel<8>, 16);
+  else launch(gated_rmsnorm_kernel<2>, 4);
   return launch_status();
 }
 

@@ -28,7 +28,8 @@
 // Measured (W = 512, 16 q / 4 kv heads), with every tile on attend_group before and now:
 // 72 padded rows of 2 to 64 steps 147 -> 92 us (49 us of it whole groups past their rows' lengths, which ran their
 // keys), 64 rows of 4 steps 41.6 -> 28.0 us, one such row 34.9 -> 21.6 us. Splitting the keys of longer rows' tiles too
-// reads K and V once per tile instead of once per group: 72 rows of 64 steps 264 us against 165.
+// reads K and V once per tile instead of once per group: 72 rows of 64 steps 264 us against 165. A sequence of 8,000
+// tokens (no ring): 203 us, against 270 us over rings gathered from it (and 0.2 ms of gathers).
 #include <math.h>
 
 #include <type_traits>
@@ -67,6 +68,7 @@ struct RingParams {
   int min_len;
   int pairs;        // rows x kv heads
   int qgroups;      // workgroups (groups of NW tiles) per (row, kv head)
+  int qg0;          // first group
   uint16_t* out; int64_t o_sn, o_sl, o_sh, o_sg;
 };
 
@@ -615,7 +617,7 @@ __global__ __launch_bounds__(NW * 64, 2) void ring_attn_kernel(const RingParams 
   } else {
     const int i = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     pair = i / p.qgroups;
-    qg = i - pair * p.qgroups;
+    qg = p.qg0 + i - pair * p.qgroups;
     if (pair >= p.pairs) return;
   }
   const int n = pair / p.hkv;
@@ -748,5 +750,49 @@ extern "C" int hsg_ring_attention(const void* q, int64_t q_sn, int64_t q_sl, int
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(ring_attn_kernel, dim3((unsigned)(p.pairs * p.qgroups)), dim3(NW * 64), 0, st, p);
   if (write_ring) hipLaunchKernelGGL(ring_write_kernel, dim3((unsigned)(n_rows * hkv)), dim3(256), 0, st, p);
+  return launch_status();
+}
+
+extern "C" int hsg_window_attention(const void* q, int64_t q_sl, int64_t q_sh, int64_t q_sg, const void* k,
+                                    int64_t k_sl, int64_t k_sh, const void* v, int64_t v_sl, int64_t v_sh,
+                                    const void* gate, int64_t g_sl, int64_t g_sh, int64_t g_sg, int64_t g_off,
+                                    const int64_t* lens, const int64_t* offsets, int32_t n_rows, int32_t max_len,
+                                    int32_t first, int32_t count, int32_t window, int32_t hkv, int32_t groups,
+                                    int32_t head_dim, float scale, void* out, int64_t o_sl, int64_t o_sh,
+                                    int64_t o_sg, void* stream) {
+  using namespace hsg;
+  if (n_rows < 0 || max_len <= 0 || first < 0 || count <= 0 || hkv <= 0 || groups <= 0) return HSG_ERR_ARG;
+  if (n_rows == 0) return HSG_OK;
+  if (!q || !k || !v || !lens || !offsets || !out) return HSG_ERR_ARG;
+  if (head_dim != D || window <= 0 || window > W_MAX) return HSG_ERR_SHAPE;
+  constexpr int GR = NW * TQ;   // query rows of a workgroup
+  const int64_t rows = (int64_t)groups * max_len;
+  if (rows > (1 << 30) || (int64_t)first * groups % GR) return HSG_ERR_SHAPE;
+  const int64_t strides[] = {q_sl, q_sh, q_sg, k_sl, k_sh, v_sl, v_sh};
+  for (int64_t st : strides)
+    if (st % 8) return HSG_ERR_ALIGN;
+  const int64_t s4[] = {g_sl, g_sh, g_sg, g_off, o_sl, o_sh, o_sg};
+  for (int64_t st : s4)
+    if (st % 4) return HSG_ERR_ALIGN;
+  if (!aligned(q, 16) || !aligned(k, 16) || !aligned(v, 16) || !aligned(out, 8) || (gate && !aligned(gate, 8)))
+    return HSG_ERR_ALIGN;
+  if (first >= max_len) return HSG_OK;
+  const int64_t last = (int64_t)first + count < max_len ? (int64_t)first + count : max_len;
+  const int64_t qgroups = (last * groups + GR - 1) / GR - (int64_t)first * groups / GR;
+  const int64_t blocks = ((int64_t)n_rows * hkv * qgroups + 7) / 8 * 8;
+  if (blocks > 0x7fffffff) return HSG_ERR_SHAPE;
+  RingParams p{};
+  p.q = static_cast<const uint16_t*>(q); p.q_sl = q_sl; p.q_sh = q_sh; p.q_sg = q_sg;
+  p.W = window;
+  p.new_k = static_cast<const uint16_t*>(k); p.nk_sl = k_sl; p.nk_sh = k_sh;
+  p.new_v = static_cast<const uint16_t*>(v); p.nv_sl = v_sl; p.nv_sh = v_sh;
+  p.gate = static_cast<const uint16_t*>(gate); p.g_sl = g_sl; p.g_sh = g_sh; p.g_sg = g_sg; p.g_off = g_off;
+  p.lens = lens; p.offsets = offsets;
+  p.lb = max_len; p.hkv = hkv; p.G = groups; p.scale = scale; p.min_len = 0;
+  p.pairs = n_rows * hkv;
+  p.qgroups = (int)qgroups;
+  p.qg0 = (int)((int64_t)first * groups / GR);
+  p.out = static_cast<uint16_t*>(out); p.o_sl = o_sl; p.o_sh = o_sh; p.o_sg = o_sg;
+  hipLaunchKernelGGL(ring_attn_kernel, dim3((unsigned)blocks), dim3(NW * 64), 0, reinterpret_cast<hipStream_t>(stream), p);
   return launch_status();
 }

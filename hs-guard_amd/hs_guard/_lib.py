@@ -79,6 +79,13 @@ SIGNATURES = {
         _I32, _I32, _I32, _I32, _I32, _F, _I32, _I32,  # n_rows, lb, hkv, groups, head_dim, scale, write_ring,
                                                          # min_len
         _P, _I64, _I64, _I64, _I64, _P]),    # out, o_sn, o_sl, o_sh, o_sg, stream
+    "hsg_window_attention": (ctypes.c_int, [
+        _P, _I64, _I64, _I64,                # q, q_sl, q_sh, q_sg
+        _P, _I64, _I64, _P, _I64, _I64,      # k, k_sl, k_sh, v, v_sl, v_sh
+        _P, _I64, _I64, _I64, _I64,          # gate, g_sl, g_sh, g_sg, g_off
+        _P, _P, _I32, _I32, _I32, _I32,      # lens, offsets, n_rows, max_len, first, count
+        _I32, _I32, _I32, _I32, _F,          # window, hkv, groups, head_dim, scale
+        _P, _I64, _I64, _I64, _P]),          # out, o_sl, o_sh, o_sg, stream
     "hsg_ring_decode_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32, _I32]),
     "hsg_ring_decode": (ctypes.c_int, [
         _P, _I64, _I64, _I64, _I64,          # q, q_sn, q_sl, q_sh, q_sg

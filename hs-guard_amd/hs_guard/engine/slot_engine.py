@@ -454,8 +454,9 @@ class SlotStreamEngine(PreparedWeights):
                     conv = self._view("conv", tb, C)
                     check(L.hsg_conv_silu_update(proj.data_ptr(), self.gdn_in, self.conv[idx].data_ptr(), S,
                                                  Lw["conv_w"].data_ptr(), cfg.linear_conv_kernel_dim,
-                                                 slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb, 0, C,
-                                                 conv.data_ptr(), C, st), "hsg_conv_silu_update")
+                                                 slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb,
+                                                 self.max_tick_tokens if R else 0, C, conv.data_ptr(), C, st),
+                          "hsg_conv_silu_update")
                     check(L.hsg_gdn_slot_step_gated(
                         conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
                         base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), self.gdn_in,

@@ -5,19 +5,15 @@ Qwen3.5 backbone with FLA's ``chunk_gated_delta_rule`` in the GDN layers (runtim
 512-token window attention (src/hs_guard/window_attention.py:34-53, 56-72) in the attention layers, then both
 roles' risk heads (runtime.py:71-74).
 
-* GDN layers: fused projection GEMM -> causal conv + SiLU -> ``hsg_gdn_chunk_prefill`` from a zero state (the
-  WY/UT chunk form on MFMA) -> ``hsg_gated_rmsnorm`` -> out_proj.
-* Attention layers: fused q|k|v GEMM -> q/k RMSNorm + RoPE at positions 0 .. T-1 -> window attention ->
-  sigmoid(gate) -> o_proj.
+* GDN layers: fused projection GEMM -> causal conv + SiLU from a zero history -> ``hsg_gdn_chunk_prefill`` from a
+  zero state (the WY/UT chunk form on MFMA) -> ``hsg_gated_rmsnorm`` -> out_proj.
+* Attention layers: fused q|k|v GEMM -> q/k RMSNorm + RoPE at positions 0 .. T-1 -> ``hsg_window_attention`` (the
+  window mask 0 <= p <= q, p > q - W over the sequence's own keys, gated by sigmoid(gate)) -> o_proj.
 * Risk heads in float32, as the reference's readout on ``hidden.float()`` outside autocast (runtime.py:70-73,
   141): an fp32 GEMM with the heads' fp32 weights, then ``hsg_risk_head_f32`` (LayerNorm, SiLU, logits and
   softmax, nothing rounded to bf16).
-* The sequence is cut into 64-token segments for the conv and the attention. Segment s is given, as its conv
-  history, the 3 tokens before it and, as its "ring", the keys and values of the W positions before it
-  (positions [64 s - W, 64 s) at columns p mod W, ring_pos = p, or -1 before the sequence start), gathered on
-  the device. ``hsg_conv_silu_update`` and ``hsg_ring_attention`` (no ring write) then compute exactly the
-  whole sequence's causal conv and window mask (0 <= p <= q, p > q - W). No per-slot state of the streaming
-  engine is read or written.
+
+No per-slot state of the streaming engine is read or written.
 
 GEMMs run at the whole sequence's M, so results differ from the streaming path's in the last bits of some
 products; the two agree within the tolerances the tests state (the reference's own stream-vs-whole check
@@ -25,15 +21,13 @@ allows 0.05, examples/demo/server.py:483).
 """
 from __future__ import annotations
 
-import math
-
 import torch
 
 from .._lib import check, lib
 from .slot_engine import ROLES, PreparedWeights, gdn_proj_width
 
-SEG = 64                  # tokens per conv / attention segment (the tiled ring kernel's row limit)
-MAX_ATT_SEGMENTS = 128    # segments per attention launch: bounds the gathered rings to ~270 MB at W = 512
+SEG = 64                  # query tokens of an attention segment
+MAX_ATT_SEGMENTS = 1 << 17    # segments per attention launch: bounds its grid for sequences of millions of tokens
 
 
 def fp32_heads(model, roles=ROLES):
@@ -88,101 +82,64 @@ class WholeSequenceScorer(PreparedWeights):
         C = cfg.conv_dim
         gdn_in = gdn_proj_width(cfg)       # row stride of the GDN projection (zero-padded weight rows)
         att_in = hq * 2 * D + 2 * hkv * D
-        i64 = dict(dtype=torch.long, device=dev)
+        VD = cfg.value_dim
+        I = cfg.intermediate_size
 
-        ids_d = torch.tensor(list(ids), **i64)
-        pos = torch.arange(T, **i64)
-        nseg = math.ceil(T / SEG)
-        seg_off = torch.arange(nseg, **i64) * SEG
-        seg_len = torch.clamp(T - seg_off, max=SEG)
-        seg_slot = torch.arange(nseg, **i64)
-        # conv history of segment s: tokens 64 s - 3 .. 64 s - 1 (zero before the sequence start)
-        K1 = cfg.linear_conv_kernel_dim - 1
-        hist = seg_off[:, None] - K1 + torch.arange(K1, **i64)[None, :]
-        hist_ok = (hist >= 0)[..., None]
-        hist = hist.clamp(min=0)
-        # window ring of segment s: column c holds position 64 s - W + ((c - 64 s) mod W)
-        cols = torch.arange(W, **i64)[None, :]
-        ring_p = seg_off[:, None] - W + torch.remainder(cols - seg_off[:, None], W)
-        ring_pos_all = torch.full((nseg, W + 1), -1, **i64)
-        ring_pos_all[:, :W] = torch.where(ring_p >= 0, ring_p, torch.full_like(ring_p, -1))
-        ring_src = ring_p.clamp(min=0)
-
-        hidden = torch.empty(T, H, dtype=bf16, device=dev)
-        normed = torch.empty_like(hidden)
-        mix = torch.empty_like(hidden)
+        ids_d = torch.tensor(list(ids), dtype=torch.long, device=dev)
+        # positions 0 .. T - 1, then the sequence as one packed row: its slot and offset (0) and its length
+        index = torch.arange(T + 1, dtype=torch.long, device=dev)
+        pos, row0, row_len = index.data_ptr(), index.data_ptr(), index[T:].data_ptr()
+        # one buffer per role of an activation, reused by every layer
+        hidden, normed, mix = (torch.empty(T, H, dtype=bf16, device=dev) for _ in range(3))
+        proj = torch.empty(T * max(gdn_in, att_in, 2 * I), dtype=bf16, device=dev)
+        mid = torch.empty(T * max(C, hq * D, I), dtype=bf16, device=dev)
+        heads = torch.empty(T * max(2 * VD, (hq + hkv) * D), dtype=bf16, device=dev)
+        proj_p, mid_p, heads_p, normed_p, mix_p = (t.data_ptr() for t in (proj, mid, heads, normed, mix))
+        gdn_proj, att_proj, gate_up = (proj[:T * n].view(T, n) for n in (gdn_in, att_in, 2 * I))
+        gated, att, act = heads[T * VD:2 * T * VD].view(T, VD), mid[:T * hq * D].view(T, hq * D), mid[:T * I].view(T, I)
+        n_gdn = sum(1 for k, _ in self.kind if k == "linear_attention")
+        state = torch.zeros(n_gdn, hv, kd, vd, dtype=torch.float32, device=dev)
+        ws_bytes = max(int(L.hsg_gdn_chunk_workspace_bytes(1, T, hv)), 256) if n_gdn else 256
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        mm = torch.mm
         check(L.hsg_embed_rmsnorm(ids_d.data_ptr(), self.emb.data_ptr(), cfg.vocab_size,
-                                  self.layers[0]["in_w1"].data_ptr(), eps, hidden.data_ptr(), normed.data_ptr(), T, H,
-                                  st), "hsg_embed_rmsnorm")
-        ws = state = None
-        row0 = torch.zeros(1, **i64)
-        row_len = torch.full((1,), T, **i64)
-        for i, ((kind, _), Lw) in enumerate(zip(self.kind, self.layers)):
+                                  self.layers[0]["in_w1"].data_ptr(), eps, hidden.data_ptr(), normed_p, T, H, st),
+              "hsg_embed_rmsnorm")
+        for i, ((kind, idx), Lw) in enumerate(zip(self.kind, self.layers)):
             if kind == "linear_attention":
-                proj = torch.mm(normed, Lw["w_in"].t())
-                pools = torch.where(hist_ok, proj[:, :C][hist], torch.zeros((), dtype=bf16, device=dev)).contiguous()
-                conv = torch.empty(T, C, dtype=bf16, device=dev)
-                check(L.hsg_conv_silu_update(proj.data_ptr(), gdn_in, pools.data_ptr(), nseg,
-                                             Lw["conv_w"].data_ptr(), cfg.linear_conv_kernel_dim, seg_slot.data_ptr(),
-                                             seg_len.data_ptr(), seg_off.data_ptr(), nseg, 0, C, conv.data_ptr(), C,
-                                             st), "hsg_conv_silu_update")
-                if ws is None:
-                    ws = torch.empty(max(int(L.hsg_gdn_chunk_workspace_bytes(1, T, hv)), 256), dtype=torch.uint8,
-                                     device=dev)
-                    state = torch.empty(1, hv, kd, vd, dtype=torch.float32, device=dev)
-                state.zero_()
-                o = torch.empty(T, hv, vd, dtype=bf16, device=dev)
-                base = proj.data_ptr()
+                mm(normed, Lw["w_in"].t(), out=gdn_proj)
+                check(L.hsg_conv_silu_update(proj_p, gdn_in, None, 0, Lw["conv_w"].data_ptr(),
+                                             cfg.linear_conv_kernel_dim, None, row_len, row0, 1, T, C, mid_p, C, st),
+                      "hsg_conv_silu_update")
                 check(L.hsg_gdn_chunk_prefill(
-                    conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
-                    base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), gdn_in,
-                    Lw["A_log"].data_ptr(), Lw["dt_bias"].data_ptr(), state.data_ptr(), 0, 1, row0.data_ptr(),
-                    row_len.data_ptr(), row0.data_ptr(), 1, T, nh, hv, kd, vd, kd ** -0.5, o.data_ptr(), None, 0,
-                    ws.data_ptr(), ws.numel(), st), "hsg_gdn_chunk_prefill")
-                gated = torch.empty(T, cfg.value_dim, dtype=bf16, device=dev)
-                check(L.hsg_gated_rmsnorm(o.data_ptr(), cfg.value_dim, base + 2 * C, gdn_in, Lw["norm_w"].data_ptr(),
-                                          eps, gated.data_ptr(), cfg.value_dim, T, hv, vd, st), "hsg_gated_rmsnorm")
-                torch.mm(gated, Lw["w_out"].t(), out=mix)
+                    mid_p, C, 0, cfg.key_dim, 2 * cfg.key_dim, proj_p + 2 * (C + VD + hv), proj_p + 2 * (C + VD), gdn_in,
+                    Lw["A_log"].data_ptr(), Lw["dt_bias"].data_ptr(), state[idx].data_ptr(), 0, 1, row0,
+                    row_len, row0, 1, T, nh, hv, kd, vd, kd ** -0.5, heads_p, None, 0, ws.data_ptr(), ws_bytes, st),
+                      "hsg_gdn_chunk_prefill")
+                check(L.hsg_gated_rmsnorm(heads_p, VD, proj_p + 2 * C, gdn_in, Lw["norm_w"].data_ptr(), eps,
+                                          heads_p + 2 * T * VD, VD, T, hv, vd, st), "hsg_gated_rmsnorm")
+                mm(gated, Lw["w_out"].t(), out=mix)
             else:
-                proj = torch.mm(normed, Lw["w_in"].t())
-                q = torch.empty(T, hq * D, dtype=bf16, device=dev)
-                k = torch.empty(T, hkv * D, dtype=bf16, device=dev)
-                base = proj.data_ptr()
-                check(L.hsg_norm_rope(base, att_in, 2 * D, hq, Lw["q_w1"].data_ptr(), eps, q.data_ptr(), hq * D, D,
-                                      base + 2 * hq * 2 * D, att_in, D, hkv, Lw["k_w1"].data_ptr(), eps,
-                                      k.data_ptr(), hkv * D, D, pos.data_ptr(), self.inv_freq.data_ptr(),
-                                      cfg.rotary_dim, T, D, st), "hsg_norm_rope")
-                v = proj[:, hq * 2 * D + hkv * D:].view(T, hkv, D)
-                kh = k.view(T, hkv, D)
-                att = torch.empty(T, hq * D, dtype=bf16, device=dev)
-                for s0 in range(0, nseg, MAX_ATT_SEGMENTS):
-                    s1 = min(nseg, s0 + MAX_ATT_SEGMENTS)
-                    n = s1 - s0
-                    ring_k = torch.zeros(n, hkv, W + 1, D, dtype=bf16, device=dev)
-                    ring_v = torch.zeros_like(ring_k)
-                    ring_k[:, :, :W] = kh[ring_src[s0:s1]].permute(0, 2, 1, 3)
-                    ring_v[:, :, :W] = v[ring_src[s0:s1]].permute(0, 2, 1, 3)
-                    rpos = ring_pos_all[s0:s1].contiguous()
-                    offs = seg_off[s0:s1].contiguous()
-                    lens = seg_len[s0:s1].contiguous()
-                    slots = torch.arange(n, **i64)
-                    check(L.hsg_ring_attention(
-                        q.data_ptr(), 0, hq * D, G * D, D, ring_k.data_ptr(), ring_v.data_ptr(), n, W,
-                        k.data_ptr(), 0, hkv * D, D, base + 2 * (hq * 2 * D + hkv * D), 0, att_in, D,
-                        base, 0, att_in, G * 2 * D, 2 * D, D, rpos.data_ptr(), slots.data_ptr(), offs.data_ptr(),
-                        lens.data_ptr(), offs.data_ptr(), n, SEG, hkv, G, D, D ** -0.5, 0, 0,
-                        att.data_ptr(), 0, hq * D, G * D, D, st), "hsg_ring_attention")
-                torch.mm(att, Lw["w_out"].t(), out=mix)
-            check(L.hsg_add_rmsnorm(hidden.data_ptr(), mix.data_ptr(), Lw["post_w1"].data_ptr(), eps,
-                                    normed.data_ptr(), T, H, st), "hsg_add_rmsnorm")
-            I = cfg.intermediate_size
-            gu = torch.mm(normed, Lw["w_gu"].t())
-            act = torch.empty(T, I, dtype=bf16, device=dev)
-            check(L.hsg_silu_mul(gu.data_ptr(), 2 * I, I, act.data_ptr(), T, st), "hsg_silu_mul")
-            torch.mm(act, Lw["w_down"].t(), out=mix)
+                mm(normed, Lw["w_in"].t(), out=att_proj)
+                k_p = heads_p + 2 * T * hq * D
+                check(L.hsg_norm_rope(proj_p, att_in, 2 * D, hq, Lw["q_w1"].data_ptr(), eps, heads_p, hq * D, D,
+                                      proj_p + 2 * hq * 2 * D, att_in, D, hkv, Lw["k_w1"].data_ptr(), eps, k_p,
+                                      hkv * D, D, pos, self.inv_freq.data_ptr(), cfg.rotary_dim, T, D, st),
+                      "hsg_norm_rope")
+                for first in range(0, T, SEG * MAX_ATT_SEGMENTS):
+                    check(L.hsg_window_attention(
+                        heads_p, hq * D, G * D, D, k_p, hkv * D, D, proj_p + 2 * (hq * 2 * D + hkv * D), att_in, D,
+                        proj_p, att_in, G * 2 * D, 2 * D, D, row_len, row0, 1, T, first, SEG * MAX_ATT_SEGMENTS, W,
+                        hkv, G, D, D ** -0.5, mid_p, hq * D, G * D, D, st), "hsg_window_attention")
+                mm(att, Lw["w_out"].t(), out=mix)
+            check(L.hsg_add_rmsnorm(hidden.data_ptr(), mix_p, Lw["post_w1"].data_ptr(), eps, normed_p, T, H, st),
+                  "hsg_add_rmsnorm")
+            mm(normed, Lw["w_gu"].t(), out=gate_up)
+            check(L.hsg_silu_mul(proj_p, 2 * I, I, mid_p, T, st), "hsg_silu_mul")
+            mm(act, Lw["w_down"].t(), out=mix)
             nxt = self.layers[i + 1]["in_w1"] if i + 1 < len(self.layers) else self.final_w1
-            check(L.hsg_add_rmsnorm(hidden.data_ptr(), mix.data_ptr(), nxt.data_ptr(), eps, normed.data_ptr(), T, H,
-                                    st), "hsg_add_rmsnorm")
+            check(L.hsg_add_rmsnorm(hidden.data_ptr(), mix_p, nxt.data_ptr(), eps, normed_p, T, H, st),
+                  "hsg_add_rmsnorm")
         R, E = len(self.roles), cfg.head_hidden
         h32 = self.head32
         y = torch.addmm(h32["b1"], normed.float(), h32["w1"].t())

@@ -179,6 +179,22 @@ int hsg_ring_attention(const void* q, int64_t q_sn, int64_t q_sl, int64_t q_sh, 
                        int64_t o_sn, int64_t o_sl, int64_t o_sh, int64_t o_sg, void* stream);
 
 /*
+ * The same attention of whole sequences over their own keys (no ring): query step l of row n sees the keys j <= l,
+ * j > l - window of its row. Replaces the tiled window attention of the complete-message forward
+ * (src/hs_guard/window_attention.py:34-72). Packed rows (offsets required): row n's tokens are offsets[n] ..
+ * offsets[n] + lens[n] - 1, at most max_len of them (longer rows are treated as empty); element addresses and the gate
+ * as hsg_ring_attention's packed layout. Only the query steps first .. first + count - 1 of every row are computed
+ * (first x groups a multiple of 64), so that a caller can cut a long sequence into launches; every output is the same
+ * in whichever launch it falls. Supported: head_dim == 256, window <= 512, groups x max_len <= 2^30.
+ */
+int hsg_window_attention(const void* q, int64_t q_sl, int64_t q_sh, int64_t q_sg, const void* k, int64_t k_sl,
+                         int64_t k_sh, const void* v, int64_t v_sl, int64_t v_sh, const void* gate, int64_t g_sl,
+                         int64_t g_sh, int64_t g_sg, int64_t g_off, const int64_t* lens, const int64_t* offsets,
+                         int32_t n_rows, int32_t max_len, int32_t first, int32_t count, int32_t window, int32_t hkv,
+                         int32_t groups, int32_t head_dim, float scale, void* out, int64_t o_sl, int64_t o_sh,
+                         int64_t o_sg, void* stream);
+
+/*
  * Ring attention for decode steps: the same contract and numerics as hsg_ring_attention for rows with
  * lens[n] == 1 (one query position; lb is 1 and the padded layout is [n_rows, 1, ...]). Replaces
  * ring_attention_v8 at its decode shape (src/hs_guard/engine/fused_kernels.py:358-376 with Lb == 1,
@@ -291,7 +307,9 @@ int hsg_gated_rmsnorm(const void* x, int64_t x_stride, const void* z, int64_t z_
  * (src/hs_guard/engine/fused_kernels.py:126-136; kernel :94-123):
  *   qkv [tokens, qkv_stride] bf16 (first `channels` columns), pool [pool_rows, kernel_size-1, channels]
  *   bf16 (updated in place at slots[n] when lens[n] > 0), weight [channels, kernel_size] bf16,
- *   out [tokens, out_stride] bf16. Padded layout computes all L positions of every row like the reference.
+ *   out [tokens, out_stride] bf16. Padded layout computes all L positions of every row like the reference. Packed
+ *   layout: rows of any length; L (0: unknown) is their usual largest length, by which a row's tokens are spread over
+ *   workgroups. pool NULL: rows start from a zero history, and none is kept (slots is not read).
  * Supported: kernel_size == 4.
  */
 int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* pool, int64_t pool_rows, const void* weight,

@@ -244,3 +244,37 @@ def test_ring_pos_update_bit_exact():
                                          torch.from_numpy(ln).to(DEV).data_ptr(), nb, 64, _stream()) == 0
         length[slots] += lens
     np.testing.assert_array_equal(rp_d.cpu().numpy(), rp)
+
+
+@pytest.mark.parametrize("lens,L,C,history", [([40, 1, 16, 17, 0, 2], 40, 6144, True), ([33, 70], 33, 258, True),
+                                              ([19, 3], 19, 77, True), ([300], 300, 6144, False)])
+def test_conv_token_blocks(lens, L, C, history):
+    """hsg_conv_silu_update with a row's tokens spread over workgroups (packed rows, L given; one longer than L): block
+    edges, odd channel counts, and rows without a history pool."""
+    from hs_guard._lib import lib
+    print(f"[glue] conv blocks {lens} C={C}", flush=True)
+    rng = np.random.default_rng(7)
+    N, S, Lm = len(lens), len(lens) + 1, max(lens)
+    slots, lens = rng.permutation(S)[:N], np.array(lens)
+    qkv = bf16(rng.standard_normal((N, Lm, C)))
+    pool = bf16(rng.standard_normal((S, 3, C))) if history else np.zeros((S, 3, C), np.float32)
+    w = bf16(rng.standard_normal((C, 4)) * 0.5)
+    ref_out, ref_pool = oglue.conv_silu_update(qkv, pool, w, slots, lens)
+    # the bound of test_conv_silu_update: 2 bf16 ulps + the fp32 sum's absolute error
+    atol = 4 * 2.0 ** -24 * float(np.abs(w).max()) * float(max(np.abs(qkv).max(), np.abs(pool).max())) * 4
+    pool_d, w_d = _bf(pool).to(DEV), _bf(w).to(DEV)
+    sl_d, ln_d = torch.from_numpy(slots).to(DEV), torch.from_numpy(lens).to(DEV)
+    offs = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    of_d = torch.from_numpy(offs).to(DEV)
+    q_d = _bf(np.concatenate([qkv[n, :lens[n]] for n in range(N)])).to(DEV)
+    out = torch.zeros(len(q_d), C, dtype=torch.bfloat16, device=DEV)
+    rc = lib().hsg_conv_silu_update(q_d.data_ptr(), C, pool_d.data_ptr() if history else None, S if history else 0,
+                                    w_d.data_ptr(), 4, sl_d.data_ptr() if history else None, ln_d.data_ptr(),
+                                    of_d.data_ptr(), N, L, C, out.data_ptr(), C, _stream())
+    assert rc == 0
+    got = _np(out)
+    for n in range(N):
+        if lens[n]:
+            _close(got[offs[n]:offs[n] + lens[n]], ref_out[n, :lens[n]], f"conv row {n}", atol=atol, ulps=2)
+    if history:
+        np.testing.assert_array_equal(_np(pool_d), ref_pool)

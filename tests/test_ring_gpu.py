@@ -438,3 +438,40 @@ def test_query_tiles_match_oracle(G, W):
     _check(_np(out), ref)
     for n, k in enumerate(lens):
         assert torch.count_nonzero(out[n, k:]).item() == 0
+
+
+@pytest.mark.parametrize("lens,W,G", [([1, 17], 512, 4), ([600, 35], 512, 4), ([130, 16, 0, 64], 48, 8)])
+def test_window_attention_of_sequences(lens, W, G):
+    """hsg_window_attention: packed rows over their own keys at the edges of tiles, groups and windows, against the
+    masked softmax in float64; a second call that cuts the rows into two launches gives the same bits."""
+    from hs_guard._lib import lib
+    print(f"[ring] window attention {lens} W={W} G={G}", flush=True)
+    gen = torch.Generator().manual_seed(50 + G)
+    Hkv, D, T = 2, 256, sum(lens)
+    dev = torch.device("cuda:0")
+    q = torch.randn(T, Hkv, G, D, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(T, Hkv, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    gate = torch.randn(T, Hkv, G, D, generator=gen).to(torch.bfloat16)
+    ref = torch.zeros(T, Hkv, G, D, dtype=torch.float64)
+    offs = [sum(lens[:i]) for i in range(len(lens))]
+    for o, n in zip(offs, lens):
+        i = torch.arange(n)
+        ok = (i[None] <= i[:, None]) & (i[None] > i[:, None] - W)
+        s = torch.einsum("ihgd,jhd->hgij", q[o:o + n].double(), k[o:o + n].double()) * D ** -0.5
+        pr = torch.softmax(s.masked_fill(~ok, -torch.inf), -1)
+        ref[o:o + n] = torch.einsum("hgij,jhd->ihgd", pr, v[o:o + n].double())
+    ref = ref * torch.sigmoid(gate.double())
+    d = [x.to(dev) for x in (q, k, v, gate)]
+    lens_d, offs_d = torch.tensor(lens, device=dev), torch.tensor(offs, device=dev)
+    outs = []
+    for cuts in ([(0, max(lens))], [(0, 64), (64, max(lens))]):
+        out = torch.zeros(T, Hkv, G, D, dtype=torch.bfloat16, device=dev)
+        for first, count in cuts:
+            rc = lib().hsg_window_attention(
+                d[0].data_ptr(), Hkv * G * D, G * D, D, d[1].data_ptr(), Hkv * D, D, d[2].data_ptr(), Hkv * D, D,
+                d[3].data_ptr(), Hkv * G * D, G * D, D, 0, lens_d.data_ptr(), offs_d.data_ptr(), len(lens), max(lens),
+                first, count, W, Hkv, G, D, D ** -0.5, out.data_ptr(), Hkv * G * D, G * D, D, None)
+            assert rc == 0
+        outs.append(out)
+    _check(_np(outs[0]), ref.numpy())
+    assert torch.equal(outs[0], outs[1])
