@@ -140,11 +140,15 @@ __device__ __forceinline__ float pow2_scale(float amax, float* inv) {
   return __uint_as_float((uint32_t)(127 + e) << 23);
 }
 
-// y = x * scale (scale a power of two) as fp16 hi + fp16 lo of the remainder: y = hi + lo + O(2^-22 |y|)
+// y = x * scale (scale a power of two) as fp16 hi + fp16 lo of the remainder: y = hi + lo + O(2^-22 |y|). The remainder
+// is one fused multiply-add rounded to fp16 (v_fma_mixlo / mixhi_f16): x scale - hi, exact before the rounding.
 __device__ __forceinline__ void split4h(f32x4 x, float scale, s16x4& hi, s16x4& lo) {
-  const f32x4 y = x * scale;
-  const f16x4 h = __builtin_convertvector(y, f16x4);
-  const f16x4 l = __builtin_convertvector(y - __builtin_convertvector(h, f32x4), f16x4);
+  f16x4 h, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    h[i] = (_Float16)(x[i] * scale);
+    l[i] = (_Float16)__builtin_fmaf(x[i], scale, -(float)h[i]);
+  }
   hi = __builtin_bit_cast(s16x4, h);
   lo = __builtin_bit_cast(s16x4, l);
 }
@@ -173,6 +177,7 @@ __device__ __forceinline__ u32x4 bf16x8_to_f16x8(u32x4 w) {
 __device__ __forceinline__ s16x8 cat(s16x4 x, s16x4 y) { return __builtin_shufflevector(x, y, 0, 1, 2, 3, 4, 5, 6, 7); }
 
 __device__ __forceinline__ f32x4 ld4f(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
+__device__ __forceinline__ s16x8 ld8h(const uint16_t* p) { return *reinterpret_cast<const s16x8*>(p); }
 __device__ __forceinline__ s16x4 ld4h(const uint16_t* p) { return *reinterpret_cast<const s16x4*>(p); }
 
 // e^x for x <= 0 given in fp64, on the hardware exp2 (v_exp_f32, 1 ulp): x log2 e = n + f is split in fp64 (n
@@ -193,39 +198,38 @@ __device__ __forceinline__ s16x4 ld4h_tr(const uint16_t* p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(p));
 }
 
-// The state kernel's K and Q tiles are unpadded 256-byte token rows whose 8-byte pieces are permuted within each
-// row: logical piece c of row r is stored at piece c ^ swz(r). A row read (16 lanes: 16 consecutive rows, one
-// piece) and a transpose read (16 lanes: 4 rows x 4 consecutive pieces) then both touch 16 distinct 8-byte bank
-// pairs, where any padding of the row leaves one of the two patterns with 2- to 4-way bank conflicts.
+// Rows of keys (K, Q) and of token columns (the M' and P planes) in LDS. An MFMA operand of 32 reduction slots takes, for
+// lane group g, the 8-byte pieces 4 J + g and 4 (J + 1) + g of a row (4 columns each of 16-column blocks J and J + 1, J
+// even); the two are kept adjacent, so one 16-byte read yields the operand (two 8-byte reads took a move per register to
+// assemble it: 151 of the state kernel's 279; with the split's remainders on one fma each, 16 rows of 512 to 8,000 tokens
+// 611 -> 586 us of state kernel, one of 8,000 457 -> 444): 8-byte piece c = 4 J + g is half J % 2 of 16-byte slot
+// 4 (J / 2) + g. Slots are permuted within the row.
+// K and Q (256-byte rows): slot s of row r at s ^ swz(r). A row read (16 lanes: 16 consecutive rows, one slot) and a
+// transpose read (16 lanes: 4 rows x 4 consecutive slots, one half) then both touch 16 distinct slots.
 __device__ __forceinline__ int swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
 
-// offset (bf16) of logical 4-element piece c in swizzled row r
-__device__ __forceinline__ int swz_at(int r, int c) { return r * KD + 4 * (c ^ swz(r)); }
+// offset (bf16) of slot s in swizzled row r
+__device__ __forceinline__ int swz_at(int r, int s) { return r * KD + 8 * (s ^ swz(r)); }
 
-// the same for the 64-column planes M' and P (16 pieces per row; the XOR permutes all of them)
-__device__ __forceinline__ int pw_at(int r, int c) { return r * PW + 4 * (c ^ swz(r)); }
+// the planes (128-byte rows): slot s of row r at s ^ (r / 2 mod 8), so a row read's 16 rows touch 16 distinct slots of two
+// rows' banks. Offset of slot s, and of 8-byte piece c, in row r:
+__device__ __forceinline__ int pw_slot(int r, int s) { return r * PW + 8 * (s ^ ((r >> 1) & 7)); }
+__device__ __forceinline__ int pw_at(int r, int c) { return pw_slot(r, 4 * (c >> 3) + (c & 3)) + 4 * ((c >> 2) & 1); }
 
-// The lower-triangle blocks of a plane pair (hi then lo plane) are the only part of M' and P the state kernel
-// reads: 320 16-byte slots per plane, row block I holding 2 (I + 1) slots per row. Slot q of the pair holds 16-byte
-// piece k of its row's lower triangle, i.e. logical pieces 4 (k / 2) .. +3, whose physical 16-byte slot is
-// 2 ((k / 2) ^ (swz(row) >> 2)) + k % 2 (the XOR keeps aligned groups of four). Returns its offset (bf16) in
-// the pair.
-constexpr int TRI_SLOTS = 320;
+// The slots of a plane pair (hi then lo plane) that hold lower-triangle blocks are all of M' and P that the state kernel
+// reads: 4 per row of row blocks 0 and 1, 8 of blocks 2 and 3 (block (2 I, 2 I + 1) rides along above the diagonal).
+// Returns the offset (bf16) of the pair's q-th.
+constexpr int TRI_SLOTS = 384;
 __device__ __forceinline__ int tri_slot_offset(int q) {
   const int e = q >= TRI_SLOTS;
   const int qq = q - TRI_SLOTS * e;
-  const int I = qq >= 192 ? 3 : qq >= 96 ? 2 : qq >= 32 ? 1 : 0;
-  const int n2 = 2 * (I + 1);
-  const int q2 = qq - (I == 3 ? 192 : I == 2 ? 96 : I == 1 ? 32 : 0);
-  const int row = 16 * I + q2 / n2;
-  const int k = q2 - (q2 / n2) * n2;
-  return e * PL + row * PW + 8 * (2 * ((k >> 1) ^ (swz(row) >> 2)) + (k & 1));
+  return e * PL + (qq < 128 ? pw_slot(qq >> 2, qq & 3) : pw_slot(32 + ((qq - 128) >> 3), qq & 7));
 }
 
 // acc += sum_{J < NJ} M[row block I][col block J] . B_J for a matrix M kept in LDS as scaled fp16 hi / lo planes
-// (swizzled rows): hrow / lrow = row 16 I + m of the hi / lo planes, po[J] = offset of the lane's logical piece
-// 4 J + g in that row (rows 16 I + m share swz(m)); B_J are scaled fp16 hi / lo pairs in B layout. Three passes per
-// product (lo.hi + hi.lo + hi.hi). TR: the same operands with the MFMA operand order swapped, which yields the
+// (swizzled rows): hrow / lrow = row 16 I + m of the hi / lo planes, po[j] = offset in that row of the lane's slot of
+// blocks 2 j, 2 j + 1 (rows 16 I + m share the permutation of m); B_J are scaled fp16 hi / lo pairs in B layout. Three
+// passes per product (lo.hi + hi.lo + hi.hi). TR: the same operands with the MFMA operand order swapped, which yields the
 // transposed product (sum_J B_J^T M_IJ^T) in accumulator layout. The odd block rides in a 16x16x32 product with
 // zero upper k-slots: one accumulation chain never mixes MFMA shapes (a 16x16x16 accumulating onto a 16x16x32
 // result lost that result in some rows).
@@ -235,8 +239,7 @@ __device__ __forceinline__ f32x4 split_product_sw(const uint16_t* hrow, const ui
   auto mm = [](s16x8 m, s16x8 b, f32x4 c) { return TR ? mmh32(b, m, c) : mmh32(m, b, c); };
 #pragma unroll
   for (int J = 0; J + 1 < NJ; J += 2) {
-    const s16x8 ah = cat(ld4h(hrow + po[J]), ld4h(hrow + po[J + 1]));
-    const s16x8 al = cat(ld4h(lrow + po[J]), ld4h(lrow + po[J + 1]));
+    const s16x8 ah = ld8h(hrow + po[J / 2]), al = ld8h(lrow + po[J / 2]);
     const s16x8 b_h = cat(bh[J], bh[J + 1]), b_l = cat(bl[J], bl[J + 1]);
     acc = mm(al, b_h, acc);
     acc = mm(ah, b_l, acc);
@@ -245,7 +248,7 @@ __device__ __forceinline__ f32x4 split_product_sw(const uint16_t* hrow, const ui
   if constexpr (NJ % 2 == 1) {
     constexpr int J = NJ - 1;
     const s16x4 z = {0, 0, 0, 0};
-    const s16x8 ah = cat(ld4h(hrow + po[J]), z), al = cat(ld4h(lrow + po[J]), z);
+    const s16x8 ah = cat(ld4h(hrow + po[J / 2]), z), al = cat(ld4h(lrow + po[J / 2]), z);
     const s16x8 b_h = cat(bh[J], z), b_l = cat(bl[J], z);
     acc = mm(al, b_h, acc);
     acc = mm(ah, b_l, acc);
@@ -553,14 +556,11 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
   }
   lds_barrier();
   // the two planes have the same swizzled rows in LDS and in the workspace: a copy of the lower-triangle slots,
-  // all that the state kernel reads (640 of the pair's 1,024 16-byte pieces)
+  // all that the state kernel reads (768 of the pair's 1,024 16-byte pieces)
 #pragma unroll
-  for (int i = 0; i < (2 * TRI_SLOTS + 255) / 256; ++i) {
-    const int q = threadIdx.x + 256 * i;
-    if (q < 2 * TRI_SLOTS) {
-      const int off = tri_slot_offset(q);
-      *reinterpret_cast<u32x4*>(Mh_g + off) = *reinterpret_cast<const u32x4*>(Mh_s + off);
-    }
+  for (int i = 0; i < 2 * TRI_SLOTS / 256; ++i) {
+    const int off = tri_slot_offset(threadIdx.x + 256 * i);
+    *reinterpret_cast<u32x4*>(Mh_g + off) = *reinterpret_cast<const u32x4*>(Mh_s + off);
   }
 }
 
@@ -664,21 +664,21 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       for (int r = 0; r < 4; ++r) S[mt][r] = load_state<ST>(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD);
   }
 
-  // ---- swizzled K / Q read offsets (bf16), fixed per lane. Logical piece c of row r sits at c ^ swz(r), and
-  // the XOR touches only the low four bits of c, so bit 4 of c (64 bf16) and the row block (16 rows, whose
-  // swz is the same) are plain offsets added at the read.
-  // yo[2 b + h]: row m16, logical piece g4 + 4 h + 8 b (the row reads of Y and Q S);
-  // ko[u]:       row kr = 4 g4 + m16 / 4, logical piece 4 u + m16 % 4 (the transpose reads of K^T). ----
-  // po[J]:       plane row m16, logical piece 4 J + g4 (the row reads of M' and P). ----
-  int yo[4], ko[4], po[4];
+  // ---- read offsets (bf16), fixed per lane; a row block (16 rows) is a plain offset added at the read (its rows'
+  // permutations repeat).
+  // yo[q]: row m16, slot 4 q + g4 (the row reads of Y and Q S: key blocks 2 q, 2 q + 1);
+  // ko[q]: row kr = 4 g4 + m16 / 4, slot 4 q + m16 % 4 (the transpose reads of K^T: key block 2 q, 2 q + 1 4 on). ----
+  // po[j]: plane row m16, slot 4 j + g4 (the row reads of M' and P). ----
+  int yo[4], ko[4], po[2];
   {
     const int kr = 4 * g4 + (m16 >> 2);
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      yo[u] = swz_at(m16, g4 + 4 * (u & 1) + 8 * (u >> 1));
+      yo[u] = swz_at(m16, 4 * u + g4);
       ko[u] = swz_at(kr, 4 * u + (m16 & 3));
-      po[u] = 4 * ((4 * u + g4) ^ swz(m16));
     }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) po[u] = pw_slot(m16, 4 * u + g4) - m16 * PW;
   }
 
   // ---- staging: thread x of a role (x = threadIdx.x % 256) handles token st_t = x / 4 of the chunk: 16-byte
@@ -693,18 +693,18 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
   // the lower-triangle slots of a plane pair this thread stages (tri_slot_offset)
   int qoff[3];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) qoff[i] = tri_slot_offset(min(rx + 256 * i, 2 * TRI_SLOTS - 1));
-  const bool third = rx + 512 < 2 * TRI_SLOTS;
+  for (int i = 0; i < 3; ++i) qoff[i] = tri_slot_offset(rx + 256 * i);
+  static_assert(2 * TRI_SLOTS == 3 * 256, "three plane slots per thread");
   auto row_of = [&](int c0) { return p.qkv + (tok0 + (c0 + st_t < ntok ? c0 + st_t : 0)) * p.qkv_stride; };
-  // 16-byte piece j of a K / Q row holds logical 8-byte pieces 2j, 2j + 1: it lands in 16-byte slot
-  // j ^ (swz >> 1), its halves exchanged when swz is odd. The raw bf16 values are staged as fp16 (exact).
+  // 16-byte piece sp + 4 j of a K / Q row holds 8-byte pieces 4 J + g, 4 J + g + 1 with J = 2 j + sp / 2, g = 2 (sp % 2):
+  // half sp / 2 of slots 4 j + g and 4 j + g + 1. The raw bf16 values are staged as fp16 (exact).
   auto stage_rows = [&](uint16_t* tile, const u32x4* pr) {
-    const int sg = swz(st_t);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int at = st_t * KD + 8 * ((sp + 4 * j) ^ (sg >> 1));
       const u32x4 h = bf16x8_to_f16x8(pr[j]);
-      *reinterpret_cast<u32x4*>(&tile[at]) = (sg & 1) ? h.zwxy : h;
+      const int s0 = 4 * j + 2 * (sp & 1);
+      *reinterpret_cast<u32x2*>(&tile[swz_at(st_t, s0) + 4 * (sp >> 1)]) = h.xy;
+      *reinterpret_cast<u32x2*>(&tile[swz_at(st_t, s0 + 1) + 4 * (sp >> 1)]) = h.zw;
     }
   };
   uint16_t* const sx = Sx + w * 16 * XP + 4 * lane;
@@ -727,7 +727,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       stage_rows(Ks[buf], pk);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        if (i < 2 || third) *reinterpret_cast<u32x4*>(Ms + qoff[i]) = pm[i];
+        *reinterpret_cast<u32x4*>(Ms + qoff[i]) = pm[i];
       vec_s[buf][rx] = pf;
     };
     fetch(0);
@@ -763,9 +763,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
         f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q2 = 0; q2 < 4; ++q2) {
-          const int a0 = yo[2 * (q2 & 1)] + 64 * (q2 >> 1) + 16 * I * KD;
-          const int a1 = yo[2 * (q2 & 1) + 1] + 64 * (q2 >> 1) + 16 * I * KD;
-          const s16x8 ka = cat(ld4h(K_ + a0), ld4h(K_ + a1));
+          const s16x8 ka = ld8h(K_ + yo[q2] + 16 * I * KD);
           y = mmh32(ka, cat(Sl[2 * q2], Sl[2 * q2 + 1]), y);
           y = mmh32(ka, cat(Sh[2 * q2], Sh[2 * q2 + 1]), y);
         }
@@ -840,7 +838,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        const int ka0 = ko[mt & 3] + 64 * (mt >> 2);
+        const int ka0 = ko[mt >> 1] + 4 * (mt & 1);
 #pragma unroll
         for (int J = 0; J < 4; J += 2) {
           const s16x8 ka = cat(ld4h_tr(K_ + ka0 + 16 * J * KD), ld4h_tr(K_ + ka0 + 16 * (J + 1) * KD));
@@ -877,7 +875,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4*>(&Vs[st_t * VS + 8 * (sp + 4 * j)]) = pv[j];
 #pragma unroll
       for (int i = 0; i < 3; ++i)
-        if (i < 2 || third) *reinterpret_cast<u32x4*>(Ps[buf] + qoff[i]) = pp[i];
+        *reinterpret_cast<u32x4*>(Ps[buf] + qoff[i]) = pp[i];
     };
     fetch(0);
     stage(0);
@@ -903,9 +901,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
         f32x4 qs = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int q2 = 0; q2 < 4; ++q2) {
-          const int a0 = yo[2 * (q2 & 1)] + 64 * (q2 >> 1) + 16 * I * KD;
-          const int a1 = yo[2 * (q2 & 1) + 1] + 64 * (q2 >> 1) + 16 * I * KD;
-          const s16x8 qa = cat(ld4h(Qs + a0), ld4h(Qs + a1));
+          const s16x8 qa = ld8h(Qs + yo[q2] + 16 * I * KD);
           qs = mmh32(cat(Sl[2 * q2], Sl[2 * q2 + 1]), qa, qs);
           qs = mmh32(cat(Sh[2 * q2], Sh[2 * q2 + 1]), qa, qs);
         }
