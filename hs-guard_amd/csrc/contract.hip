@@ -6,9 +6,14 @@
 // rounding points of src/hs_guard/engine/fused_kernels.py.
 //
 // Every kernel here is element-wise once the per-row variance is given, so each thread owns VEC consecutive
-// elements of one row (VEC = 4: 8-byte bf16 loads and 16-byte fp32 stores, used when the row width and every
-// pointer allow it; VEC = 1 otherwise), and rows of any width and count work.
+// elements of one row: the most of 8 (16-byte bf16 loads), 4 and 1 that the row width and every pointer and stride
+// allow, so rows of any width and count work. The vector forms need a flat index of 31 bits (a cheap division).
+// They move each byte once and are bound by that and, below ~10 MB, by the launch. At 1,473 tokens norm_rope over 16
+// query and 4 key heads (two launches) takes 14.9 us, 38.5 with one element per thread; the others, cache-resident at
+// that size, gain up to a fifth from 8 elements over 4 (rms_finish 4.2 -> 3.5 us) or stay (silu_mul 8.2).
 #include <math.h>
+
+#include <type_traits>
 
 #include "hsg_common.h"
 
@@ -19,7 +24,9 @@ constexpr int CT_THREADS = 256;
 
 template <int VEC>
 __device__ __forceinline__ void load_bf(const uint16_t* p, float* x) {
-  if constexpr (VEC == 4) {
+  if constexpr (VEC == 8) {
+    load8_bf16(p, x);
+  } else if constexpr (VEC == 4) {
     load4_bf16(p, x);
   } else {
     x[0] = bf2f(p[0]);
@@ -28,7 +35,10 @@ __device__ __forceinline__ void load_bf(const uint16_t* p, float* x) {
 
 template <int VEC>
 __device__ __forceinline__ void store_bf(uint16_t* p, const float* x) {
-  if constexpr (VEC == 4) {
+  if constexpr (VEC == 8) {
+    *reinterpret_cast<u32x4*>(p) = (u32x4){pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]),
+                                           pack_bf16x2(x[6], x[7])};
+  } else if constexpr (VEC == 4) {
     store4_bf16(p, x);
   } else {
     p[0] = f2bf(x[0]);
@@ -37,17 +47,37 @@ __device__ __forceinline__ void store_bf(uint16_t* p, const float* x) {
 
 template <int VEC>
 __device__ __forceinline__ void store_f32(float* p, const float* x) {
-  if constexpr (VEC == 4) {
-    *reinterpret_cast<float4*>(p) = make_float4(x[0], x[1], x[2], x[3]);
-  } else {
+  if constexpr (VEC == 1) {
     p[0] = x[0];
+  } else {
+#pragma unroll
+    for (int e = 0; e < VEC; e += 4) *reinterpret_cast<f32x4_n*>(p + e) = (f32x4_n){x[e], x[e + 1], x[e + 2], x[e + 3]};
   }
 }
 
 template <int VEC>
-__device__ __forceinline__ int64_t first_element(int64_t n) {
-  const int64_t i = ((int64_t)blockIdx.x * CT_THREADS + threadIdx.x) * VEC;
-  return i < n ? i : -1;
+__device__ __forceinline__ void load_f32(const float* p, float* x) {
+  if constexpr (VEC == 1) {
+    x[0] = p[0];
+  } else {
+#pragma unroll
+    for (int e = 0; e < VEC; e += 4) {
+      const f32x4_n v = *reinterpret_cast<const f32x4_n*>(p + e);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[e + k] = v[k];
+    }
+  }
+}
+
+// flat indices: 32-bit in the vector forms
+template <int VEC>
+using index_t = std::conditional_t<VEC == 1, int64_t, uint32_t>;
+
+// the thread's first element, n when it has none
+template <int VEC>
+__device__ __forceinline__ index_t<VEC> first_element(int64_t n) {
+  const index_t<VEC> i = ((index_t<VEC>)blockIdx.x * CT_THREADS + threadIdx.x) * VEC;
+  return i < (index_t<VEC>)n ? i : (index_t<VEC>)n;
 }
 
 // add_square (src/hs_guard/engine/fused_kernels.py:30-52): h = bf16(res + mix) with a plain fp32 add (no
@@ -55,8 +85,8 @@ __device__ __forceinline__ int64_t first_element(int64_t n) {
 template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void add_square_kernel(const uint16_t* res, const uint16_t* mix,
                                                                 uint16_t* out, float* sq, int64_t n) {
-  const int64_t i = first_element<VEC>(n);
-  if (i < 0) return;
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
   float h[VEC];
   load_bf<VEC>(res + i, h);
   if (mix) {
@@ -75,15 +105,16 @@ __global__ __launch_bounds__(CT_THREADS) void add_square_kernel(const uint16_t* 
 template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void rms_finish_kernel(const uint16_t* x, const float* var, const float* w1,
                                                                 float eps, uint16_t* out, int64_t n, int width) {
-  const int64_t i = first_element<VEC>(n);
-  if (i < 0) return;
-  const int64_t row = i / width;
-  const int col = (int)(i - row * width);
-  float h[VEC];
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
+  const index_t<VEC> row = i / (index_t<VEC>)width;
+  const int col = (int)(i - row * (index_t<VEC>)width);
+  float h[VEC], wv[VEC];
   load_bf<VEC>(x + i, h);
+  load_f32<VEC>(w1 + col, wv);
   const float r = rsqrtf(var[row] + eps);
 #pragma unroll
-  for (int e = 0; e < VEC; ++e) h[e] = (h[e] * r) * w1[col + e];
+  for (int e = 0; e < VEC; ++e) h[e] = (h[e] * r) * wv[e];
   store_bf<VEC>(out + i, h);
 }
 
@@ -91,8 +122,8 @@ __global__ __launch_bounds__(CT_THREADS) void rms_finish_kernel(const uint16_t* 
 template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void silu_mul_pair_kernel(const uint16_t* gate, const uint16_t* up,
                                                                    uint16_t* out, int64_t n) {
-  const int64_t i = first_element<VEC>(n);
-  if (i < 0) return;
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
   float g[VEC], u[VEC];
   load_bf<VEC>(gate + i, g);
   load_bf<VEC>(up + i, u);
@@ -106,10 +137,10 @@ template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void gated_finish_kernel(const uint16_t* x, const float* var,
                                                                   const uint16_t* w, const uint16_t* z, float eps,
                                                                   uint16_t* out, int64_t n, int width) {
-  const int64_t i = first_element<VEC>(n);
-  if (i < 0) return;
-  const int64_t row = i / width;
-  const int col = (int)(i - row * width);
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
+  const index_t<VEC> row = i / (index_t<VEC>)width;
+  const int col = (int)(i - row * (index_t<VEC>)width);
   float h[VEC], g[VEC], wv[VEC];
   load_bf<VEC>(x + i, h);
   load_bf<VEC>(z + i, g);
@@ -126,11 +157,11 @@ template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void square_rows_kernel(const uint16_t* src, float* sq, int heads,
                                                                  int64_t row_stride, int64_t head_stride, int dim,
                                                                  int64_t n) {
-  const int64_t i = first_element<VEC>(n);
-  if (i < 0) return;
-  const int64_t r = i / dim;
-  const int c = (int)(i - r * dim);
-  const int64_t token = r / heads;
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
+  const index_t<VEC> r = i / (index_t<VEC>)dim;
+  const int c = (int)(i - r * (index_t<VEC>)dim);
+  const int64_t token = r / (index_t<VEC>)heads;
   const int j = (int)(r - token * heads);
   float x[VEC];
   load_bf<VEC>(src + token * row_stride + j * head_stride + c, x);
@@ -144,47 +175,70 @@ __global__ __launch_bounds__(CT_THREADS) void square_rows_kernel(const uint16_t*
 //   x = bf16((src[d] * rsqrt(var + eps)) * w1[d]), xp the same at d's partner (d +- rot/2),
 //   out[d] = bf16(bf16(x * cos) + bf16(+-xp * sin)) for d < rot, bf16(x) beyond,
 // written at out + n*out_n + (j / groups)*out_h + ((j % groups)*lb + l)*out_row + d for head j of token n*lb + l.
-// One thread per element; the partner is a second (cached) load of the same row.
+// A thread's VEC elements lie in one half of the rotary dims (or beyond them); their partners are a second (cached) load
+// of the same row.
+template <int VEC>
 __global__ __launch_bounds__(CT_THREADS) void norm_rope_grouped_kernel(
     const uint16_t* src, const float* var, const float* w1, const uint16_t* cosv, const uint16_t* sinv, int rot,
     float eps, int heads, int lb, int groups, int64_t row_stride, int64_t head_stride, int dim, uint16_t* out,
     int64_t out_n, int64_t out_h, int64_t out_row, int64_t n) {
-  const int64_t i = first_element<1>(n);
-  if (i < 0) return;
-  const int64_t r = i / dim;
-  const int d = (int)(i - r * dim);
-  const int64_t token = r / heads;
-  const int j = (int)(r - token * heads);
-  const int64_t nn = token / lb;
-  const int l = (int)(token - nn * lb);
+  const index_t<VEC> i = first_element<VEC>(n);
+  if (i == (index_t<VEC>)n) return;
+  const index_t<VEC> r = i / (index_t<VEC>)dim;
+  const int d = (int)(i - r * (index_t<VEC>)dim);
+  const index_t<VEC> token = r / (index_t<VEC>)heads;
+  const int j = (int)(r - token * (index_t<VEC>)heads);
+  const index_t<VEC> nn = token / (index_t<VEC>)lb;
+  const int l = (int)(token - nn * (index_t<VEC>)lb);
   const int half = rot / 2;
   const int partner = d < half ? d + half : (d < rot ? d - half : d);
   const float rr = rsqrtf(var[r] + eps);
-  const uint16_t* base = src + token * row_stride + j * head_stride;
-  const float x = rbf((bf2f(base[d]) * rr) * w1[d]);
-  float y = x;
+  const uint16_t* base = src + (int64_t)token * row_stride + j * head_stride;
+  float x[VEC], wv[VEC];
+  load_bf<VEC>(base + d, x);
+  load_f32<VEC>(w1 + d, wv);
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) x[e] = rbf((x[e] * rr) * wv[e]);
   if (d < rot) {
-    const float xp = rbf((bf2f(base[partner]) * rr) * w1[partner]);
-    const float c = bf2f(cosv[token * rot + d]);
-    const float s = bf2f(sinv[token * rot + d]);
-    const float rh = d < half ? -xp : xp;
-    y = __fadd_rn(rbf(x * c), rbf(rh * s));
+    float xp[VEC], c[VEC], s[VEC];
+    load_bf<VEC>(base + partner, xp);
+    load_f32<VEC>(w1 + partner, wv);
+    load_bf<VEC>(cosv + (int64_t)token * rot + d, c);
+    load_bf<VEC>(sinv + (int64_t)token * rot + d, s);
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+      xp[e] = rbf((xp[e] * rr) * wv[e]);
+      const float rh = d < half ? -xp[e] : xp[e];
+      x[e] = __fadd_rn(rbf(x[e] * c[e]), rbf(rh * s[e]));
+    }
   }
-  out[nn * out_n + (j / groups) * out_h + ((int64_t)(j % groups) * lb + l) * out_row + d] = f2bf(y);
+  store_bf<VEC>(out + (int64_t)nn * out_n + (j / groups) * out_h + ((int64_t)(j % groups) * lb + l) * out_row + d, x);
 }
 
-unsigned blocks_for(int64_t n, int vec) {
-  return (unsigned)((n / vec + CT_THREADS - 1) / CT_THREADS);
-}
-
-// VEC = 4 needs rows of a multiple of 4 elements and 8-byte aligned bf16 / 16-byte aligned fp32 pointers
-bool vec4_ok(int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32) {
-  if (width % 4) return false;
-  for (const void* p : bf)
-    if (p && !aligned(p, 8)) return false;
+// Elements per thread of a call over n elements in rows of `width`, given its bf16 and fp32 pointers and its strides: bf16
+// pieces of VEC elements and fp32 pieces of 4 are aligned to their size.
+int vec_of(int64_t n, int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32,
+           std::initializer_list<int64_t> strides = {}) {
+  if (n >= (1ll << 31)) return 1;
   for (const void* p : f32)
-    if (p && !aligned(p, 16)) return false;
-  return true;
+    if (p && !aligned(p, 16)) return 1;
+  for (int vec : {8, 4}) {
+    bool ok = width % vec == 0;
+    for (const void* p : bf) ok = ok && (!p || aligned(p, 2 * vec));
+    for (int64_t s : strides) ok = ok && s % vec == 0;
+    if (ok) return vec;
+  }
+  return 1;
+}
+
+// launch(vec constant, grid) for the chosen vector width
+template <typename Launch>
+int launch_vec(int vec, int64_t n, Launch launch) {
+  const dim3 grid((unsigned)((n / vec + CT_THREADS - 1) / CT_THREADS));
+  if (vec == 8) launch(std::integral_constant<int, 8>{}, grid);
+  else if (vec == 4) launch(std::integral_constant<int, 4>{}, grid);
+  else launch(std::integral_constant<int, 1>{}, grid);
+  return launch_status();
 }
 
 }  // namespace
@@ -202,11 +256,9 @@ extern "C" int hsg_add_square(const void* residual, const void* mixed, void* out
   const auto* r = static_cast<const uint16_t*>(residual);
   const auto* m = static_cast<const uint16_t*>(mixed);
   auto* o = static_cast<uint16_t*>(out);
-  if (vec4_ok(width, {residual, mixed, out}, {sq}))
-    hipLaunchKernelGGL(add_square_kernel<4>, dim3(blocks_for(n, 4)), dim3(CT_THREADS), 0, s, r, m, o, sq, n);
-  else
-    hipLaunchKernelGGL(add_square_kernel<1>, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0, s, r, m, o, sq, n);
-  return launch_status();
+  return launch_vec(vec_of(n, width, {residual, mixed, out}, {sq}), n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(add_square_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, r, m, o, sq, n);
+  });
 }
 
 extern "C" int hsg_rms_finish(const void* x, const float* var, const float* w1, float eps, void* out, int64_t rows,
@@ -218,13 +270,9 @@ extern "C" int hsg_rms_finish(const void* x, const float* var, const float* w1, 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* xi = static_cast<const uint16_t*>(x);
   auto* o = static_cast<uint16_t*>(out);
-  if (vec4_ok(width, {x, out}, {}))
-    hipLaunchKernelGGL(rms_finish_kernel<4>, dim3(blocks_for(n, 4)), dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n,
-                       width);
-  else
-    hipLaunchKernelGGL(rms_finish_kernel<1>, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n,
-                       width);
-  return launch_status();
+  return launch_vec(vec_of(n, width, {x, out}, {w1}), n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(rms_finish_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n, width);
+  });
 }
 
 extern "C" int hsg_silu_mul_pair(const void* gate, const void* up, void* out, int64_t n, void* stream) {
@@ -235,11 +283,9 @@ extern "C" int hsg_silu_mul_pair(const void* gate, const void* up, void* out, in
   const auto* g = static_cast<const uint16_t*>(gate);
   const auto* u = static_cast<const uint16_t*>(up);
   auto* o = static_cast<uint16_t*>(out);
-  if (vec4_ok(n, {gate, up, out}, {}))
-    hipLaunchKernelGGL(silu_mul_pair_kernel<4>, dim3(blocks_for(n, 4)), dim3(CT_THREADS), 0, s, g, u, o, n);
-  else
-    hipLaunchKernelGGL(silu_mul_pair_kernel<1>, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0, s, g, u, o, n);
-  return launch_status();
+  return launch_vec(vec_of(n, n, {gate, up, out}, {}), n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(silu_mul_pair_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, g, u, o, n);
+  });
 }
 
 extern "C" int hsg_gated_finish(const void* x, const float* var, const void* weight, const void* z, float eps,
@@ -253,13 +299,9 @@ extern "C" int hsg_gated_finish(const void* x, const float* var, const void* wei
   const auto* w = static_cast<const uint16_t*>(weight);
   const auto* zi = static_cast<const uint16_t*>(z);
   auto* o = static_cast<uint16_t*>(out);
-  if (vec4_ok(width, {x, weight, z, out}, {}))
-    hipLaunchKernelGGL(gated_finish_kernel<4>, dim3(blocks_for(n, 4)), dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o,
-                       n, width);
-  else
-    hipLaunchKernelGGL(gated_finish_kernel<1>, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o,
-                       n, width);
-  return launch_status();
+  return launch_vec(vec_of(n, width, {x, weight, z, out}, {}), n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(gated_finish_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o, n, width);
+  });
 }
 
 extern "C" int hsg_square_rows(const void* src, float* sq, int64_t tokens, int32_t heads, int64_t row_stride,
@@ -270,13 +312,9 @@ extern "C" int hsg_square_rows(const void* src, float* sq, int64_t tokens, int32
   const int64_t n = tokens * heads * dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* x = static_cast<const uint16_t*>(src);
-  if (vec4_ok(dim, {src}, {sq}) && row_stride % 4 == 0 && head_stride % 4 == 0)
-    hipLaunchKernelGGL(square_rows_kernel<4>, dim3(blocks_for(n, 4)), dim3(CT_THREADS), 0, s, x, sq, heads,
-                       row_stride, head_stride, dim, n);
-  else
-    hipLaunchKernelGGL(square_rows_kernel<1>, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0, s, x, sq, heads,
-                       row_stride, head_stride, dim, n);
-  return launch_status();
+  return launch_vec(vec_of(n, dim, {src}, {sq}, {row_stride, head_stride}), n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(square_rows_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, x, sq, heads, row_stride, head_stride, dim, n);
+  });
 }
 
 extern "C" int hsg_norm_rope_grouped(const void* src, const float* var, const float* w1, const void* cos,
@@ -289,9 +327,12 @@ extern "C" int hsg_norm_rope_grouped(const void* src, const float* var, const fl
   if (n_rows == 0) return HSG_OK;
   if (!src || !var || !w1 || !cos || !sin || !out) return HSG_ERR_ARG;
   const int64_t n = (int64_t)n_rows * lb * heads * dim;
-  hipLaunchKernelGGL(norm_rope_grouped_kernel, dim3(blocks_for(n, 1)), dim3(CT_THREADS), 0,
-                     reinterpret_cast<hipStream_t>(stream), static_cast<const uint16_t*>(src), var, w1,
-                     static_cast<const uint16_t*>(cos), static_cast<const uint16_t*>(sin), rot, eps, heads, lb,
-                     groups, row_stride, head_stride, dim, static_cast<uint16_t*>(out), out_n, out_h, out_row, n);
-  return launch_status();
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  return launch_vec(vec_of(n, dim, {src, cos, sin, out}, {w1}, {rot / 2, row_stride, head_stride, out_n, out_h, out_row}),
+                    n, [&](auto vec, dim3 grid) {
+    hipLaunchKernelGGL(norm_rope_grouped_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s,
+                       static_cast<const uint16_t*>(src), var, w1, static_cast<const uint16_t*>(cos),
+                       static_cast<const uint16_t*>(sin), rot, eps, heads, lb, groups, row_stride, head_stride, dim,
+                       static_cast<uint16_t*>(out), out_n, out_h, out_row, n);
+  });
 }

@@ -371,3 +371,25 @@ def test_reference_composition_matches_oracle():
     for s in range(4):
         rel = np.linalg.norm(rec[:, s] - orc.rec[:, s]) / np.linalg.norm(orc.rec[:, s])
         assert rel < 1e-3, f"slot {s} state rel err {rel:.2e}"
+
+
+@pytest.mark.parametrize("dim,rot,shift", [(256, 64, 0), (256, 64, 4), (264, 24, 0), (12, 8, 0), (10, 6, 2)])
+def test_norm_rope_vector_widths(dim, rot, shift):
+    """norm_rope at the widths, rotary sizes and alignments that take 8, 4 and 1 elements per thread, against the oracle
+    (bf16 within one step: the fp32 rsqrt may move a rounding)."""
+    from hs_guard.engine.kernels import norm_rope
+    print(f"[contract] norm_rope dim={dim} rot={rot} shift={shift}", flush=True)
+    rng = np.random.default_rng(dim + rot)
+    n, lb, heads, groups = 3, 5, 6, 3
+    head_stride = dim + shift
+    src = bf16(rng.standard_normal((n * lb, heads * head_stride)))
+    x = src.reshape(n, lb, heads, head_stride)[..., :dim]
+    w1 = (1 + 0.02 * rng.standard_normal(dim)).astype(np.float32)
+    ang = rng.uniform(0, 6, (n, lb, rot // 2))
+    cos, sin = (bf16(np.concatenate([f(ang), f(ang)], -1)) for f in (np.cos, np.sin))
+    var = (x.astype(np.float64) ** 2).mean(-1).astype(np.float32)
+    got = norm_rope(_bf(src), torch.from_numpy(var.reshape(-1)).to(DEV), torch.from_numpy(w1).to(DEV), _bf(cos), _bf(sin),
+                    1e-6, n, lb, heads, groups, heads * head_stride, head_stride, dim)
+    ref = oglue.norm_rope_given(x, var[..., None], w1, 1e-6, cos, sin)
+    ref = ref.reshape(n, lb, heads // groups, groups, dim).transpose(0, 2, 3, 1, 4).reshape(n, heads // groups, groups * lb, dim)
+    _close(_np(got), ref, "norm_rope")
