@@ -166,6 +166,24 @@ def lib():
     return _lib
 
 
+_calls = None
+
+
+def calls():
+    """The C ABI's entry points as native functions (hs_guard._hsgcall), loaded with the library: the same positional
+    arguments and status as ``lib()``'s, without ctypes' per-argument converters. For calls made per launch."""
+    global _calls
+    if _calls is None:
+        lib()
+        try:
+            from . import _hsgcall
+        except ImportError as e:
+            raise RuntimeError(f"HS-Guard native call module not built: {e} "
+                               "(run `python -c 'import __graft_entry__ as g; g.build()'` at the repo root)") from e
+        _calls = _hsgcall
+    return _calls
+
+
 def check(rc, name):
     """Map a non-zero return code of an hsg_* call to an exception (ValueError for rejected arguments)."""
     if rc == 0:

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import torch
 
-from .._lib import HSG_GDN_BURST_MIN_DEFAULT, check, lib
+from .._lib import HSG_GDN_BURST_MIN_DEFAULT, calls, check, lib
 
 HSG_STATE_F32 = 0
 HSG_STATE_F16 = 1
@@ -25,19 +25,30 @@ def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
-def _stream(device):
-    return torch.cuda.current_stream(device).cuda_stream
+# The address of the current stream of a GPU tensor's device. torch.cuda.current_stream builds a Stream object for it,
+# 1.5 us of a call whose kernel takes 5.
+_current_stream = torch._C._cuda_getCurrentRawStream
+
+
+def _stream(t):
+    index = t.get_device()
+    if index < 0:
+        raise ValueError(f"Expected a GPU tensor, got one on {t.device}")
+    return _current_stream(index)
 
 
 def _gpu(*tensors):
     for t in tensors:
-        _require(t is None or t.is_cuda, "HS-Guard kernels take GPU tensors")
+        if not (t is None or t.is_cuda):
+            raise AssertionError("HS-Guard kernels take GPU tensors")
 
 
 def _bf16_in(*tensors):
     for t in tensors:
-        _require(t.dtype == torch.bfloat16, "bf16 tensors expected")
-        _require(t.is_contiguous(), "tensors must be contiguous")
+        if t.dtype is not torch.bfloat16:
+            raise AssertionError("bf16 tensors expected")
+        if not t.is_contiguous():
+            raise AssertionError("tensors must be contiguous")
 
 
 def add_square(residual, mixed=None):
@@ -47,10 +58,11 @@ def add_square(residual, mixed=None):
     _bf16_in(residual, *(() if mixed is None else (mixed,)))
     _require(mixed is None or mixed.shape == residual.shape, "residual and mixed must have one shape")
     n = residual.shape[-1]
-    sq = torch.empty(residual.shape, dtype=torch.float32, device=residual.device)
+    sq = torch.empty_like(residual, dtype=torch.float32)
     out = residual if mixed is None else torch.empty_like(residual)
-    check(lib().hsg_add_square(_ptr(residual), _ptr(mixed), None if mixed is None else _ptr(out), _ptr(sq),
-                               residual.numel() // n, n, _stream(residual.device)), "hsg_add_square")
+    rc = calls().hsg_add_square(_ptr(residual), _ptr(mixed), None if mixed is None else _ptr(out), _ptr(sq),
+                                residual.numel() // n, n, _stream(residual))
+    check(rc, "hsg_add_square")
     return out, sq
 
 
@@ -64,8 +76,9 @@ def rms_finish(x, var, w1, eps):
     _require(var.dtype == torch.float32 and var.is_contiguous() and var.numel() == rows, "var must be [rows] fp32")
     _require(w1.dtype == torch.float32 and w1.is_contiguous() and w1.numel() == n, "w1 must be [width] fp32")
     out = torch.empty_like(x)
-    check(lib().hsg_rms_finish(_ptr(x), _ptr(var), _ptr(w1), float(eps), _ptr(out), rows, n,
-                               _stream(x.device)), "hsg_rms_finish")
+    rc = calls().hsg_rms_finish(_ptr(x), _ptr(var), _ptr(w1), float(eps), _ptr(out), rows, n,
+                                _stream(x))
+    check(rc, "hsg_rms_finish")
     return out
 
 
@@ -75,8 +88,8 @@ def silu_mul(gate, up):
     _bf16_in(gate, up)
     _require(gate.shape == up.shape, "gate and up must have one shape")
     out = torch.empty_like(gate)
-    check(lib().hsg_silu_mul_pair(_ptr(gate), _ptr(up), _ptr(out), gate.numel(), _stream(gate.device)),
-          "hsg_silu_mul_pair")
+    rc = calls().hsg_silu_mul_pair(_ptr(gate), _ptr(up), _ptr(out), gate.numel(), _stream(gate))
+    check(rc, "hsg_silu_mul_pair")
     return out
 
 
@@ -91,9 +104,9 @@ def conv_silu_update(qkv, pool, weight, slots, lens):
     _gpu(qkv, pool, weight, slots, lens)
     _bf16_in(qkv, pool, weight)
     out = torch.empty_like(qkv)
-    check(lib().hsg_conv_silu_update(_ptr(qkv), c, _ptr(pool), pool.shape[0], _ptr(weight), ks, _ptr(slots),
-                                     _ptr(lens), None, n, length, c, _ptr(out), c, _stream(qkv.device)),
-          "hsg_conv_silu_update")
+    rc = calls().hsg_conv_silu_update(_ptr(qkv), c, _ptr(pool), pool.shape[0], _ptr(weight), ks, _ptr(slots),
+                                      _ptr(lens), None, n, length, c, _ptr(out), c, _stream(qkv))
+    check(rc, "hsg_conv_silu_update")
     return out
 
 
@@ -107,8 +120,9 @@ def gated_finish(x, var, weight, z, eps):
     _require(z.shape == x.shape and weight.numel() == n, "z must match x and weight its last dim")
     _require(var.dtype == torch.float32 and var.is_contiguous() and var.numel() == rows, "var must be [rows] fp32")
     out = torch.empty_like(x)
-    check(lib().hsg_gated_finish(_ptr(x), _ptr(var), _ptr(weight), _ptr(z), float(eps), _ptr(out), rows, n,
-                                 _stream(x.device)), "hsg_gated_finish")
+    rc = calls().hsg_gated_finish(_ptr(x), _ptr(var), _ptr(weight), _ptr(z), float(eps), _ptr(out), rows, n,
+                                  _stream(x))
+    check(rc, "hsg_gated_finish")
     return out
 
 
@@ -119,9 +133,10 @@ def square_rows(src, tokens, heads, row_stride, head_stride, dim):
     _bf16_in(src)
     _require(tokens == 0 or (tokens - 1) * row_stride + (heads - 1) * head_stride + dim <= src.numel(),
              "rows reach past src")
-    sq = torch.empty(tokens, heads, dim, dtype=torch.float32, device=src.device)
-    check(lib().hsg_square_rows(_ptr(src), _ptr(sq), tokens, heads, row_stride, head_stride, dim,
-                                _stream(src.device)), "hsg_square_rows")
+    sq = src.new_empty((tokens, heads, dim), dtype=torch.float32)
+    rc = calls().hsg_square_rows(_ptr(src), _ptr(sq), tokens, heads, row_stride, head_stride, dim,
+                                 _stream(src))
+    check(rc, "hsg_square_rows")
     return sq
 
 
@@ -141,10 +156,11 @@ def norm_rope(src, var, w1, cos, sin, eps, n, lb, heads, groups, row_stride, hea
                                       <= src.numel()), "src must be contiguous and hold every head row")
     _require(heads % groups == 0, "heads must be a multiple of groups")
     rot = cos.shape[-1]
-    out = torch.empty(n, heads // groups, groups * lb, dim, dtype=torch.bfloat16, device=src.device)
-    check(lib().hsg_norm_rope_grouped(_ptr(src), _ptr(var), _ptr(w1), _ptr(cos), _ptr(sin), rot, float(eps), n, lb,
-                                      heads, groups, row_stride, head_stride, dim, _ptr(out), out.stride(0),
-                                      out.stride(1), out.stride(2), _stream(src.device)), "hsg_norm_rope_grouped")
+    out = src.new_empty((n, heads // groups, groups * lb, dim))
+    rc = calls().hsg_norm_rope_grouped(_ptr(src), _ptr(var), _ptr(w1), _ptr(cos), _ptr(sin), rot, float(eps), n, lb,
+                                       heads, groups, row_stride, head_stride, dim, _ptr(out), out.stride(0),
+                                       out.stride(1), out.stride(2), _stream(src))
+    check(rc, "hsg_norm_rope_grouped")
     return out
 
 
@@ -162,12 +178,12 @@ def gdn_slot_v8(packed, key_dim, heads, head_k, value_heads, head_v, a, b, A_log
     _require(packed.dtype == torch.bfloat16, "packed must be bf16")
     _require(state.dtype in _STATE_CODES, "state must be float32 or float16")
     _require(state.shape[1:] == (value_heads, head_k, head_v), "state must be [S, HV, K, V]")
-    o = torch.empty(n, length, value_heads, head_v, dtype=packed.dtype, device=packed.device)
-    sq = torch.empty(o.shape, dtype=torch.float32, device=packed.device)
-    rc = lib().hsg_gdn_slot_step(
+    o = packed.new_empty((n, length, value_heads, head_v))
+    sq = torch.empty_like(o, dtype=torch.float32)
+    rc = calls().hsg_gdn_slot_step(
         _ptr(packed), c, 0, key_dim, 2 * key_dim, _ptr(a), _ptr(b), value_heads, _ptr(A_log), _ptr(dt_bias),
         _ptr(state), _STATE_CODES[state.dtype], state.shape[0], _ptr(slots), _ptr(lens), None, n, length,
-        heads, value_heads, head_k, head_v, head_k ** -0.5, _ptr(o), _ptr(sq), int(burst_min), _stream(packed.device))
+        heads, value_heads, head_k, head_v, head_k ** -0.5, _ptr(o), _ptr(sq), int(burst_min), _stream(packed))
     check(rc, "hsg_gdn_slot_step")
     return o, sq
 
@@ -184,10 +200,10 @@ def gdn_slot_recurrent(q, k, v, a, b, A_log, dt_bias, state, slots, lens, scale=
     scale = kd ** -0.5 if scale is None else scale
     qkv = torch.cat([q.reshape(n, length, -1), k.reshape(n, length, -1), v.reshape(n, length, -1)], -1)
     o = torch.empty(n, length, hv, vd, dtype=v.dtype, device=v.device)
-    rc = lib().hsg_gdn_slot_step(
+    rc = calls().hsg_gdn_slot_step(
         _ptr(qkv), qkv.shape[-1], 0, h * kd, 2 * h * kd, _ptr(a), _ptr(b), hv, _ptr(A_log), _ptr(dt_bias),
         _ptr(state), _STATE_CODES[state.dtype], state.shape[0], _ptr(slots), _ptr(lens), None, n, length,
-        h, hv, kd, vd, scale, _ptr(o), None, int(burst_min), _stream(v.device))
+        h, hv, kd, vd, scale, _ptr(o), None, int(burst_min), _stream(v))
     check(rc, "hsg_gdn_slot_step")
     return o
 
@@ -225,11 +241,11 @@ def gdn_chunk_prefill(packed, key_dim, heads, head_k, value_heads, head_v, a, b,
     if workspace is None:
         workspace = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=packed.device)
     _require(workspace.numel() >= ws_bytes, f"workspace needs {ws_bytes} bytes")
-    rc = lib().hsg_gdn_chunk_prefill(
+    rc = calls().hsg_gdn_chunk_prefill(
         _ptr(packed), c, 0, key_dim, 2 * key_dim, _ptr(a), _ptr(b), value_heads, _ptr(A_log), _ptr(dt_bias),
         _ptr(state), _STATE_CODES[state.dtype], state.shape[0], _ptr(slots), _ptr(lens), _ptr(offsets), n,
         max(length, 1), heads, value_heads, head_k, head_v, scale, _ptr(o), _ptr(sq), 0, _ptr(workspace),
-        workspace.numel(), _stream(packed.device))
+        workspace.numel(), _stream(packed))
     check(rc, "hsg_gdn_chunk_prefill")
     return o, sq
 
@@ -249,13 +265,13 @@ def ring_attention_v8(q, ring_k, ring_v, new_k, value, gate, ring_pos, slots, st
     for tensor in (q, ring_k, ring_v, new_k, value, gate, ring_pos):
         _require(tensor.is_contiguous(), "tensors must be contiguous")
     _gpu(q, ring_k, ring_v, new_k, value, gate, ring_pos, slots, starts, lens)
-    out = torch.empty(n, lb, hkv * groups * d, dtype=torch.bfloat16, device=q.device)
+    out = q.new_empty((n, lb, hkv * groups * d), dtype=torch.bfloat16)
     if lb == 1 and split_k:
         # the split-K kernels (more than 8 query heads per kv head) keep their partial results in a workspace; the
         # fused kernel below that needs none
         ws_bytes = lib().hsg_ring_decode_workspace_bytes(n, hkv, groups, window) if groups > 8 else 0
         ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=q.device)
-        rc = lib().hsg_ring_decode(
+        rc = calls().hsg_ring_decode(
             _ptr(q), hkv * m * d, d, m * d, d,
             _ptr(ring_k), _ptr(ring_v), ring_k.shape[0], window,
             _ptr(new_k), hkv * d, d, d,
@@ -263,10 +279,10 @@ def ring_attention_v8(q, ring_k, ring_v, new_k, value, gate, ring_pos, slots, st
             _ptr(gate), gate.stride(0), gate.stride(1), groups * 2 * d, 2 * d, d,
             _ptr(ring_pos), _ptr(slots), _ptr(starts), _ptr(lens), None,
             n, hkv, groups, d, float(scale), int(bool(write_ring)),
-            _ptr(out), hkv * groups * d, hkv * groups * d, groups * d, d, _ptr(ws), ws.numel(), _stream(q.device))
+            _ptr(out), hkv * groups * d, hkv * groups * d, groups * d, d, _ptr(ws), ws.numel(), _stream(q))
         check(rc, "hsg_ring_decode")
         return out
-    rc = lib().hsg_ring_attention(
+    rc = calls().hsg_ring_attention(
         _ptr(q), hkv * m * d, d, m * d, lb * d,
         _ptr(ring_k), _ptr(ring_v), ring_k.shape[0], window,
         _ptr(new_k), hkv * lb * d, d, lb * d,
@@ -274,7 +290,7 @@ def ring_attention_v8(q, ring_k, ring_v, new_k, value, gate, ring_pos, slots, st
         _ptr(gate), gate.stride(0), gate.stride(1), groups * 2 * d, 2 * d, d,
         _ptr(ring_pos), _ptr(slots), _ptr(starts), _ptr(lens), None,
         n, lb, hkv, groups, d, float(scale), int(bool(write_ring)), 0,
-        _ptr(out), lb * hkv * groups * d, hkv * groups * d, groups * d, d, _stream(q.device))
+        _ptr(out), lb * hkv * groups * d, hkv * groups * d, groups * d, d, _stream(q))
     check(rc, "hsg_ring_attention")
     return out
 
@@ -291,7 +307,7 @@ def ring_attention(q, ring_k, ring_v, new_k, new_v, ring_pos, slots, starts, len
     for tensor in (q, ring_k, ring_v, new_k, new_v, ring_pos):
         _require(tensor.is_contiguous(), "tensors must be contiguous")
     out = torch.empty_like(q)
-    rc = lib().hsg_ring_attention(
+    rc = calls().hsg_ring_attention(
         _ptr(q), hkv * m * d, d, m * d, lb * d,
         _ptr(ring_k), _ptr(ring_v), ring_k.shape[0], window,
         _ptr(new_k), hkv * lb * d, d, lb * d,
@@ -299,6 +315,6 @@ def ring_attention(q, ring_k, ring_v, new_k, new_v, ring_pos, slots, starts, len
         None, 0, 0, 0, 0, 0,
         _ptr(ring_pos), _ptr(slots), _ptr(starts), _ptr(lens), None,
         n, lb, hkv, groups, d, float(scale), 0, 0,
-        _ptr(out), hkv * m * d, d, m * d, lb * d, _stream(q.device))
+        _ptr(out), hkv * m * d, d, m * d, lb * d, _stream(q))
     check(rc, "hsg_ring_attention")
     return out

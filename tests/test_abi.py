@@ -133,3 +133,22 @@ def test_argument_errors_are_rejected_before_launch():
     assert L.hsg_ring_decode_rope(*rope, None, need, None) == -1
     rope[12] = 32
     assert L.hsg_ring_decode_rope(*rope, 256, need, None) == -3
+
+
+def test_native_calls_take_the_same_arguments():
+    """hs_guard._hsgcall: every function's argument count is its ctypes signature's, statuses are the library's, and
+    wrong counts, types and out-of-range integers raise before the call."""
+    from hs_guard._lib import SIGNATURES, calls, lib
+    names = [n for n in dir(calls()) if n.startswith("hsg_")]
+    assert "hsg_gdn_slot_step" in names
+    for name in names:
+        restype, argtypes = SIGNATURES[name]
+        assert restype is ctypes.c_int
+        with pytest.raises(TypeError, match=f"expected {len(argtypes)} arguments, got {len(argtypes) + 1}"):
+            getattr(calls(), name)(*[0] * (len(argtypes) + 1))
+    for args in ((None, None, None, None, 0, 4, None), (None, None, None, None, 1, 4, None), (8, 8, 8, 8, -1, 4, None)):
+        assert calls().hsg_add_square(*args) == lib().hsg_add_square(*args)
+    with pytest.raises(OverflowError):
+        calls().hsg_add_square(None, None, None, None, 1, 1 << 40, None)
+    with pytest.raises(TypeError):
+        calls().hsg_add_square(None, None, None, None, 1, "4", None)
