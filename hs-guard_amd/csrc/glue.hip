@@ -377,7 +377,8 @@ __global__ void ring_pos_kernel(int64_t* ring_pos, int64_t ring_rows, const int6
   if (slot < 0 || slot >= ring_rows || len <= 0) return;
   if (len > lb_max) len = lb_max;
   const int64_t start = starts[n];
-  for (int j = threadIdx.x; j < len; j += blockDim.x) {
+  // of a row longer than the window only its last W steps have columns of their own
+  for (int64_t j = max(len - W, (int64_t)0) + threadIdx.x; j < len; j += blockDim.x) {
     const int64_t p = start + j;
     ring_pos[slot * (W + 1) + p % W] = p;
   }

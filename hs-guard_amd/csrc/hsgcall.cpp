@@ -62,6 +62,7 @@ PyMethodDef methods[] = {HSG_ENTRY(hsg_gdn_slot_step),
                          HSG_ENTRY(hsg_gdn_chunk_prefill),
                          HSG_ENTRY(hsg_ring_attention),
                          HSG_ENTRY(hsg_window_attention),
+                         HSG_ENTRY(hsg_ring_prefill),
                          HSG_ENTRY(hsg_ring_decode),
                          HSG_ENTRY(hsg_embed_rmsnorm),
                          HSG_ENTRY(hsg_add_rmsnorm),
@@ -75,7 +76,17 @@ PyMethodDef methods[] = {HSG_ENTRY(hsg_gdn_slot_step),
                          HSG_ENTRY(hsg_square_rows),
                          HSG_ENTRY(hsg_norm_rope_grouped),
                          HSG_ENTRY(hsg_silu_mul),
+                         HSG_ENTRY(hsg_risk_head),
                          HSG_ENTRY(hsg_risk_head_f32),
+                         HSG_ENTRY(hsg_gdn_slot_step_gated),
+                         HSG_ENTRY(hsg_gdn_conv_slot_step_gated),
+                         HSG_ENTRY(hsg_gdn_chunk_prefill_gated),
+                         HSG_ENTRY(hsg_ring_decode_rope),
+                         HSG_ENTRY(hsg_ring_pos_update),
+                         HSG_ENTRY(hsg_gemm_bf16),
+                         HSG_ENTRY(hsg_gemm_bf16_skinny),
+                         HSG_ENTRY(hsg_gemm_bf16_skinny_silu),
+                         HSG_ENTRY(hsg_gemm_bf16_skinny_addnorm),
                          {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_hsgcall", "Entry points of libhsg.so", -1, methods, nullptr, nullptr, nullptr,

@@ -29,7 +29,8 @@
 // 72 padded rows of 2 to 64 steps 147 -> 92 us (49 us of it whole groups past their rows' lengths, which ran their
 // keys), 64 rows of 4 steps 41.6 -> 28.0 us, one such row 34.9 -> 21.6 us. Splitting the keys of longer rows' tiles too
 // reads K and V once per tile instead of once per group: 72 rows of 64 steps 264 us against 165. A sequence of 8,000
-// tokens (no ring): 203 us, against 270 us over rings gathered from it (and 0.2 ms of gathers).
+// tokens (no ring): 203 us, against 270 us over rings gathered from it (and 0.2 ms of gathers). Three rows of 900 tokens
+// over rings (hsg_ring_prefill): 95 us, against 15 ticks of 25 us.
 #include <math.h>
 
 #include <type_traits>
@@ -69,6 +70,7 @@ struct RingParams {
   int pairs;        // rows x kv heads
   int qgroups;      // workgroups (groups of NW tiles) per (row, kv head)
   int qg0;          // first group
+  int sequences;    // rows of any length: each XCD takes a contiguous eighth of the workgroups
   uint16_t* out; int64_t o_sn, o_sl, o_sh, o_sg;
 };
 
@@ -608,10 +610,10 @@ __global__ __launch_bounds__(NW * 64, 2) void ring_attn_kernel(const RingParams 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Workgroups are dealt round-robin over the 8 XCDs. Ticks: query group slowest, so that consecutive workgroups take
   // consecutive (row, kv head) pairs (the live workgroups of a short-row tick spread over all XCDs, and a pair's
-  // groups share one XCD's L2 when the pairs are a multiple of 8). Sequences (no ring): each XCD takes a
+  // groups share one XCD's L2 when the pairs are a multiple of 8). Sequences: each XCD takes a
   // contiguous eighth of the groups, whose windows overlap.
   int pair, qg;
-  if (p.ring_k) {
+  if (!p.sequences) {
     qg = blockIdx.x / p.pairs;
     pair = blockIdx.x - qg * p.pairs;
   } else {
@@ -642,6 +644,8 @@ __global__ __launch_bounds__(NW * 64, 2) void ring_attn_kernel(const RingParams 
   ro.ring_base = ((ro.slot * p.hkv + h) * (int64_t)(p.W + 1)) * D;
   ro.ring_pos = p.ring_pos + ro.slot * (int64_t)(p.W + 1);
   const int r_lo = qg * (NW * TQ);
+  // a sequence's ring holds only positions before its start, which steps from W - 1 on do not see
+  if (p.sequences && r_lo / p.G >= p.W - 1) ro.RB = 0;
   const int M = p.G * ro.steps, Mv = p.G * ro.len;      // query rows of this (row, kv head), and the valid ones
   // rows past the length of a padded row are zeros; attend_group and attend_tile store those of the tiles they take
   const int tiles = r_lo >= Mv ? 0 : min((Mv - r_lo + TQ - 1) / TQ, NW);
@@ -651,8 +655,9 @@ __global__ __launch_bounds__(NW * 64, 2) void ring_attn_kernel(const RingParams 
     const int l = r / p.G;
     *reinterpret_cast<u32x2*>(ro.orow + l * p.o_sl + (r - l * p.G) * p.o_sg + 4 * (e % (D / 4))) = (u32x2){0u, 0u};
   }
-  if (tiles == 1) attend_tile(p, ro, r_lo, lds.split, lane, wave);
-  else if (tiles > 1) attend_group(p, ro, r_lo, lds.group, lane, wave);
+  // (a tile that may see ring blocks and many new-key blocks could need more than SLOTS of attend_tile's slots)
+  if (tiles == 1 && (ro.RB == 0 || ro.len <= LB_MAX)) attend_tile(p, ro, r_lo, lds.split, lane, wave);
+  else if (tiles > 0) attend_group(p, ro, r_lo, lds.group, lane, wave);
 }
 
 // In-place ring write of the tick's valid keys/values, launched after the attention kernel (whose query
@@ -670,17 +675,18 @@ __global__ __launch_bounds__(256) void ring_write_kernel(const RingParams p) {
   const bool rejected = (slot < 0) | (slot >= p.ring_rows) | (len < 0) | (len > (padded ? LB_MAX : p.lb));
   if (rejected | (!padded & (len < p.min_len))) return;
   if (padded && len > p.lb) len = p.lb;
+  const int64_t first = max(len - p.W, (int64_t)0);   // of a row longer than the window its last W steps stay
   const int64_t base_tok = padded ? 0 : off;
-  const int64_t nk_row = padded ? n * p.nk_sn : base_tok * p.nk_sl;
-  const int64_t nv_row = padded ? n * p.nv_sn : base_tok * p.nv_sl;
+  const int64_t nk_row = (padded ? n * p.nk_sn : base_tok * p.nk_sl) + first * p.nk_sl;
+  const int64_t nv_row = (padded ? n * p.nv_sn : base_tok * p.nv_sl) + first * p.nv_sl;
   const int64_t ring_base = ((slot * p.hkv + h) * (int64_t)(p.W + 1)) * D;
-  const int c0 = (int)(start % p.W);   // ring column of the tick's first step; j < len <= W follow it
+  const int c0 = (int)((start + first) % p.W);   // ring column of the first step written; at most W follow it
   // 8-byte pieces e = (token j, dims 4 i ..): a thread's pieces are loaded in batches of WB before any of them
   // is stored (the ring and the new rows could alias as far as the compiler knows, so a load after a store
   // would wait for it)
   constexpr int WB = 8;
-  const int total = (int)len * (D / 4);
-  for (int e0 = threadIdx.x; e0 < total; e0 += 256 * WB) {
+  const int total = (int)(len - first) * (D / 4);
+  for (int e0 = blockIdx.y * (256 * WB) + threadIdx.x; e0 < total; e0 += gridDim.y * (256 * WB)) {
     uint2 kw[WB], vw[WB];
 #pragma unroll
     for (int u = 0; u < WB; ++u) {
@@ -780,7 +786,7 @@ extern "C" int hsg_window_attention(const void* q, int64_t q_sl, int64_t q_sh, i
   const int64_t last = (int64_t)first + count < max_len ? (int64_t)first + count : max_len;
   const int64_t qgroups = (last * groups + GR - 1) / GR - (int64_t)first * groups / GR;
   const int64_t blocks = ((int64_t)n_rows * hkv * qgroups + 7) / 8 * 8;
-  if (blocks > 0x7fffffff) return HSG_ERR_SHAPE;
+  if (blocks >= (1 << 24)) return HSG_ERR_SHAPE;   // a launch holds less than 2^32 threads
   RingParams p{};
   p.q = static_cast<const uint16_t*>(q); p.q_sl = q_sl; p.q_sh = q_sh; p.q_sg = q_sg;
   p.W = window;
@@ -792,7 +798,56 @@ extern "C" int hsg_window_attention(const void* q, int64_t q_sl, int64_t q_sh, i
   p.pairs = n_rows * hkv;
   p.qgroups = (int)qgroups;
   p.qg0 = (int)((int64_t)first * groups / GR);
+  p.sequences = 1;
   p.out = static_cast<uint16_t*>(out); p.o_sl = o_sl; p.o_sh = o_sh; p.o_sg = o_sg;
   hipLaunchKernelGGL(ring_attn_kernel, dim3((unsigned)blocks), dim3(NW * 64), 0, reinterpret_cast<hipStream_t>(stream), p);
+  return launch_status();
+}
+
+extern "C" int hsg_ring_prefill(const void* q, int64_t q_sl, int64_t q_sh, int64_t q_sg, void* ring_k, void* ring_v,
+                                int64_t ring_rows, int32_t window, const void* new_k, int64_t nk_sl, int64_t nk_sh,
+                                const void* new_v, int64_t nv_sl, int64_t nv_sh, const void* gate, int64_t g_sl,
+                                int64_t g_sh, int64_t g_sg, int64_t g_off, const int64_t* ring_pos,
+                                const int64_t* slots, const int64_t* starts, const int64_t* lens,
+                                const int64_t* offsets, int32_t n_rows, int32_t max_len, int32_t hkv, int32_t groups,
+                                int32_t head_dim, float scale, void* out, int64_t o_sl, int64_t o_sh, int64_t o_sg,
+                                void* stream) {
+  using namespace hsg;
+  if (n_rows < 0 || max_len <= 0 || hkv <= 0 || groups <= 0 || ring_rows <= 0) return HSG_ERR_ARG;
+  if (n_rows == 0) return HSG_OK;
+  if (!q || !ring_k || !ring_v || !new_k || !new_v || !ring_pos || !slots || !starts || !lens || !offsets || !out)
+    return HSG_ERR_ARG;
+  if (head_dim != D || window <= 0 || window > W_MAX || window % KB != 0) return HSG_ERR_SHAPE;
+  if ((int64_t)groups * max_len > (1 << 30)) return HSG_ERR_SHAPE;
+  const int64_t s16[] = {q_sl, q_sh, q_sg, nk_sl, nk_sh, nv_sl, nv_sh};
+  for (int64_t st : s16)
+    if (st % 8) return HSG_ERR_ALIGN;
+  const int64_t s4[] = {g_sl, g_sh, g_sg, g_off, o_sl, o_sh, o_sg};
+  for (int64_t st : s4)
+    if (st % 4) return HSG_ERR_ALIGN;
+  if (!aligned(q, 16) || !aligned(ring_k, 16) || !aligned(ring_v, 16) || !aligned(new_k, 16) ||
+      !aligned(new_v, 16) || !aligned(out, 8) || (gate && !aligned(gate, 8)))
+    return HSG_ERR_ALIGN;
+  const int64_t qgroups = ((int64_t)groups * max_len + NW * TQ - 1) / (NW * TQ);
+  const int64_t blocks = ((int64_t)n_rows * hkv * qgroups + 7) / 8 * 8;
+  if (blocks >= (1 << 24)) return HSG_ERR_SHAPE;   // a launch holds less than 2^32 threads
+  RingParams p{};
+  p.q = static_cast<const uint16_t*>(q); p.q_sl = q_sl; p.q_sh = q_sh; p.q_sg = q_sg;
+  p.ring_k = static_cast<uint16_t*>(ring_k); p.ring_v = static_cast<uint16_t*>(ring_v);
+  p.ring_rows = ring_rows; p.W = window;
+  p.new_k = static_cast<const uint16_t*>(new_k); p.nk_sl = nk_sl; p.nk_sh = nk_sh;
+  p.new_v = static_cast<const uint16_t*>(new_v); p.nv_sl = nv_sl; p.nv_sh = nv_sh;
+  p.gate = static_cast<const uint16_t*>(gate); p.g_sl = g_sl; p.g_sh = g_sh; p.g_sg = g_sg; p.g_off = g_off;
+  p.ring_pos = ring_pos; p.slots = slots; p.starts = starts; p.lens = lens; p.offsets = offsets;
+  p.lb = max_len; p.hkv = hkv; p.G = groups; p.scale = scale; p.write_ring = 1; p.min_len = 1;
+  p.pairs = n_rows * hkv;
+  p.qgroups = (int)qgroups;
+  p.sequences = 1;
+  p.out = static_cast<uint16_t*>(out); p.o_sl = o_sl; p.o_sh = o_sh; p.o_sg = o_sg;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  hipLaunchKernelGGL(ring_attn_kernel, dim3((unsigned)blocks), dim3(NW * 64), 0, st, p);
+  // 32 steps (one batch of the kernel) a workgroup: with one workgroup a pair, 12 pairs of 512 steps took 31 us
+  const unsigned batches = (unsigned)((max_len < window ? max_len : window) + 31) / 32;
+  hipLaunchKernelGGL(ring_write_kernel, dim3((unsigned)p.pairs, batches), dim3(256), 0, st, p);
   return launch_status();
 }

@@ -86,6 +86,14 @@ SIGNATURES = {
         _P, _P, _I32, _I32, _I32, _I32,      # lens, offsets, n_rows, max_len, first, count
         _I32, _I32, _I32, _I32, _F,          # window, hkv, groups, head_dim, scale
         _P, _I64, _I64, _I64, _P]),          # out, o_sl, o_sh, o_sg, stream
+    "hsg_ring_prefill": (ctypes.c_int, [
+        _P, _I64, _I64, _I64,                # q, q_sl, q_sh, q_sg
+        _P, _P, _I64, _I32,                  # ring_k, ring_v, ring_rows, window
+        _P, _I64, _I64, _P, _I64, _I64,      # new_k, nk_sl, nk_sh, new_v, nv_sl, nv_sh
+        _P, _I64, _I64, _I64, _I64,          # gate, g_sl, g_sh, g_sg, g_off
+        _P, _P, _P, _P, _P,                  # ring_pos, slots, starts, lens, offsets
+        _I32, _I32, _I32, _I32, _I32, _F,    # n_rows, max_len, hkv, groups, head_dim, scale
+        _P, _I64, _I64, _I64, _P]),          # out, o_sl, o_sh, o_sg, stream
     "hsg_ring_decode_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32, _I32]),
     "hsg_ring_decode": (ctypes.c_int, [
         _P, _I64, _I64, _I64, _I64,          # q, q_sn, q_sl, q_sh, q_sg

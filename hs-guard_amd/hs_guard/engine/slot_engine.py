@@ -3,7 +3,8 @@
 Host orchestration mirrors SlotStreamEngineV7/V8 (src/hs_guard/engine/slot_engine_v7.py:117-167,
 slot_engine_v8.py:30-89): a request list is cut into ticks of at most ``max_tick_tokens`` tokens per slot
 and at most the largest session bucket of rows; each tick is one H2D copy of a packed int64 buffer, one
-graph replay, one D2H copy of the per-token class probabilities of both roles and one stream sync.
+graph replay, one D2H copy of the per-token class probabilities of both roles and one stream sync. Up to 32
+sessions' contexts (more than a tick of tokens a row) run in long pieces instead, without a graph (_long_piece).
 
 Differences by design (the device program is the MI355X one, not a translation):
 * Tokens are PACKED: row n owns tokens offsets[n] .. offsets[n] + lens[n] - 1 of the tick, so GEMMs and
@@ -25,7 +26,7 @@ import numpy as np
 import torch
 
 from .. import _hostpack
-from .._lib import HSG_ERR_SHAPE, HSG_GDN_BURST_MIN_DEFAULT, HSG_GEMM_SKINNY_M_MAX, check, lib
+from .._lib import HSG_ERR_SHAPE, HSG_GDN_BURST_MIN_DEFAULT, HSG_GEMM_SKINNY_M_MAX, calls, check, lib
 from ..model import ROLES, GuardModel
 from .gemm_plan import WORKSPACE_BYTES as GEMM_WORKSPACE_BYTES
 from .gemm_plan import GemmPlans
@@ -33,6 +34,8 @@ from .gemm_plan import GemmPlans
 SESSION_BUCKETS = (1, 2, 4, 8, 16, 32, 48, 64, 96, 128, 160, 192, 224, 256, 320, 352, 384, 448, 512)
 STATE_DTYPES = {"float32": torch.float32, "float16": torch.float16}
 _STATE_CODE = {torch.float32: 0, torch.float16: 1}
+# Tokens of a long piece (SlotStreamEngine._run_long): enough for the products to run at their large-M rate
+LONG_TOKENS = 4096
 
 
 def bucket(value, choices):
@@ -251,39 +254,44 @@ class SlotStreamEngine(PreparedWeights):
         self._allocate_buffers()
 
     # ------------------------------------------------------------------------------------------------
+    def _activations(self, T, rows):
+        """Buffers of a program over T tokens of up to ``rows`` rows (inputs, activations, probabilities)."""
+        cfg, dev = self.cfg, self.device
+        bf16 = torch.bfloat16
+        hq, hkv, D = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
+        widest = max(self.gdn_in, self.att_in, 2 * cfg.intermediate_size)
+        buf = {name: torch.empty(T * width, dtype=bf16, device=dev) for name, width in (
+            ("hidden", cfg.hidden_size), ("normed", cfg.hidden_size), ("mix", cfg.hidden_size), ("proj", widest),
+            ("conv", cfg.conv_dim), ("mid", max(cfg.value_dim, hq * D, cfg.intermediate_size)), ("q", hq * D),
+            ("k", hkv * D), ("head", cfg.head_hidden * len(self.roles)))}
+        buf["probs"] = torch.empty(len(self.roles) * T * 3, dtype=torch.float32, device=dev)
+        buf["inputs"] = torch.empty(2 * T + 4 * rows, dtype=torch.long, device=dev)
+        if self.chunk_min_tokens:
+            buf["gdn_o"] = torch.empty(T * cfg.value_dim, dtype=bf16, device=dev)
+        return buf
+
     def _allocate_buffers(self):
         cfg, T, dev = self.cfg, self.max_tokens, self.device
-        bf16 = torch.bfloat16
         hq, hkv, D = cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim
         self.gdn_in = gdn_proj_width(cfg)       # row stride of the GDN projection (padded, see gdn_proj_width)
         self.att_in = hq * 2 * D + 2 * hkv * D
-        widest = max(self.gdn_in, self.att_in, 2 * cfg.intermediate_size)
-        self.buf = {
-            "hidden": torch.zeros(T * cfg.hidden_size, dtype=bf16, device=dev),
-            # the residual stream's second buffer for ticks whose add + RMSNorm runs inside the next product
-            "hidden2": torch.zeros(max(self.gemm_skinny_rows, 1) * cfg.hidden_size, dtype=bf16, device=dev),
-            "normed": torch.zeros(T * cfg.hidden_size, dtype=bf16, device=dev),
-            "mix": torch.zeros(T * cfg.hidden_size, dtype=bf16, device=dev),
-            "proj": torch.zeros(T * widest, dtype=bf16, device=dev),
-            "conv": torch.zeros(T * cfg.conv_dim, dtype=bf16, device=dev),
-            "mid": torch.zeros(T * max(cfg.value_dim, hq * D, cfg.intermediate_size), dtype=bf16, device=dev),
-            "q": torch.zeros(T * hq * D, dtype=bf16, device=dev),
-            "k": torch.zeros(T * hkv * D, dtype=bf16, device=dev),
-            "head": torch.zeros(T * cfg.head_hidden * len(self.roles), dtype=bf16, device=dev),
-            "probs": torch.zeros(len(self.roles) * T * 3, dtype=torch.float32, device=dev),
-            "inputs": torch.zeros(2 * T + 4 * self.max_rows, dtype=torch.long, device=dev),
-        }
+        self.buf = {name: t.zero_() for name, t in self._activations(T, self.max_rows).items()}
+        # the residual stream's second buffer for ticks whose add + RMSNorm runs inside the next product
+        self.buf["hidden2"] = torch.zeros(max(self.gemm_skinny_rows, 1) * cfg.hidden_size, dtype=torch.bfloat16,
+                                          device=dev)
         # hipBLASLt workspace of the projection GEMMs and their committed solution table (hs_guard/engine/gemm_plan.py)
         self.gemm_plans = GemmPlans.load()
         self.gemm_ws = torch.empty(GEMM_WORKSPACE_BYTES, dtype=torch.uint8, device=dev)
         # decode workspace for the single-step rows of a tick (used by hsg_ring_decode above 8 query heads per kv head)
         ws = lib().hsg_ring_decode_workspace_bytes(self.max_rows, hkv, hq // hkv, self.window)
         self.ring_ws = torch.empty(max(int(ws), 16), dtype=torch.uint8, device=dev)
-        # chunked-GDN scratch for the long rows of a tick (one 64-token chunk per row) and their raw outputs
+        # chunked-GDN scratch for the long rows of a tick (one 64-token chunk per row)
         if self.chunk_min_tokens:
-            ws = lib().hsg_gdn_chunk_workspace_bytes(self.max_rows, self.max_tick_tokens, cfg.linear_num_value_heads)
-            self.chunk_ws = torch.empty(max(int(ws), 256), dtype=torch.uint8, device=dev)
-            self.buf["gdn_o"] = torch.zeros(T * cfg.value_dim, dtype=bf16, device=dev)
+            self.chunk_ws = self._chunk_workspace(self.max_rows, self.max_tick_tokens)
+
+    def _chunk_workspace(self, rows, max_len):
+        ws = lib().hsg_gdn_chunk_workspace_bytes(rows, max_len, self.cfg.linear_num_value_heads)
+        return torch.empty(max(int(ws), 256), dtype=torch.uint8, device=self.device)
 
     def mm(self, x, w, out):
         """out[M, N] = x[M, K] . w[N, K]^T (bf16, row-major, unit column stride) on the current stream: through
@@ -297,19 +305,20 @@ class SlotStreamEngine(PreparedWeights):
             raise ValueError("mm: shapes or strides do not match D[M, N] = A[M, K] . W[N, K]^T")
         stream = torch.cuda.current_stream(self.device).cuda_stream
         if self._skinny(x, w, K):
-            check(lib().hsg_gemm_bf16_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
-                                             out.stride(0), M, N, K, stream), "hsg_gemm_bf16_skinny")
+            check(calls().hsg_gemm_bf16_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
+                                               out.stride(0), M, N, K, stream), "hsg_gemm_bf16_skinny")
             return out
         index = self.gemm_plans.index(M, N, K)
-        rc = lib().hsg_gemm_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
-                                 M, N, K, index, self.gemm_ws.data_ptr(), self.gemm_ws.numel(), stream)
+        rc = calls().hsg_gemm_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
+                                   M, N, K, index, self.gemm_ws.data_ptr(), self.gemm_ws.numel(), stream)
         if rc == HSG_ERR_SHAPE and index >= 0:
             # the running hipBLASLt rejected the table's solution before launching anything: use the heuristic's
             # first candidate for this shape from now on
             warnings.warn(f"hipBLASLt rejected solution {index} for ({M}, {N}, {K}); using its heuristic instead")
             self.gemm_plans.drop(M, N, K)
-            rc = lib().hsg_gemm_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
-                                     out.stride(0), M, N, K, -1, self.gemm_ws.data_ptr(), self.gemm_ws.numel(), stream)
+            rc = calls().hsg_gemm_bf16(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
+                                       out.stride(0), M, N, K, -1, self.gemm_ws.data_ptr(), self.gemm_ws.numel(),
+                                       stream)
         check(rc, "hsg_gemm_bf16")
         return out
 
@@ -328,18 +337,22 @@ class SlotStreamEngine(PreparedWeights):
             raise ValueError("mm_silu: shapes or strides do not match")
         stream = torch.cuda.current_stream(self.device).cuda_stream
         if self._skinny(gu, w, I) and w.stride(1) == 1:
-            check(lib().hsg_gemm_bf16_skinny_silu(gu.data_ptr(), gu.stride(0), w.data_ptr(), w.stride(0),
-                                                  out.data_ptr(), out.stride(0), M, w.shape[0], I, stream),
+            check(calls().hsg_gemm_bf16_skinny_silu(gu.data_ptr(), gu.stride(0), w.data_ptr(), w.stride(0),
+                                                    out.data_ptr(), out.stride(0), M, w.shape[0], I, stream),
                   "hsg_gemm_bf16_skinny_silu")
             return out
-        check(lib().hsg_silu_mul(gu.data_ptr(), gu.stride(0), I, act.data_ptr(), M, stream), "hsg_silu_mul")
+        check(calls().hsg_silu_mul(gu.data_ptr(), gu.stride(0), I, act.data_ptr(), M, stream), "hsg_silu_mul")
         return self.mm(act, w, out)
 
     def _view(self, name, *shape):
+        return self._view_of(self.buf, name, *shape)
+
+    @staticmethod
+    def _view_of(buf, name, *shape):
         n = 1
         for s in shape:
             n *= s
-        return self.buf[name][:n].view(*shape)
+        return buf[name][:n].view(*shape)
 
     # ------------------------------------------------------------------------------------------------
     def state_bytes_per_session(self):
@@ -379,16 +392,24 @@ class SlotStreamEngine(PreparedWeights):
         self.length[slot] = snap["length"]
 
     # ------------------------------------------------------------------------------------------------
-    def _inputs(self, nb, tb):
-        x = self.buf["inputs"]
+    def _inputs(self, nb, tb, buf=None):
+        x = (buf or self.buf)["inputs"]
         return {"ids": x[:tb], "pos": x[tb:2 * tb], "offsets": x[2 * tb:2 * tb + nb],
                 "lens": x[2 * tb + nb:2 * tb + 2 * nb], "slots": x[2 * tb + 2 * nb:2 * tb + 3 * nb],
                 "starts": x[2 * tb + 3 * nb:2 * tb + 4 * nb], "all": x[:2 * tb + 4 * nb]}
 
-    def _forward(self, nb, tb, inp):
+    def _forward(self, nb, tb, inp, scratch=None, max_len=0):
         """The tick's device program (src/hs_guard/engine/slot_engine_v8.py:30-58), launched on the current
-        stream. Reads only device memory, so it can be captured into a hipGraph."""
-        L = lib()
+        stream. Reads only device memory, so it can be captured into a hipGraph. max_len > 0: a long piece's program
+        (_run_long) over its own ``scratch``, every row of up to max_len tokens on the chunk kernels and
+        hsg_ring_prefill."""
+        L = calls()
+        long = max_len > 0
+        buf, chunk_ws = scratch or (self.buf, getattr(self, "chunk_ws", None))
+
+        def view(name, *shape):
+            return self._view_of(buf, name, *shape)
+
         cfg = self.cfg
         st = torch.cuda.current_stream(self.device).cuda_stream
         H, W = cfg.hidden_size, self.window
@@ -400,9 +421,9 @@ class SlotStreamEngine(PreparedWeights):
             cfg.linear_value_head_dim
         ids, pos, offsets, lens, slots, starts = (inp[k] for k in ("ids", "pos", "offsets", "lens", "slots",
                                                                     "starts"))
-        hid = [self._view("hidden", tb, H)]
-        normed = self._view("normed", tb, H)
-        mix = self._view("mix", tb, H)
+        hid = [view("hidden", tb, H)]
+        normed = view("normed", tb, H)
+        mix = view("mix", tb, H)
         check(L.hsg_embed_rmsnorm(ids.data_ptr(), self.emb.data_ptr(), cfg.vocab_size,
                                   self.layers[0]["in_w1"].data_ptr(), eps, hid[0].data_ptr(), normed.data_ptr(), tb,
                                   H, st), "hsg_embed_rmsnorm")
@@ -410,9 +431,9 @@ class SlotStreamEngine(PreparedWeights):
         # reads normed. In ticks of at most gemm_skinny_rows tokens both run in one hsg_gemm_bf16_skinny_addnorm
         # launch, which writes the residual to the other of two buffers (hid[0] -> hid[1] -> hid[0] ...); otherwise
         # hsg_add_rmsnorm updates hid[0] in place and the product follows.
-        fuse = tb <= self.gemm_skinny_rows and H == 1024
+        fuse = tb <= self.gemm_skinny_rows and H == 1024 and not long
         if fuse:
-            hid.append(self._view("hidden2", tb, H))
+            hid.append(view("hidden2", tb, H))
         pending = []    # the (mix, w1) of an add + RMSNorm not yet applied
 
         def norm_mm(w, out):
@@ -433,13 +454,13 @@ class SlotStreamEngine(PreparedWeights):
         for i, ((kind, idx), Lw) in enumerate(zip(self.kind, self.layers)):
             if kind == "linear_attention":
                 C = cfg.conv_dim
-                proj = self._view("proj", tb, self.gdn_in)
+                proj = view("proj", tb, self.gdn_in)
                 norm_mm(Lw["w_in"], proj)
-                out = self._view("mid", tb, cfg.value_dim)
+                out = view("mid", tb, cfg.value_dim)
                 base = proj.data_ptr()
                 # rows are packed longest first: in a prefill-like tick the rows of >= chunk_min_tokens tokens go
                 # to the chunked kernels (one WY/UT chunk each), the rest to the slot step
-                R = self._chunk_rows(nb, tb)
+                R = nb if long else self._chunk_rows(nb, tb)
                 if self.fuse_conv and R == 0:
                     # causal conv + SiLU inside the slot step, from the raw projection and the conv history pool
                     check(L.hsg_gdn_conv_slot_step_gated(
@@ -451,38 +472,40 @@ class SlotStreamEngine(PreparedWeights):
                         Lw["norm_w"].data_ptr(), eps, out.data_ptr(), self.gdn_burst_min, st),
                           "hsg_gdn_conv_slot_step_gated")
                 else:
-                    conv = self._view("conv", tb, C)
+                    conv = view("conv", tb, C)
                     check(L.hsg_conv_silu_update(proj.data_ptr(), self.gdn_in, self.conv[idx].data_ptr(), S,
                                                  Lw["conv_w"].data_ptr(), cfg.linear_conv_kernel_dim,
                                                  slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb,
-                                                 self.max_tick_tokens if R else 0, C, conv.data_ptr(), C, st),
+                                                 max_len or (self.max_tick_tokens if R else 0), C,
+                                                 conv.data_ptr(), C, st),
                           "hsg_conv_silu_update")
-                    check(L.hsg_gdn_slot_step_gated(
-                        conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
-                        base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), self.gdn_in,
-                        Lw["A_log"].data_ptr(), Lw["dt_bias"].data_ptr(), self.rec[idx].data_ptr(),
-                        _STATE_CODE[self.state_dtype], S, slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb,
-                        0, nh, hv, kd, vd, kd ** -0.5, base + 2 * C, self.gdn_in, Lw["norm_w"].data_ptr(), eps,
-                        out.data_ptr(), R, max(self.chunk_min_tokens, 1), self.gdn_burst_min, st),
-                          "hsg_gdn_slot_step_gated")
+                    if not long:
+                        check(L.hsg_gdn_slot_step_gated(
+                            conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
+                            base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), self.gdn_in,
+                            Lw["A_log"].data_ptr(), Lw["dt_bias"].data_ptr(), self.rec[idx].data_ptr(),
+                            _STATE_CODE[self.state_dtype], S, slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb,
+                            0, nh, hv, kd, vd, kd ** -0.5, base + 2 * C, self.gdn_in, Lw["norm_w"].data_ptr(), eps,
+                            out.data_ptr(), R, max(self.chunk_min_tokens, 1), self.gdn_burst_min, st),
+                              "hsg_gdn_slot_step_gated")
                     if R:
                         check(L.hsg_gdn_chunk_prefill_gated(
                             conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
                             base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), self.gdn_in,
                             Lw["A_log"].data_ptr(), Lw["dt_bias"].data_ptr(), self.rec[idx].data_ptr(),
                             _STATE_CODE[self.state_dtype], S, slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(),
-                            R, self.max_tick_tokens, nh, hv, kd, vd, kd ** -0.5,
-                            self._view("gdn_o", tb, cfg.value_dim).data_ptr(), base + 2 * C, self.gdn_in,
-                            Lw["norm_w"].data_ptr(), eps, out.data_ptr(), self.chunk_min_tokens,
-                            self.chunk_ws.data_ptr(), self.chunk_ws.numel(), st), "hsg_gdn_chunk_prefill_gated")
+                            R, max_len or self.max_tick_tokens, nh, hv, kd, vd, kd ** -0.5,
+                            view("gdn_o", tb, cfg.value_dim).data_ptr(), base + 2 * C, self.gdn_in,
+                            Lw["norm_w"].data_ptr(), eps, out.data_ptr(), 0 if long else self.chunk_min_tokens,
+                            chunk_ws.data_ptr(), chunk_ws.numel(), st), "hsg_gdn_chunk_prefill_gated")
                 self.mm(out, Lw["w_out"], mix)
             else:
-                proj = self._view("proj", tb, self.att_in)
+                proj = view("proj", tb, self.att_in)
                 norm_mm(Lw["w_in"], proj)
-                q = self._view("q", tb, hq * D)
-                k = self._view("k", tb, hkv * D)
+                q = view("q", tb, hq * D)
+                k = view("k", tb, hkv * D)
                 base = proj.data_ptr()
-                att = self._view("mid", tb, hq * D)
+                att = view("mid", tb, hq * D)
                 if tb == 1 and cfg.rotary_dim == 64 and D == 256:
                     # a one-token tick: the q / k norm and RoPE run inside the decode's scores kernel (one launch
                     # fewer), bitwise hsg_norm_rope + hsg_ring_decode; k receives the new keys
@@ -502,42 +525,50 @@ class SlotStreamEngine(PreparedWeights):
                                           hq * D, D, base + 2 * hq * 2 * D, self.att_in, D, hkv,
                                           Lw["k_w1"].data_ptr(), eps, k.data_ptr(), hkv * D, D, pos.data_ptr(),
                                           self.inv_freq.data_ptr(), cfg.rotary_dim, tb, D, st), "hsg_norm_rope")
-                    # single-step rows: hsg_ring_decode; rows of two or more steps: the tiled kernel (min_len 2)
-                    check(L.hsg_ring_decode(
-                        q.data_ptr(), 0, hq * D, G * D, D,
-                        self.ring_k[idx].data_ptr(), self.ring_v[idx].data_ptr(), S, W,
-                        k.data_ptr(), 0, hkv * D, D,
-                        base + 2 * (hq * 2 * D + hkv * D), 0, self.att_in, D,
-                        base, 0, self.att_in, G * 2 * D, 2 * D, D,
-                        self.ring_pos.data_ptr(), slots.data_ptr(), starts.data_ptr(), lens.data_ptr(),
-                        offsets.data_ptr(), nb, hkv, G, D, D ** -0.5, 1,
-                        att.data_ptr(), 0, hq * D, G * D, D, self.ring_ws.data_ptr(), self.ring_ws.numel(), st),
-                        "hsg_ring_decode")
-                    if tb >= 2:
-                        # a one-token bucket has no row of two or more steps: its program leaves the tiled kernel
-                        # out
-                        check(L.hsg_ring_attention(
+                    if long:
+                        check(L.hsg_ring_prefill(
+                            q.data_ptr(), hq * D, G * D, D, self.ring_k[idx].data_ptr(), self.ring_v[idx].data_ptr(), S,
+                            W, k.data_ptr(), hkv * D, D, base + 2 * (hq * 2 * D + hkv * D), self.att_in, D,
+                            base, self.att_in, G * 2 * D, 2 * D, D, self.ring_pos.data_ptr(), slots.data_ptr(),
+                            starts.data_ptr(), lens.data_ptr(), offsets.data_ptr(), nb, max_len, hkv, G, D, D ** -0.5,
+                            att.data_ptr(), hq * D, G * D, D, st), "hsg_ring_prefill")
+                    else:
+                        # single-step rows: hsg_ring_decode; rows of two or more steps: the tiled kernel (min_len 2)
+                        check(L.hsg_ring_decode(
                             q.data_ptr(), 0, hq * D, G * D, D,
                             self.ring_k[idx].data_ptr(), self.ring_v[idx].data_ptr(), S, W,
                             k.data_ptr(), 0, hkv * D, D,
                             base + 2 * (hq * 2 * D + hkv * D), 0, self.att_in, D,
                             base, 0, self.att_in, G * 2 * D, 2 * D, D,
                             self.ring_pos.data_ptr(), slots.data_ptr(), starts.data_ptr(), lens.data_ptr(),
-                            offsets.data_ptr(), nb, self.max_tick_tokens, hkv, G, D, D ** -0.5, 1, 2,
-                            att.data_ptr(), 0, hq * D, G * D, D, st), "hsg_ring_attention")
+                            offsets.data_ptr(), nb, hkv, G, D, D ** -0.5, 1,
+                            att.data_ptr(), 0, hq * D, G * D, D, self.ring_ws.data_ptr(), self.ring_ws.numel(), st),
+                            "hsg_ring_decode")
+                        if tb >= 2:
+                            # a one-token bucket has no row of two or more steps: its program leaves the tiled kernel
+                            # out
+                            check(L.hsg_ring_attention(
+                                q.data_ptr(), 0, hq * D, G * D, D,
+                                self.ring_k[idx].data_ptr(), self.ring_v[idx].data_ptr(), S, W,
+                                k.data_ptr(), 0, hkv * D, D,
+                                base + 2 * (hq * 2 * D + hkv * D), 0, self.att_in, D,
+                                base, 0, self.att_in, G * 2 * D, 2 * D, D,
+                                self.ring_pos.data_ptr(), slots.data_ptr(), starts.data_ptr(), lens.data_ptr(),
+                                offsets.data_ptr(), nb, self.max_tick_tokens, hkv, G, D, D ** -0.5, 1, 2,
+                                att.data_ptr(), 0, hq * D, G * D, D, st), "hsg_ring_attention")
                 self.mm(att, Lw["w_out"], mix)
             pending.append((mix, Lw["post_w1"]))
             I = cfg.intermediate_size
-            gu = self._view("proj", tb, 2 * I)
+            gu = view("proj", tb, 2 * I)
             norm_mm(Lw["w_gu"], gu)
-            self.mm_silu(gu, Lw["w_down"], mix, self._view("mid", tb, I))
+            self.mm_silu(gu, Lw["w_down"], mix, view("mid", tb, I))
             nxt = self.layers[i + 1]["in_w1"] if i + 1 < len(self.layers) else self.final_w1
             pending.append((mix, nxt))
         # the final norm feeds the heads' first Linear (with bias): one skinny launch in small ticks, else the norm
         # and torch.addmm
         mx, w1 = pending.pop()
         R, E = len(self.roles), cfg.head_hidden
-        y = self._view("head", tb, R * E)
+        y = view("head", tb, R * E)
         if fuse and self._skinny(normed, self.head_w1, H):
             check(L.hsg_gemm_bf16_skinny_addnorm(hid[0].data_ptr(), H, mx.data_ptr(), H, w1.data_ptr(), eps,
                                                  hid[1].data_ptr(), H, self.head_w1.data_ptr(), self.head_w1.stride(0),
@@ -547,12 +578,12 @@ class SlotStreamEngine(PreparedWeights):
             check(L.hsg_add_rmsnorm(hid[0].data_ptr(), mx.data_ptr(), w1.data_ptr(), eps, normed.data_ptr(), tb, H,
                                     st), "hsg_add_rmsnorm")
             torch.addmm(self.head_b1, normed, self.head_w1.t(), out=y)
-        probs = self._view("probs", R, tb, 3)
+        probs = view("probs", R, tb, 3)
         check(L.hsg_risk_head(y.data_ptr(), R * E, self.head_ln_w.data_ptr(), self.head_ln_b.data_ptr(),
                               self.head_w2.data_ptr(), self.head_b2.data_ptr(), cfg.layer_norm_eps, R, E,
                               probs.data_ptr(), tb, st), "hsg_risk_head")
         check(L.hsg_ring_pos_update(self.ring_pos.data_ptr(), S, W, slots.data_ptr(), starts.data_ptr(),
-                                    lens.data_ptr(), nb, self.max_tick_tokens, st), "hsg_ring_pos_update")
+                                    lens.data_ptr(), nb, max_len or self.max_tick_tokens, st), "hsg_ring_pos_update")
         return probs
 
     def _chunk_rows(self, nb, tb):
@@ -621,6 +652,47 @@ class SlotStreamEngine(PreparedWeights):
         self._replay(nb, tb, graph, inp, probs, host_in, host_out)
         self.length[slots] += lens
         return out_np[:, :total].copy(), lens, offsets
+
+    def _long_piece(self, rows, longest):
+        """Tokens a row of ``rows`` pending ones may bring to one long piece (0: ticks). A few sessions with contexts
+        make small ticks (3 rows: 192 tokens) that are bound by their launches and by reading the weights once a tick;
+        a piece of LONG_TOKENS tokens in all does both once: 3 rows of 900 tokens through 4 layers 7.15 -> 1.70 ms, and
+        at 24 layers one row of 65 tokens 2.88 -> 2.58 ms, 32 rows of 256 23.4 -> 18.7 ms, one of 65 beside 31 of 1 token
+        3.67 -> 3.16 ms. From 33 rows on a piece would hold no more than two ticks a row, and ticks keep their graphs
+        (32 rows of 128 gained 20 %). Engines set up with smaller ticks or without the chunk kernels keep ticks."""
+        if not self.chunk_min_tokens or self.max_tick_tokens < 64 or longest <= 64:
+            return 0
+        piece = LONG_TOKENS // rows // 64 * 64
+        return piece if piece >= 128 else 0
+
+    def _long_scratch(self, rows, piece):
+        """(activations, chunk workspace) of a long piece, or None where the card has no room for them (the step then
+        runs in ticks). Taken from the caching allocator for the length of the piece: an engine that only streams
+        keeps none."""
+        try:
+            return self._activations(LONG_TOKENS, rows), self._chunk_workspace(rows, piece)
+        except torch.OutOfMemoryError:
+            return None
+
+    def _run_long(self, chunks, slots, scratch):
+        """One long piece: rows of any length (LONG_TOKENS in all), outside the graphs. Returns as _run_arrays."""
+        n = len(chunks)
+        row_lens = np.fromiter(map(len, chunks), dtype=np.int64, count=n)
+        total = int(row_lens.sum())
+        tb = bucket(total, token_buckets(LONG_TOKENS))
+        order = np.argsort(-row_lens, kind="stable")
+        host = torch.empty(2 * tb + 4 * n, dtype=torch.long)
+        lens_p, offsets_p = pack_ticks([chunks[r] for r in order], np.asarray(slots)[order], self.length, n, tb,
+                                       self.max_slots, host.numpy())
+        lens, offsets = np.empty(n, dtype=np.int64), np.empty(n, dtype=np.int64)
+        lens[order] = lens_p
+        offsets[order] = offsets_p
+        inp = self._inputs(n, tb, scratch[0])
+        inp["all"].copy_(host)
+        probs = self._forward(n, tb, inp, scratch, int(row_lens.max())).cpu()
+        self.stats["eager_steps"] += 1
+        self.length[slots] += lens
+        return probs.numpy()[:, :total], lens, offsets
 
     def _validate(self, requests):
         slots = [s for s, _ in requests]
@@ -731,18 +803,25 @@ class SlotStreamEngine(PreparedWeights):
         results = {role: [[] for _ in requests] for role in self.roles}
         pending = [(i, s, list(ids)) for i, (s, ids) in enumerate(requests)]
         while pending:
-            batch = [(i, s, ids[:largest]) for i, s, ids in pending]
+            n = min(len(pending), rows)
+            piece = self._long_piece(n, max(len(ids) for _, _, ids in pending))
+            scratch = self._long_scratch(n, piece) if piece else None
+            take = piece if scratch else largest
+            batch = [(i, s, ids[:take]) for i, s, ids in pending]
             for start in range(0, len(batch), rows):
                 part = batch[start:start + rows]
+                chunks = [c for _, _, c in part]
                 slots = np.fromiter((s for _, s, _ in part), dtype=np.int64, count=len(part))
-                flat, lens, offsets = self._run_arrays([c for _, _, c in part], slots)
+                flat, lens, offsets = (self._run_long(chunks, slots, scratch) if scratch else
+                                       self._run_arrays(chunks, slots))
                 # one gather into request order, then one split per role (per-row slicing in Python cost ~700
                 # tensor constructions per 352-row tick)
                 probs = torch.from_numpy(request_order(flat, lens, offsets))
                 sizes = lens.tolist()
                 for role_index, role in enumerate(self.roles):
-                    for (i, _, _), piece in zip(part, torch.split(probs[role_index], sizes)):
-                        results[role][i].append(piece)
-            pending = [(i, s, ids[largest:]) for i, s, ids in pending if len(ids) > largest]
+                    for (i, _, _), part_probs in zip(part, torch.split(probs[role_index], sizes)):
+                        results[role][i].append(part_probs)
+            scratch = None
+            pending = [(i, s, ids[take:]) for i, s, ids in pending if len(ids) > take]
         return {role: [chunks[0] if len(chunks) == 1 else torch.cat(chunks) for chunks in rows_]
                 for role, rows_ in results.items()}

@@ -195,6 +195,20 @@ int hsg_window_attention(const void* q, int64_t q_sl, int64_t q_sh, int64_t q_sg
                          int64_t o_sg, void* stream);
 
 /*
+ * hsg_ring_attention with the ring write for rows of any length (an initial context's, in few long pieces): packed rows
+ * (offsets required) of at most max_len tokens, rows with lens[n] == 0 or > max_len left alone. Every ring position must
+ * lie before the row's start, as streaming leaves it. Of a row longer than the window the last `window` steps stay in
+ * the ring. Two launches. Supported as hsg_ring_attention, with groups x max_len <= 2^30 and under 2^24 workgroups.
+ */
+int hsg_ring_prefill(const void* q, int64_t q_sl, int64_t q_sh, int64_t q_sg, void* ring_k, void* ring_v,
+                     int64_t ring_rows, int32_t window, const void* new_k, int64_t nk_sl, int64_t nk_sh,
+                     const void* new_v, int64_t nv_sl, int64_t nv_sh, const void* gate, int64_t g_sl, int64_t g_sh,
+                     int64_t g_sg, int64_t g_off, const int64_t* ring_pos, const int64_t* slots,
+                     const int64_t* starts, const int64_t* lens, const int64_t* offsets, int32_t n_rows,
+                     int32_t max_len, int32_t hkv, int32_t groups, int32_t head_dim, float scale, void* out,
+                     int64_t o_sl, int64_t o_sh, int64_t o_sg, void* stream);
+
+/*
  * Ring attention for decode steps: the same contract and numerics as hsg_ring_attention for rows with
  * lens[n] == 1 (one query position; lb is 1 and the padded layout is [n_rows, 1, ...]). Replaces
  * ring_attention_v8 at its decode shape (src/hs_guard/engine/fused_kernels.py:358-376 with Lb == 1,
@@ -422,7 +436,7 @@ int hsg_risk_head_f32(const float* y, int64_t y_stride, const float* ln_w, const
 /*
  * Ring position bookkeeping after all layers. Replaces ring_pos[slots, ring_col] = where(valid, pos, -1)
  * (src/hs_guard/engine/slot_engine_v8.py:41,57): ring_pos[slot, (start + j) % window] = start + j for
- * j < min(lens[n], lb_max); column `window` is never written (it stays -1).
+ * j < min(lens[n], lb_max), of which the last `window`; column `window` is never written (it stays -1).
  */
 int hsg_ring_pos_update(int64_t* ring_pos, int64_t ring_rows, int32_t window, const int64_t* slots,
                         const int64_t* starts, const int64_t* lens, int32_t n_rows, int32_t lb_max,

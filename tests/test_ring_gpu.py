@@ -475,3 +475,59 @@ def test_window_attention_of_sequences(lens, W, G):
         outs.append(out)
     _check(_np(outs[0]), ref.numpy())
     assert torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("W,G,lens,starts", [
+    (512, 4, [900, 65, 0, 513, 17, 1], [0, 700, 3, 200, 5 * 512 - 9, 511]),
+    (96, 8, [64, 95, 97, 300, 2], [96, 50, 1000, 0, 7]),
+    (32, 1, [129, 33], [31, 64])])
+def test_ring_prefill_of_long_rows(W, G, lens, starts):
+    """hsg_ring_prefill: packed rows around and beyond the window over empty, partial and full rings, against the masked
+    softmax in float64 over the history; afterwards the ring holds exactly the last W positions of every row, and
+    hsg_ring_pos_update numbers them."""
+    from hs_guard._lib import lib
+    print(f"[ring] prefill {lens} W={W} G={G}", flush=True)
+    gen = torch.Generator().manual_seed(60 + G)
+    Hkv, D, T, N, S = 2, 256, sum(lens), len(lens), len(lens) + 2
+    dev = torch.device("cuda:0")
+    q = torch.randn(T, Hkv, G, D, generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(T, Hkv, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    gate = torch.randn(T, Hkv, G, D, generator=gen).to(torch.bfloat16)
+    ring = [torch.randn(S, Hkv, W + 1, D, generator=gen).to(torch.bfloat16) for _ in range(2)]
+    pos = torch.full((S, W + 1), -1, dtype=torch.long)
+    slots = torch.randperm(S, generator=gen)[:N]
+    offs = [sum(lens[:i]) for i in range(N)]
+    ref = torch.zeros(T, Hkv, G, D, dtype=torch.float64)
+    want, want_pos = [r.clone() for r in ring], pos.clone()
+    for s, st, n, o in zip(slots.tolist(), starts, lens, offs):
+        h = torch.arange(max(0, st - W), st)
+        pos[s, h % W] = want_pos[s, h % W] = h
+        allpos = torch.cat([h, st + torch.arange(n)])
+        ka, va = (torch.cat([r[s][:, h % W].transpose(0, 1), x[o:o + n]]).double() for r, x in zip(ring, (k, v)))
+        i = st + torch.arange(n)
+        ok = (allpos[None] <= i[:, None]) & (allpos[None] > i[:, None] - W)
+        sc = torch.einsum("ihgd,jhd->hgij", q[o:o + n].double(), ka) * D ** -0.5
+        ref[o:o + n] = torch.einsum("hgij,jhd->ihgd", torch.softmax(sc.masked_fill(~ok, -torch.inf), -1), va)
+        last = torch.arange(max(0, n - W), n)
+        want_pos[s, (st + last) % W] = st + last
+        for r, x in zip(want, (k, v)):
+            r[s][:, (st + last) % W] = x[o + last].transpose(0, 1)
+    ref = ref * torch.sigmoid(gate.double())
+    d = [x.to(dev) for x in (q, k, v, gate, *ring, pos, slots, torch.tensor(starts), torch.tensor(lens),
+                             torch.tensor(offs))]
+    out = torch.zeros(T, Hkv, G, D, dtype=torch.bfloat16, device=dev)
+
+    def call(max_len):
+        return lib().hsg_ring_prefill(
+            d[0].data_ptr(), Hkv * G * D, G * D, D, d[4].data_ptr(), d[5].data_ptr(), S, W, d[1].data_ptr(), Hkv * D, D,
+            d[2].data_ptr(), Hkv * D, D, d[3].data_ptr(), Hkv * G * D, G * D, D, 0, d[6].data_ptr(), d[7].data_ptr(),
+            d[8].data_ptr(), d[9].data_ptr(), d[10].data_ptr(), N, max_len, Hkv, G, D, D ** -0.5, out.data_ptr(),
+            Hkv * G * D, G * D, D, None)
+
+    assert call(0) != 0 and call(1 << 30) != 0      # refused on the host
+    assert call(max(lens)) == 0
+    _check(_np(out), ref.numpy())
+    assert torch.equal(d[4].cpu(), want[0]) and torch.equal(d[5].cpu(), want[1])
+    assert lib().hsg_ring_pos_update(d[6].data_ptr(), S, W, d[7].data_ptr(), d[8].data_ptr(), d[9].data_ptr(), N,
+                                     max(lens), None) == 0
+    assert torch.equal(d[6].cpu(), want_pos)
