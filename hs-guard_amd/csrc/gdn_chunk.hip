@@ -1,4 +1,4 @@
-// Chunked gated-delta-rule prefill for gfx950 (WY/UT chunk form on MFMA), as two kernels.
+// Chunked gated-delta-rule prefill for gfx950 (WY/UT chunk form on MFMA).
 //
 // Same recurrence as the slot step (src/hs_guard/engine/fused_kernels.py:166-188), evaluated 64 tokens at a
 // time in the chunk form behind FLA's chunk_gated_delta_rule (called at src/hs_guard/runtime.py:80-89 and
@@ -103,6 +103,9 @@ struct ChunkParams {
   float* sq;
   uint8_t* ws;
   int32_t* order;                  // state kernel row order (in the workspace after the units)
+  int segs;                        // segments a row's chunks are cut into (1: walked whole)
+  float* bound;                    // [pairs][segs][KD][VD]: the state at each segment's start
+  float* trans;                    // [pairs][segs][KD][VD]: each segment's transition matrix
   // gated epilogue (hsg_gdn_chunk_prefill_gated): out = gated RMSNorm of o with z
   const uint16_t* z;
   int64_t z_stride;
@@ -605,17 +608,43 @@ __global__ __launch_bounds__(1024) void gdn_chunk_order_kernel(const ChunkParams
 // ---------------------------------------------------------------------------------------------------------
 constexpr int XP = 64 * 4;         // one handed-over fragment: 64 lanes x 4 bf16
 
-template <typename ST>
-__global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams p) {
+// The segment of a row's chunks that workgroup seg walks: [c_lo, c_hi) of its nch chunks; the row has n_segs of them.
+struct Segment {
+  int n_segs, c_lo, c_hi;
+};
+__device__ __forceinline__ Segment segment_of(int nch, int segs, int seg) {
+  const int cs = (nch + segs - 1) / segs;
+  return {(nch + cs - 1) / cs, seg * cs, min(nch, (seg + 1) * cs)};
+}
+__device__ __forceinline__ int64_t matrix_at(const ChunkParams& p, int n, int hv, int seg) {
+  return (((int64_t)n * p.HV + hv) * p.segs + seg) * (KD * VD);
+}
+
+// Few long rows (SEGMENTS): one workgroup per (row, head, value block) leaves most of the chip idle while each walks a
+// serial chain of 3.5 us a chunk. The chunk's update is linear in the state, S <- A S + B, so a row's chunks are cut
+// into segments that are walked at once, in three launches:
+//   transition (TRANS): every segment but the last from S = 0 (segment 0 from the row's state), which gives B of the
+//               whole segment, and every one but the first and last from S = I with V = 0, which gives A;
+//   combine:    S of each segment's start, S_{g+1} = A_g S_g + B_g, in fp32 (gdn_chunk_combine_kernel);
+//   output:     every segment from its start, with the outputs.
+// TRANS runs the chain waves alone: without the output waves' tiles two workgroups fit on a CU.
+// Measured with 16 heads (all launches of the call, whole -> segments): one row of 1,024 tokens 74.6 -> 63.5 us, 2,048
+// 137 -> 85, 8,000 493 -> 200 (state products 444 -> 80 + 20 + 70); two rows of 2,048 146 -> 117, of 8,000 535 -> 350.
+template <typename ST, bool TRANS>
+__global__ __launch_bounds__(TRANS ? 256 : 512) void gdn_chunk_state_kernel(const ChunkParams p) {
+  constexpr int THREADS = TRANS ? 256 : 512;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int w = wave & 3;                              // column group of the wave (both roles)
-  const bool chain = __builtin_amdgcn_readfirstlane(wave) < 4;   // wave-uniform role
+  const bool chain = TRANS || __builtin_amdgcn_readfirstlane(wave) < 4;   // wave-uniform role
   const int m16 = lane & 15;
   const int g4 = lane >> 4;
   // the two value blocks of one (row, head) are dispatched 8 workgroups apart, i.e. on the same XCD, so
   // their identical K / Q / workspace reads share that XCD's L2
   const int bid = blockIdx.x;
+  // TRANS: y < segs - 1: B of segment y; else A of segment y - (segs - 1) + 1
+  const bool identity = TRANS && (int)blockIdx.y >= p.segs - 1;
+  const int seg = (int)blockIdx.y - (identity ? p.segs - 2 : 0);
   const int vb = (bid >> 3) & 1;
   const int pair = ((bid >> 4) << 3) | (bid & 7);
   if (pair >= p.pairs) return;
@@ -629,39 +658,60 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
   const int vcol = vb * BV + w * 16 + m16;             // this lane's value column (accumulator layout)
   const int64_t ostride = (int64_t)p.HV * VD;
 
-  if (padded) {  // positions past the row's length are zeros in the padded layout
-    for (int t = ntok + threadIdx.x / BV; t < p.L; t += 512 / BV) {
+  if (!TRANS && padded && seg == 0) {  // positions past the row's length are zeros in the padded layout
+    for (int t = ntok + threadIdx.x / BV; t < p.L; t += THREADS / BV) {
       const int64_t at = (tok0 + t) * ostride + hv * VD + vb * BV + (threadIdx.x % BV);
       p.o[at] = 0;
       if (p.sq) p.sq[at] = 0.f;
     }
   }
   if (ntok == 0) return;
+  const Segment sg = segment_of((ntok + CH - 1) / CH, p.segs, seg);
+  if (TRANS ? seg >= sg.n_segs - 1 : seg >= sg.n_segs) return;
+  const int t_lo = sg.c_lo * CH, t_hi = min(ntok, sg.c_hi * CH);   // the segment's tokens
 
   // token-major K (two buffers), Q (swizzled rows, see swz) and V tiles; K^T and the token-column V fragments
   // are read with transpose reads
   __shared__ __align__(16) uint16_t Ks[2][CH * KD];
-  __shared__ __align__(16) uint16_t Qs[CH * KD];
+  __shared__ __align__(16) uint16_t Qs[TRANS ? 8 : CH * KD];
   __shared__ __align__(16) uint16_t Vs[CH * VS];
   // M' and P (two buffers) as scaled fp16 hi / lo planes of swizzled token-major rows (lower triangles used)
   __shared__ __align__(16) uint16_t Ms[2 * PL];
-  __shared__ __align__(16) uint16_t Ps[2][2 * PL];
+  __shared__ __align__(16) uint16_t Ps[2][TRANS ? 8 : 2 * PL];
   __shared__ __align__(16) float vec_s[2][VEC];
   // hand-over from chain to output waves, in the chain lanes' register layout (lane-linear 8-byte pieces):
   // Sx[w][2 mt + hl] = split S block mt of column group w, Vx[w][2 I + hl] = split V' token block I
-  __shared__ __align__(16) uint16_t Sx[4 * 16 * XP];
-  __shared__ __align__(16) uint16_t Vx[4 * 8 * XP];
+  __shared__ __align__(16) uint16_t Sx[TRANS ? 8 : 4 * 16 * XP];
+  __shared__ __align__(16) uint16_t Vx[TRANS ? 8 : 4 * 8 * XP];
   // the inverse power-of-two scales of the handed-over S and V' fragments, per value column of the block
   __shared__ __align__(16) float s_inv[BV], v_inv[BV];
 
   // ---- state S[:, vcol] in accumulator layout (chain waves): block mt holds keys 16 mt + 4 g4 + r ----
   ST* sbase = reinterpret_cast<ST*>(p.state) + ((slot * p.HV + hv) * (int64_t)KD) * VD + vcol;
+  const int64_t srow = (int64_t)(4 * g4) * VD + vcol;   // this lane's first element of a [KD][VD] matrix
   f32x4 S[8];
   if (chain) {
+    const bool from_state = TRANS ? seg == 0 : sg.n_segs == 1;
+    const float* const bound = p.bound + (from_state ? 0 : matrix_at(p, n, hv, seg)) + srow;
 #pragma unroll
     for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[mt][r] = load_state<ST>(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD);
+      for (int r = 0; r < 4; ++r) {
+        const int64_t at = (int64_t)(16 * mt + r) * VD;
+        if (TRANS && !from_state)
+          S[mt][r] = identity && 16 * mt + 4 * g4 + r == vcol ? 1.f : 0.f;
+        else if (from_state)
+          S[mt][r] = load_state<ST>(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD);
+        else
+          S[mt][r] = bound[at];
+      }
+    if (TRANS && seg == 0) {   // the output pass's start of segment 0: its last segment overwrites the row's state
+      float* const start = p.bound + matrix_at(p, n, hv, 0) + srow;
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) start[(int64_t)(16 * mt + r) * VD] = S[mt][r];
+    }
   }
 
   // ---- read offsets (bf16), fixed per lane; a row block (16 rows) is a plain offset added at the read (its rows'
@@ -712,7 +762,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
   // The two roles run separate loops with the same barriers (three per chunk, after a staging barrier), so
   // the registers of one role are not held across the other's code.
   if (chain) {
-    u32x4 pk[4], pm[3];
+    u32x4 pk[4], pm[3], pv[TRANS ? 2 : 1];
     float pf;
     auto fetch = [&](int c0) {
       const uint16_t* row = row_of(c0);
@@ -722,6 +772,11 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
 #pragma unroll
       for (int i = 0; i < 3; ++i) pm[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(unit) + qoff[i]);
       pf = reinterpret_cast<const float*>(unit + 4 * PL * 2)[rx];
+      if constexpr (TRANS) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          pv[j] = *reinterpret_cast<const u32x4*>(row + p.v_off + hv * VD + vb * BV + 8 * (sp + 4 * j));
+      }
     };
     auto stage = [&](int buf) {
       stage_rows(Ks[buf], pk);
@@ -729,16 +784,21 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       for (int i = 0; i < 3; ++i)
         *reinterpret_cast<u32x4*>(Ms + qoff[i]) = pm[i];
       vec_s[buf][rx] = pf;
+      if constexpr (TRANS) {
+        const uint32_t keep = identity ? 0u : ~0u;   // A: the recurrence without its values
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<u32x4*>(&Vs[st_t * VS + 8 * (sp + 4 * j)]) = pv[j] & keep;
+      }
     };
-    fetch(0);
+    fetch(t_lo);
     stage(0);
     lds_barrier();  // B0: chunk 0 staged
     int cb = 0;
-    for (int c0 = 0; c0 < ntok; c0 += CH, cb ^= 1) {
+    for (int c0 = t_lo; c0 < t_hi; c0 += CH, cb ^= 1) {
       const uint16_t* const K_ = Ks[cb];
       const float* const vec = vec_s[cb];
       // the next chunk (or this one again after the last: staged into idle buffers and never read)
-      fetch(c0 + CH < ntok ? c0 + CH : c0);
+      fetch(c0 + CH < t_hi ? c0 + CH : c0);
       // S 2^sS as fp16 hi / lo (sS from the largest |S| of this wave's 16 columns), handed over with 2^-sS
       s16x4 Sh[8], Sl[8];
       float amax = 0.f;
@@ -749,11 +809,15 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
 #pragma unroll
       for (int mt = 0; mt < 8; ++mt) {
         split4h(S[mt], ss, Sh[mt], Sl[mt]);
-        *reinterpret_cast<s16x4*>(sx + (2 * mt) * XP) = Sh[mt];
-        *reinterpret_cast<s16x4*>(sx + (2 * mt + 1) * XP) = Sl[mt];
+        if constexpr (!TRANS) {
+          *reinterpret_cast<s16x4*>(sx + (2 * mt) * XP) = Sh[mt];
+          *reinterpret_cast<s16x4*>(sx + (2 * mt + 1) * XP) = Sl[mt];
+        }
       }
-      if (g4 == 0) s_inv[w * 16 + m16] = inv_s;
-      lds_barrier();  // B1: split S handed over
+      if constexpr (!TRANS) {
+        if (g4 == 0) s_inv[w * 16 + m16] = inv_s;
+        lds_barrier();  // B1: split S handed over
+      }
 
       // ---- Y = Kr S for this wave's 16 value columns: S split hi / lo, key blocks paired ----
       f32x4 Y[4];
@@ -804,7 +868,7 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
         Vp[I] = acc * inv_mz;
         vmax = absmax4(Vp[I], vmax);
       }
-      {
+      if constexpr (!TRANS) {
         float inv_v;
         const float sv = pow2_scale(col_max(vmax), &inv_v);
 #pragma unroll
@@ -850,11 +914,19 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       stage(cb ^ 1);
       lds_barrier();  // B0: the next chunk is staged
     }
+    if constexpr (TRANS) {
+      float* const to = (identity ? p.trans + matrix_at(p, n, hv, seg) : p.bound + matrix_at(p, n, hv, seg + 1)) + srow;
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
+      for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) store_state(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD, S[mt][r]);
-  } else {
+        for (int r = 0; r < 4; ++r) to[(int64_t)(16 * mt + r) * VD] = S[mt][r];
+    } else if (seg == sg.n_segs - 1) {
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) store_state(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD, S[mt][r]);
+    }
+  } else if constexpr (!TRANS) {
     float inv_p;
     pow2_scale(p.scale, &inv_p);   // the P planes carry P 2^sP (gdn_chunk_prep_kernel)
     u32x4 pq[4], pv[2], pp[3];
@@ -877,14 +949,14 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
       for (int i = 0; i < 3; ++i)
         *reinterpret_cast<u32x4*>(Ps[buf] + qoff[i]) = pp[i];
     };
-    fetch(0);
+    fetch(t_lo);
     stage(0);
     lds_barrier();  // B0: chunk 0 staged
     int cb = 0;
-    for (int c0 = 0; c0 < ntok; c0 += CH, cb ^= 1) {
+    for (int c0 = t_lo; c0 < t_hi; c0 += CH, cb ^= 1) {
       const int nv = min(CH, ntok - c0);
       const float* const vec = vec_s[cb];
-      fetch(c0 + CH < ntok ? c0 + CH : c0);
+      fetch(c0 + CH < t_hi ? c0 + CH : c0);
       lds_barrier();  // B1: split S handed over
 
       // ---- QS^T = S^T Qr^T (value rows, token columns) from the handed-over split S ----
@@ -953,6 +1025,66 @@ __global__ __launch_bounds__(512) void gdn_chunk_state_kernel(const ChunkParams 
   }
 }
 
+// The states at the starts of a row's segments 2 on: bound[g + 1] holds B_g and becomes A_g bound[g] + B_g. One workgroup
+// per (row, head, 16 value columns); wave w owns rows 32 w .. 32 w + 31 of S, which the waves exchange through LDS. fp32
+// MFMA; the k order of a product is lane group g4's own four floats 16 j + 4 g4 + u, so A is read 16 bytes a lane. The
+// latency of each step's operands bounds it (20 us for the 6 steps of 8 segments; fetched a step ahead: 22 us).
+constexpr int CS = 20;             // row stride (fp32) of S in LDS: rows 4 apart are 16 banks apart
+__global__ __launch_bounds__(256) void gdn_chunk_combine_kernel(const ChunkParams p) {
+  __shared__ __align__(16) float Ss[2][KD * CS];
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+  const int m16 = lane & 15, g4 = lane >> 4;
+  const int n = blockIdx.y / p.HV;
+  const int hv = blockIdx.y - n * p.HV;
+  int64_t slot, tok0;
+  const int ntok = row_tokens(p, n, slot, tok0);
+  if (ntok == 0) return;
+  const int n_segs = segment_of((ntok + CH - 1) / CH, p.segs, 0).n_segs;
+  const int rows = 32 * w + 4 * g4;                       // + 16 b + r: this lane's rows of S
+  const int64_t col = blockIdx.x * 16 + m16;
+  if (n_segs < 3) return;
+  float* const bound = p.bound + matrix_at(p, n, hv, 0) + col;
+  const float* const trans = p.trans + matrix_at(p, n, hv, 0) + (int64_t)(32 * w + m16) * KD + 4 * g4;
+  f32x4 a[2][8], b[2];
+  auto fetch = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[t][j] = ld4f(trans + (int64_t)g * (KD * VD) + 16 * t * KD + 16 * j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) b[t][r] = bound[(int64_t)(g + 1) * (KD * VD) + (rows + 16 * t + r) * VD];
+    }
+  };
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      Ss[1][(rows + 16 * t + r) * CS + m16] = bound[(int64_t)(KD * VD) + (rows + 16 * t + r) * VD];
+  for (int g = 1; g < n_segs - 1; ++g) {
+    fetch(g);
+    lds_barrier();   // S_g is in Ss[g & 1], and the reads of S_{g - 1} are done
+    const float* const S = Ss[g & 1];
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float sv = S[(16 * j + 4 * g4 + u) * CS + m16];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] = mmf4(a[t][j][u], sv, acc[t]);
+      }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = acc[t][r] + b[t][r];
+        Ss[(g + 1) & 1][(rows + 16 * t + r) * CS + m16] = x;
+        bound[(int64_t)(g + 1) * (KD * VD) + (rows + 16 * t + r) * VD] = x;
+      }
+  }
+}
+
 // Gated RMSNorm of the chunk outputs (gated_finish, src/hs_guard/engine/fused_kernels.py:215-233, as the slot
 // step's fused epilogue computes it): one wave per token of a processed row, all value heads (2 values per lane
 // each, loads of every head issued together); out = bf16(bf16(w * bf16(o * rsqrt(mean(o^2) + eps))) * silu(z)).
@@ -994,6 +1126,15 @@ using hsg::ChunkParams;
 
 namespace {
 
+// Segments of a row's chunks (1: rows walked whole): as many as give one round of workgroups on the 256 CUs, two a
+// (row, head) and segment. Walking a row's segments twice needs four of them to pay (two rows of 16 heads: 535 -> 350 us,
+// where halves of three rows could save nothing), and 16 chunks (one row: 74.6 -> 63.5 us, and the two more launches
+// are a growing part of fewer).
+int segments(int64_t pairs, int max_chunks) {
+  const int64_t fit = 128 / pairs;
+  return fit < 4 || max_chunks < 16 ? 1 : (int)(fit < max_chunks / 2 ? fit : max_chunks / 2);
+}
+
 // Shared argument checks and the two launches (prep, state); returns HSG_OK after launching, or an error code.
 int chunk_launch(ChunkParams& p, int32_t state_dtype, int32_t n_rows, int32_t L, int32_t H, int32_t HV, int32_t K,
                  int32_t V, size_t workspace_bytes, hipStream_t s) {
@@ -1013,11 +1154,24 @@ int chunk_launch(ChunkParams& p, int32_t state_dtype, int32_t n_rows, int32_t L,
   p.order = reinterpret_cast<int32_t*>(p.ws + units * hsg::UNIT_BYTES);
   hipLaunchKernelGGL(hsg::gdn_chunk_prep_kernel, dim3((unsigned)units), dim3(256), 0, s, p);
   hipLaunchKernelGGL(hsg::gdn_chunk_order_kernel, dim3(1), dim3(1024), 0, s, p, (int)n_rows);
-  const dim3 grid((unsigned)(((p.pairs + 7) / 8) * 16));
+  // (without the workspace for segments, rows are walked whole)
+  const bool room = workspace_bytes >= hsg_gdn_chunk_segment_workspace_bytes(n_rows, L, HV);
+  p.segs = room ? segments(p.pairs, p.max_chunks) : 1;
+  const dim3 grid((unsigned)(((p.pairs + 7) / 8) * 16), (unsigned)p.segs);
+  if (p.segs > 1) {
+    p.bound = reinterpret_cast<float*>(p.ws + hsg_gdn_chunk_workspace_bytes(n_rows, L, HV));
+    p.trans = p.bound + (int64_t)p.pairs * p.segs * (hsg::KD * hsg::VD);
+    const dim3 tgrid(grid.x, (unsigned)(2 * p.segs - 3));
+    if (state_dtype == HSG_STATE_F32)
+      hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<float, true>), tgrid, dim3(256), 0, s, p);
+    else
+      hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<uint16_t, true>), tgrid, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(hsg::gdn_chunk_combine_kernel, dim3(hsg::VD / 16, (unsigned)p.pairs), dim3(256), 0, s, p);
+  }
   if (state_dtype == HSG_STATE_F32)
-    hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<float>), grid, dim3(512), 0, s, p);
+    hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<float, false>), grid, dim3(512), 0, s, p);
   else
-    hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<uint16_t>), grid, dim3(512), 0, s, p);
+    hipLaunchKernelGGL((hsg::gdn_chunk_state_kernel<uint16_t, false>), grid, dim3(512), 0, s, p);
   return HSG_OK;
 }
 
@@ -1060,6 +1214,14 @@ extern "C" size_t hsg_gdn_chunk_workspace_bytes(int32_t n_rows, int32_t L, int32
   // the units, then the state kernel's row order (int32 per row, rounded up to 256 bytes)
   return (size_t)n_rows * (size_t)((L + hsg::CH - 1) / hsg::CH) * (size_t)HV * (size_t)hsg::UNIT_BYTES +
          ((size_t)n_rows * 4 + 255) / 256 * 256;
+}
+
+extern "C" size_t hsg_gdn_chunk_segment_workspace_bytes(int32_t n_rows, int32_t L, int32_t HV) {
+  if (n_rows <= 0 || L <= 0 || HV <= 0) return 0;
+  // then the segments' start states and transition matrices
+  const int segs = segments((int64_t)n_rows * HV, (L - 1) / hsg::CH + 1);
+  return hsg_gdn_chunk_workspace_bytes(n_rows, L, HV) +
+         (segs > 1 ? (size_t)n_rows * HV * segs * 2 * (hsg::KD * hsg::VD) * sizeof(float) : 0);
 }
 
 extern "C" int hsg_gdn_chunk_prefill(const void* qkv, int64_t qkv_stride, int32_t q_off, int32_t k_off,

@@ -38,6 +38,7 @@ SIGNATURES = {
         _I32, _I32, _I32, _I32, _F,          # H, HV, K, V, scale
         _P, _P, _I32, _P]),                  # o, sq, burst_min, stream
     "hsg_gdn_chunk_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32]),
+    "hsg_gdn_chunk_segment_workspace_bytes": (ctypes.c_size_t, [_I32, _I32, _I32]),
     "hsg_gdn_chunk_prefill": (ctypes.c_int, [
         _P, _I64, _I32, _I32, _I32,
         _P, _P, _I64, _P, _P,

@@ -239,7 +239,8 @@ def gdn_chunk_prefill(packed, key_dim, heads, head_k, value_heads, head_v, a, b,
     scale = head_k ** -0.5 if scale is None else scale
     ws_bytes = lib().hsg_gdn_chunk_workspace_bytes(n, max(length, 1), value_heads)
     if workspace is None:
-        workspace = torch.empty(max(ws_bytes, 256), dtype=torch.uint8, device=packed.device)
+        best = lib().hsg_gdn_chunk_segment_workspace_bytes(n, max(length, 1), value_heads)
+        workspace = torch.empty(max(best, 256), dtype=torch.uint8, device=packed.device)
     _require(workspace.numel() >= ws_bytes, f"workspace needs {ws_bytes} bytes")
     rc = calls().hsg_gdn_chunk_prefill(
         _ptr(packed), c, 0, key_dim, 2 * key_dim, _ptr(a), _ptr(b), value_heads, _ptr(A_log), _ptr(dt_bias),

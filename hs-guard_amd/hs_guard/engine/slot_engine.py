@@ -290,7 +290,7 @@ class SlotStreamEngine(PreparedWeights):
             self.chunk_ws = self._chunk_workspace(self.max_rows, self.max_tick_tokens)
 
     def _chunk_workspace(self, rows, max_len):
-        ws = lib().hsg_gdn_chunk_workspace_bytes(rows, max_len, self.cfg.linear_num_value_heads)
+        ws = lib().hsg_gdn_chunk_segment_workspace_bytes(rows, max_len, self.cfg.linear_num_value_heads)
         return torch.empty(max(int(ws), 256), dtype=torch.uint8, device=self.device)
 
     def mm(self, x, w, out):

@@ -99,7 +99,7 @@ class WholeSequenceScorer(PreparedWeights):
         gated, att, act = heads[T * VD:2 * T * VD].view(T, VD), mid[:T * hq * D].view(T, hq * D), mid[:T * I].view(T, I)
         n_gdn = sum(1 for k, _ in self.kind if k == "linear_attention")
         state = torch.zeros(n_gdn, hv, kd, vd, dtype=torch.float32, device=dev)
-        ws_bytes = max(int(lib().hsg_gdn_chunk_workspace_bytes(1, T, hv)), 256) if n_gdn else 256
+        ws_bytes = max(int(lib().hsg_gdn_chunk_segment_workspace_bytes(1, T, hv)), 256) if n_gdn else 256
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         mm = torch.mm
         check(L.hsg_embed_rmsnorm(ids_d.data_ptr(), self.emb.data_ptr(), cfg.vocab_size,

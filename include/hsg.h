@@ -122,6 +122,12 @@ int hsg_gdn_conv_slot_step_gated(const void* proj, int64_t proj_stride, int32_t 
  * afterwards.
  */
 size_t hsg_gdn_chunk_workspace_bytes(int32_t n_rows, int32_t L, int32_t HV);
+
+/*
+ * The workspace with which a few long rows also run in segments (n_rows x HV <= 32, L > 960: five launches; elsewhere the
+ * size above). A call's launches depend on its sizes and workspace_bytes alone.
+ */
+size_t hsg_gdn_chunk_segment_workspace_bytes(int32_t n_rows, int32_t L, int32_t HV);
 int hsg_gdn_chunk_prefill(const void* qkv, int64_t qkv_stride, int32_t q_off, int32_t k_off, int32_t v_off,
                           const void* a, const void* b, int64_t ab_stride, const void* A_log,
                           const void* dt_bias, void* state, int32_t state_dtype, int64_t state_rows,

@@ -310,3 +310,55 @@ def test_chunk_output_rounding_rate_matches_slot_step():
           f"chunk state rel {worst:.2e}", flush=True)
     assert rate["chunk"] <= 1.5 * rate["step"]
     assert worst <= 1e-6
+
+
+@pytest.mark.parametrize("HV,lens,state_dtype,padded", [
+    (4, [1025, 64, 2048, 700, 0, 1, 129, 961], torch.float32, False), (16, [8000], torch.float32, False),
+    (8, [1000, 63, 1100], torch.float16, True), (2, [2000], torch.float16, False), (32, [1600], torch.float32, False)])
+def test_segments_match_whole_rows(HV, lens, state_dtype, padded):
+    """Few long rows run in segments: against the chunk form in float64, and no further from it than the same rows
+    walked whole (a workspace without room for segments) but for the noise of a float32 accumulation."""
+    from hs_guard._lib import lib
+    from hs_guard.engine.kernels import gdn_chunk_prefill
+    print(f"[chunk] segments HV={HV} {lens}", flush=True)
+    gen = torch.Generator().manual_seed(70 + HV)
+    H, K, N, L = max(HV // 2, 1), 128, len(lens), max(lens)
+    C = 2 * H * K + HV * K
+    base = lib().hsg_gdn_chunk_workspace_bytes(N, L, HV)
+    assert lib().hsg_gdn_chunk_segment_workspace_bytes(N, L, HV) > base
+    shape = (N, L) if padded else (sum(lens),)
+    offs = [n * L if padded else sum(lens[:n]) for n in range(N)]
+    packed = torch.randn(*shape, C, generator=gen).to(torch.bfloat16)
+    a, b = (torch.randn(*shape, HV, generator=gen).to(torch.bfloat16) for _ in range(2))
+    A_log = (torch.rand(HV, generator=gen) * 2 - 3).to(torch.bfloat16)     # slow decay: states cross segments
+    dt = (torch.randn(HV, generator=gen) - 3).to(torch.bfloat16)
+    state0 = (torch.randn(N + 1, HV, K, K, generator=gen) * 0.05).to(state_dtype)
+    slots = torch.randperm(N + 1, generator=gen)[:N]
+    dev = torch.device("cuda:0")
+    got = []
+    for ws in (None, torch.empty(base, dtype=torch.uint8, device=dev)):
+        state = state0.to(dev)
+        o, _ = gdn_chunk_prefill(packed.to(dev), H * K, H, K, HV, K, a.to(dev), b.to(dev), A_log.to(dev), dt.to(dev),
+                                 state, slots.to(dev), torch.tensor(lens, device=dev),
+                                 None if padded else torch.tensor(offs, device=dev), workspace=ws)
+        got.append((_np(o).reshape(-1, HV, K), _np(state)))
+    flat, af, bfl = (_np(t).reshape(-1, t.shape[-1]) for t in (packed, a, b))
+    tol = STATE_TOL if state_dtype == torch.float32 else 4e-3
+    for n, (ln, off, s) in enumerate(zip(lens, offs, slots.tolist())):
+        if padded:
+            assert np.count_nonzero(got[0][0][off + ln:off + L]) == 0
+        if ln == 0:
+            np.testing.assert_array_equal(got[0][1][s], _np(state0[s]))
+            continue
+        o_ref, s_ref = _row_reference(flat[off:off + ln], af[off:off + ln], bfl[off:off + ln], _np(A_log), _np(dt),
+                                      _np(state0[s]), H, HV, K, chunk=True)
+        errs = []
+        for o, state in got:
+            bad, worst = _out_close(o[off:off + ln], o_ref)
+            assert bad == 0, f"row {n}: {bad} outputs off (max diff {worst:.3e})"
+            errs.append(_state_err(state[s], s_ref))
+            assert max(errs[-1]) <= tol
+        print(f"[chunk] len {ln}: state err segments {errs[0]} whole {errs[1]}", flush=True)
+        assert errs[0][0] <= 1.5 * errs[1][0] + 1e-6
+    unused = [s for s in range(N + 1) if s not in slots.tolist()]
+    np.testing.assert_array_equal(got[0][1][unused], _np(state0[unused]))
