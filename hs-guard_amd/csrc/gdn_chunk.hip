@@ -63,7 +63,6 @@ constexpr int AS = CH + 4;         // row stride (fp32) of the prep kernel's -A 
                                    // 4 k-slots hits 64 distinct banks
 constexpr int VS = BV + 16;        // Vs row stride (bf16): 40 dwords, so the 4 x 4 pieces of a transpose read
                                    // fall in 16 distinct bank pairs
-constexpr int DS = 20;             // diagonal-block row stride (fp32) and diagonal-inverse row stride (bf16)
 constexpr int PW = CH;             // row width (bf16) of the workspace planes M', P (swizzled rows, see swz)
 constexpr int PL = CH * PW;        // one 64 x 64 bf16 plane of the workspace (also the state kernel's LDS layout)
 constexpr int VEC = 256;           // per-token factor floats of a workspace unit: e^G rk, rq e^G, rk e^(G_C-G),
@@ -287,8 +286,13 @@ __device__ __forceinline__ uint8_t* unit_ptr(const ChunkParams& p, int n, int c,
 
 // ---------------------------------------------------------------------------------------------------------
 // Prep: M' = (I + A)^-1 diag(beta), P and the per-token factors of one (row, chunk, value head).
+// Bound by the latency of its serial steps (token loads, decay scan, Gram tiles, inverses, four substitution steps, a
+// barrier between each) and by vector issue, so what counts is workgroups in flight: everything after the Gram tiles
+// lives in the K and Q tiles' LDS (37.6 KB in all, 4 workgroups a CU), and the tiles share their exponentials (a lane
+// took 20, now 4; 136 -> 68 registers). 16 rows of 512 to 8,000 tokens, 16 heads: 297 -> 254 us (three workgroups a
+// CU 297, four 273, with shared exponentials 254); one row of 8,000 42.3 -> 36.8 us.
 // ---------------------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p) {
+__global__ __launch_bounds__(256, 4) void gdn_chunk_prep_kernel(const ChunkParams p) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int m16 = lane & 15;
@@ -315,10 +319,9 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
   __shared__ __align__(16) uint16_t Ks[CH * KS];
   __shared__ __align__(16) uint16_t Qs[CH * KS];
   float* const nA = reinterpret_cast<float*>(Qs);                // -A (strictly lower), fp32, row stride AS
-  __shared__ __align__(16) float Dg[4 * 16 * DS];                // fp32 diagonal 16 x 16 blocks of -A
-  __shared__ __align__(16) float Tf[CH * DS];                    // their inverses, fp32 (rows 16w + i of block w)
   __shared__ __align__(16) float rk_s[CH], rq_s[CH], g_s[CH], b_s[CH], fa_s[CH];
   __shared__ __align__(16) double G_s[CH];   // in-chunk cumulative log-decay (see the scan below)
+  __shared__ __align__(16) float er_s[CH], rc_s[3][CH];   // the off-diagonal tiles' decay factors (below)
   __shared__ float red_s[4];
 
   // ---- stage token st_t: raw K, Q rows into LDS, l2-norm factors, gates. Past the row's end the chunk's
@@ -386,22 +389,34 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
     const float eg = exp_nonpos_d(x);
     G_s[lane] = x;
     fa_s[lane] = b_s[lane] * rk_s[lane];
+    // Left of the diagonal, with b the first token of row block I: e^(G_i - G_j) = e^(G_i - G_b) e^(G_b - G_j), both
+    // at most 1, so a tile needs no exponentials of its own (64 + 96 of them against 1,536 in the 12 tiles)
+    er_s[lane] = exp_nonpos_d(x - __shfl(x, lane & 48, 64));
+#pragma unroll
+    for (int I = 1; I < 4; ++I)
+      rc_s[I - 1][lane] = rk_s[lane] * exp_nonpos_d(fmin(__shfl(x, 16 * I, 64) - x, 0.0));
     vec_g[lane] = eg * rk_s[lane];
     vec_g[CH + lane] = rq_s[lane] * eg;
     vec_g[2 * CH + lane] = rk_s[lane] * exp_nonpos_d(GC - x);
     if (lane != 1) vec_g[3 * CH + lane] = lane == 0 ? exp_nonpos_d(GC) : 0.f;   // lane 1 later: M''s inverse scale
   }
 
-  // ---- Kr Kr^T and Qr Kr^T on the 10 lower 16 x 16 tiles each; tile u of wave w is number w + 4u. Each
-  // tile is computed transposed (operands swapped), so a lane holds row 16 I + m16, columns 16 J + 4 g4 .. +3 ----
+  // ---- Kr Kr^T and Qr Kr^T on the 10 lower 16 x 16 tiles each. Wave w takes both diagonal tiles of row block w (u =
+  // 0, 1: they share their decays) and tiles w, w + 4, w + 8 of the 12 others. Each tile is computed transposed
+  // (operands swapped), so a lane holds row 16 I + m16, columns 16 J + 4 g4 .. +3 ----
+  auto tile = [&](int u, bool& qk, int& I, int& J) __attribute__((always_inline)) {
+    const int t = wave + 4 * (u - 2);
+    const int idx = t >= 6 ? t - 6 : t;
+    qk = u < 2 ? u == 1 : t >= 6;
+    I = u < 2 ? wave : idx >= 3 ? 3 : idx >= 1 ? 2 : 1;
+    J = u < 2 ? wave : idx - I * (I - 1) / 2;
+  };
   f32x4 gt[5];
 #pragma unroll
   for (int u = 0; u < 5; ++u) {
-    const int tau = wave + 4 * u;
-    const bool qk = tau >= 10;
-    const int idx = qk ? tau - 10 : tau;
-    const int I = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-    const int J = idx - I * (I + 1) / 2;
+    bool qk;
+    int I, J;
+    tile(u, qk, I, J);
     const uint16_t* arow = (qk ? Qs : Ks) + (16 * I + m16) * KS + 8 * g4;
     const uint16_t* brow = Ks + (16 * J + m16) * KS + 8 * g4;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -420,43 +435,29 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
   {
     float inv_p;
     const float sp = pow2_scale(p.scale, &inv_p);
-    float fr[5];
-    double Gr[5], Gc[5][4];
-    f32x4 rkc[5];
+    f32x4 dk;   // rk_j e^(G_i - G_j) of the diagonal tiles
+    {
+      const int j0 = 16 * wave + 4 * g4;
+      const double Gr = G_s[16 * wave + m16];
+      const f32x4 rkc = ld4f(&rk_s[j0]);
 #pragma unroll
-    for (int u = 0; u < 5; ++u) {
-      const int tau = wave + 4 * u;
-      const bool qk = tau >= 10;
-      const int idx = qk ? tau - 10 : tau;
-      const int I = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-      const int J = idx - I * (I + 1) / 2;
-      const int i = 16 * I + m16;
-      const int j0 = 16 * J + 4 * g4;
-      fr[u] = qk ? rq_s[i] : fa_s[i];
-      Gr[u] = G_s[i];
-      rkc[u] = ld4f(&rk_s[j0]);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Gc[u][r] = G_s[j0 + r];
+      for (int r = 0; r < 4; ++r) dk[r] = rkc[r] * exp_nonpos_d(fmin(Gr - G_s[j0 + r], 0.0));
     }
 #pragma unroll
     for (int u = 0; u < 5; ++u) {
-      const int tau = wave + 4 * u;
-      const bool qk = tau >= 10;
-      const int idx = qk ? tau - 10 : tau;
-      const int I = idx >= 6 ? 3 : idx >= 3 ? 2 : idx >= 1 ? 1 : 0;
-      const int J = idx - I * (I + 1) / 2;
+      bool qk;
+      int I, J;
+      tile(u, qk, I, J);
       const int i = 16 * I + m16;
       const int j0 = 16 * J + 4 * g4;
-      f32x4 v;
+      const float fr = (qk ? rq_s[i] : fa_s[i]) * (u < 2 ? 1.f : er_s[i]);
+      f32x4 v = fr * (u < 2 ? dk : ld4f(&rc_s[I - 1][j0])) * gt[u];
+      if (u == 1) {   // inside a diagonal tile of P keep row >= column (sign bit of column - row - 1)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        v[r] = fr[u] * rkc[u][r] * exp_nonpos_d(fmin(Gr[u] - Gc[u][r], 0.0)) * gt[u][r];
-        // inside a diagonal tile of P keep row >= column (sign bit of column - row - 1)
-        if (qk && I == J) v[r] *= (float)((uint32_t)((4 * g4 + r) - m16 - 1) >> 31);
+        for (int r = 0; r < 4; ++r) v[r] *= (float)((uint32_t)((4 * g4 + r) - m16 - 1) >> 31);
       }
       if (!qk) {
         *reinterpret_cast<f32x4*>(&nA[i * AS + j0]) = -v;
-        if (I == J) *reinterpret_cast<f32x4*>(&Dg[i * DS + 4 * g4]) = -v;
       } else {
         s16x4 vh, vl;
         split4h(v, sp, vh, vl);
@@ -469,14 +470,14 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
 
   // ---- wave w inverts diagonal block w of (I + A) by fp32 forward substitution (lane m16 = column) ----
   {
-    const float* nb = Dg + (16 * wave) * DS;   // -A of the block
+    float* nb = nA + (16 * wave) * (AS + 1);   // -A of the block, then its inverse
     float t[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       float s0 = (i == m16) ? 1.f : 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
 #pragma unroll
       for (int k = 0; k < i; ++k) {
-        const float a = nb[i * DS + k];
+        const float a = nb[i * AS + k];
         if ((k & 3) == 0) s0 += a * t[k];
         else if ((k & 3) == 1) s1 += a * t[k];
         else if ((k & 3) == 2) s2 += a * t[k];
@@ -488,20 +489,20 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
     // by lane group was lowered to branches over a scratch copy of t and stored row 11 as row 15)
     if (g4 == 0) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) Tf[(wave * 16 + i) * DS + m16] = t[i];
+      for (int i = 0; i < 16; ++i) nb[i * AS + m16] = t[i];
     }
   }
   lds_barrier();  // diagonal inverses are complete
 
   // ---- M_I = T_II (E_I + sum_{J<I} (-A)_IJ M_J) for this wave's columns 16w + m16 (E = identity), in fp32 on
   // 16x16x4 fp32 MFMAs (lane: row / column m16, k-slot g4). Every operand is read back in B layout by other lanes
-  // of the wave, so each block goes through LDS: x_I in the wave's 16 x 16 slice of Dg (free once the diagonal
-  // inverses are done), M_I in its 64 x 16 slice of Ks. Each hand-off is a fenced workgroup barrier (all waves run
+  // of the wave, so each block goes through LDS: x_I in a 16 x 16 block of nA above the diagonal (those hold nothing that
+  // is read), M_I in its 64 x 16 slice of Ks. Each hand-off is a fenced workgroup barrier (all waves run
   // this loop): without an ordering point the compiler may hoist a lane's read of M_J above the stores of other
   // lanes whenever the lane's own store addresses provably differ, and the read then returns the stale x_J.
   // Then M' = M diag(beta). ----
   float* const Mf = reinterpret_cast<float*>(Ks) + wave * (CH * 16);
-  float* const Xf = Dg + wave * (16 * DS);
+  float* const Xf = nA + (wave == 3 ? 16 * AS + 32 : 16 * (wave + 1));
   f32x4 mp[4];
   {
     const float bcol = b_s[16 * wave + m16];
@@ -519,13 +520,13 @@ __global__ __launch_bounds__(256) void gdn_chunk_prep_kernel(const ChunkParams p
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         acc[r] += (I == wave && 4 * g4 + r == m16) ? 1.f : 0.f;
-        Xf[(4 * g4 + r) * DS + m16] = acc[r];
+        Xf[(4 * g4 + r) * AS + m16] = acc[r];
       }
       lds_barrier();   // x_I is complete (and the previous block's reads of Xf are done)
       f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        v = mmf4(Tf[(16 * I + m16) * DS + 4 * j + g4], Xf[(4 * j + g4) * DS + m16], v);
+        v = mmf4(nA[(16 * I + m16) * AS + 16 * I + 4 * j + g4], Xf[(4 * j + g4) * AS + m16], v);
 #pragma unroll
       for (int r = 0; r < 4; ++r) Mf[(16 * I + 4 * g4 + r) * 16 + m16] = v[r];
       lds_barrier();   // M_I is complete before the next block reads it, and x_I has been read
