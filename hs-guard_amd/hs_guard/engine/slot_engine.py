@@ -398,11 +398,11 @@ class SlotStreamEngine(PreparedWeights):
                 "lens": x[2 * tb + nb:2 * tb + 2 * nb], "slots": x[2 * tb + 2 * nb:2 * tb + 3 * nb],
                 "starts": x[2 * tb + 3 * nb:2 * tb + 4 * nb], "all": x[:2 * tb + 4 * nb]}
 
-    def _forward(self, nb, tb, inp, scratch=None, max_len=0):
+    def _forward(self, nb, tb, inp, scratch=None, max_len=0, short_rows=True):
         """The tick's device program (src/hs_guard/engine/slot_engine_v8.py:30-58), launched on the current
         stream. Reads only device memory, so it can be captured into a hipGraph. max_len > 0: a long piece's program
-        (_run_long) over its own ``scratch``, every row of up to max_len tokens on the chunk kernels and
-        hsg_ring_prefill."""
+        (_run_long) over its own ``scratch``, every row of up to max_len tokens on hsg_ring_prefill and, from
+        chunk_min_tokens on, the chunk kernels (short_rows False: no row is shorter)."""
         L = calls()
         long = max_len > 0
         buf, chunk_ws = scratch or (self.buf, getattr(self, "chunk_ws", None))
@@ -479,7 +479,7 @@ class SlotStreamEngine(PreparedWeights):
                                                  max_len or (self.max_tick_tokens if R else 0), C,
                                                  conv.data_ptr(), C, st),
                           "hsg_conv_silu_update")
-                    if not long:
+                    if not long or short_rows:
                         check(L.hsg_gdn_slot_step_gated(
                             conv.data_ptr(), C, 0, cfg.key_dim, 2 * cfg.key_dim,
                             base + 2 * (C + cfg.value_dim + hv), base + 2 * (C + cfg.value_dim), self.gdn_in,
@@ -496,7 +496,7 @@ class SlotStreamEngine(PreparedWeights):
                             _STATE_CODE[self.state_dtype], S, slots.data_ptr(), lens.data_ptr(), offsets.data_ptr(),
                             R, max_len or self.max_tick_tokens, nh, hv, kd, vd, kd ** -0.5,
                             view("gdn_o", tb, cfg.value_dim).data_ptr(), base + 2 * C, self.gdn_in,
-                            Lw["norm_w"].data_ptr(), eps, out.data_ptr(), 0 if long else self.chunk_min_tokens,
+                            Lw["norm_w"].data_ptr(), eps, out.data_ptr(), self.chunk_min_tokens,
                             chunk_ws.data_ptr(), chunk_ws.numel(), st), "hsg_gdn_chunk_prefill_gated")
                 self.mm(out, Lw["w_out"], mix)
             else:
@@ -659,8 +659,9 @@ class SlotStreamEngine(PreparedWeights):
         a piece of LONG_TOKENS tokens in all does both once: 3 rows of 900 tokens through 4 layers 7.15 -> 1.70 ms, and
         at 24 layers one row of 65 tokens 2.88 -> 2.58 ms, 32 rows of 256 23.4 -> 18.7 ms, one of 65 beside 31 of 1 token
         3.67 -> 3.16 ms. From 33 rows on a piece would hold no more than two ticks a row, and ticks keep their graphs
-        (32 rows of 128 gained 20 %). Engines set up with smaller ticks or without the chunk kernels keep ticks."""
-        if not self.chunk_min_tokens or self.max_tick_tokens < 64 or longest <= 64:
+        (32 rows of 128 gained 20 %). Engines set up with smaller ticks, without the chunk kernels or with a
+        chunk_min_tokens that no tick's row reaches keep ticks."""
+        if not 0 < self.chunk_min_tokens <= 64 or self.max_tick_tokens < 64 or longest <= 64:
             return 0
         piece = LONG_TOKENS // rows // 64 * 64
         return piece if piece >= 128 else 0
@@ -689,7 +690,8 @@ class SlotStreamEngine(PreparedWeights):
         offsets[order] = offsets_p
         inp = self._inputs(n, tb, scratch[0])
         inp["all"].copy_(host)
-        probs = self._forward(n, tb, inp, scratch, int(row_lens.max())).cpu()
+        short = bool(((row_lens > 0) & (row_lens < self.chunk_min_tokens)).any())
+        probs = self._forward(n, tb, inp, scratch, int(row_lens.max()), short).cpu()
         self.stats["eager_steps"] += 1
         self.length[slots] += lens
         return probs.numpy()[:, :total], lens, offsets

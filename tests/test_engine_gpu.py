@@ -502,3 +502,42 @@ def test_long_pieces_match_ticks(sizes):
     assert ticks.stats["eager_steps"] == 0
     np.testing.assert_array_equal(long.length, ticks.length)
     assert torch.equal(long.ring_pos[:len(sizes)], ticks.ring_pos[:len(sizes)])
+
+
+@pytest.mark.parametrize("chunk_min_tokens,routes", [(16, {("slot", 16), ("chunk", 16)}), (1, {("chunk", 1)}),
+                                                     (65, set())])
+def test_long_pieces_keep_the_chunk_rule(monkeypatch, chunk_min_tokens, routes):
+    """A long piece's rows of fewer than chunk_min_tokens tokens run the slot step, as in ticks, and an engine whose
+    chunk_min_tokens no tick's row reaches runs no long piece."""
+    from hs_guard.engine import slot_engine
+    from hs_guard.model import GuardConfig, GuardModel
+    cfg = GuardConfig(vocab_size=1000, hidden_size=1024, num_hidden_layers=2,
+                      layer_types=["linear_attention", "full_attention"], intermediate_size=1024,
+                      linear_num_key_heads=2, linear_num_value_heads=4, num_attention_heads=8,
+                      num_key_value_heads=2, window_tokens=96)
+    model = GuardModel.random(cfg, seed=1, device="cpu", std=0.005).to("cuda:0")
+    eng = slot_engine.SlotStreamEngine(model, 3, use_graphs=False, chunk_min_tokens=chunk_min_tokens)
+    native, seen = slot_engine.calls(), set()
+
+    class Recorded:
+        def __getattr__(self, name):
+            fn = getattr(native, name)
+            if name == "hsg_gdn_slot_step_gated":        # skip_min_len: third from last of its arguments
+                return lambda *args: seen.add(("slot", args[-3])) or fn(*args)
+            if name == "hsg_gdn_chunk_prefill_gated":    # min_len: fourth from last
+                return lambda *args: seen.add(("chunk", args[-4])) or fn(*args)
+            return fn
+
+    long_piece, pieces = eng._run_long, []
+
+    def run_long(*args):
+        with monkeypatch.context() as m:
+            m.setattr(slot_engine, "calls", Recorded)
+            pieces.append(len(args[0]))
+            return long_piece(*args)
+
+    eng._run_long = run_long
+    out = eng.step([(0, list(range(100))), (1, [1, 2, 3]), (2, list(range(17)))])
+    for role in out:
+        assert all(torch.isfinite(p).all() for p in out[role])
+    assert pieces == ([3] if routes else []) and seen == routes
