@@ -60,9 +60,9 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* hidden, const ui
 // ext = [pool rows ; new tokens]. A thread takes VEC adjacent channels (2 where every row is 4-byte aligned) over
 // blocks of CONV_TB tokens, the 3-row window sliding in registers; block z of a row starts from the 3 raw rows before
 // it, so a row's blocks run in parallel workgroups. The threads of block 0 own the pool row: they read it first and
-// write the row's last 3 raw rows back, so no other block reads or writes it. The SiLU (exp and an IEEE divide per
-// value) and the 4 bytes per value bound it about equally: one 8,000-token row of 6,144 channels 49.6 us (3.96 TB/s; 54.8
-// as 64-token segments of one channel per thread), one of 311 tokens 6.5 us (12.0).
+// write the row's last 3 raw rows back, so no other block reads or writes it. The SiLU
+// and the 4 bytes per value bound it about equally: one 8,000-token row of 6,144 channels 40.6 us (4.84 TB/s; 54.8 as
+// 64-token segments of one channel per thread, 49.5 with expf and an IEEE divide), one of 311 tokens 6.3 us (12.0).
 // ---------------------------------------------------------------------------------------------------
 constexpr int KS = 4;
 constexpr int CONV_TB = 16;
@@ -174,8 +174,8 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int
 // gated_finish (src/hs_guard/engine/fused_kernels.py:215-233), as the slot step's fused epilogue computes it:
 // r = rsqrt(mean(o^2) + eps) over the head, out = bf16(bf16(w * bf16(o * r)) * silu(z)), o already bf16.
 // A lane holds VEC values: 8 (16 lanes a head, 16-byte pieces, four heads per wave) where every row is 16-byte aligned,
-// else 2 (a wave per head). HBM-bound: 8,000 tokens of 16 heads 23.0 us (4.3 TB/s; 31.9 with
-// 2 values per lane).
+// else 2 (a wave per head). HBM-bound: 8,000 tokens of 16 heads 18.7 us (5.3 TB/s; 31.9 with
+// 2 values per lane, 22.7 before the SiLU's shorter form).
 // ---------------------------------------------------------------------------------------------------
 template <int VEC>
 __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const uint16_t* x, int64_t x_stride, const uint16_t* z,

@@ -71,8 +71,27 @@ __device__ __forceinline__ void store4_bf16(uint16_t* p, const float* x) {
   *reinterpret_cast<uint2*>(p) = w;
 }
 
-__device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
-__device__ __forceinline__ float siluf_(float x) { return x / (1.0f + expf(-x)); }
+// ---- sigmoid and SiLU: the denominator's exponential is e^-x = 2^hi (1 + lo ln 2) with hi + lo = -x log2(e) to twice
+// fp32's digits, without a range reduction (its result is only added to 1), and the quotient is a reciprocal with one
+// correction step, whose special cases v_div_fixup settles. The quarter of the denominator is used, so its reciprocal is a
+// normal number. The kernels that take a SiLU per value are bound by vector issue: with expf and an IEEE divide 8,000
+// tokens took 49.5 us in the conv (now 40.6), 22.7 in the gated norm (18.7), 28.9 in the SiLU-mul (27.5); three rows of
+// 900 tokens of ring attention 93.8 us (88.5); a one-token step of 24 layers 792 us (765). The SiLU of every bf16 value
+// rounds to the same bf16 as before. ----
+__device__ __forceinline__ float quarter_one_plus_exp_neg(float x) {   // (1 + e^-x) / 4
+  constexpr float LOG2E = 1.44269502f, LOG2E_LO = 1.92596303e-8f, LN2_4 = 0.173286795f;
+  const float y = __builtin_amdgcn_fmed3f(x, -200.f, 200.f);   // keeps lo finite
+  const float hi = y * -LOG2E;
+  const float lo = __builtin_fmaf(y, -LOG2E_LO, __builtin_fmaf(y, -LOG2E, -hi));
+  return __builtin_fmaf(__builtin_amdgcn_exp2f(hi), __builtin_fmaf(lo, LN2_4, 0.25f), 0.25f);
+}
+__device__ __forceinline__ float quotient(float a, float b) {   // a / b, 1 / b a normal number
+  const float r = __builtin_amdgcn_rcpf(b);
+  const float q = a * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), r, q), b, a);
+}
+__device__ __forceinline__ float sigmoidf_(float x) { return quotient(0.25f, quarter_one_plus_exp_neg(x)); }
+__device__ __forceinline__ float siluf_(float x) { return quotient(0.25f * x, quarter_one_plus_exp_neg(x)); }
 
 // ---- wave64 butterfly sums (every lane ends with the same bitwise value) ----
 template <int MASK>

@@ -434,7 +434,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecParams p) 
       float gt[4];
       load4_bf16(grow + g * p.g_sg + d, gt);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = y[i] * rbf(1.0f / (1.0f + expf(-gt[i])));
+      for (int i = 0; i < 4; ++i) y[i] = y[i] * rbf(sigmoidf_(gt[i]));
     }
     store4_bf16(orow + g * p.o_sg + d, y);
   }
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(256) void decode_fused_kernel(const DecParams p) {
           unpack2(gw[g].x, gt[0], gt[1]);
           unpack2(gw[g].y, gt[2], gt[3]);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) y[e] = y[e] * rbf(1.0f / (1.0f + expf(-gt[e])));
+          for (int e = 0; e < 4; ++e) y[e] = y[e] * rbf(sigmoidf_(gt[e]));
         }
         store4_bf16(orow + g * p.o_sg + 4 * lane, y);
       }

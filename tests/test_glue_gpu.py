@@ -278,3 +278,19 @@ def test_conv_token_blocks(lens, L, C, history):
             _close(got[offs[n]:offs[n] + lens[n]], ref_out[n, :lens[n]], f"conv row {n}", atol=atol, ulps=2)
     if history:
         np.testing.assert_array_equal(_np(pool_d), ref_pool)
+
+
+def test_silu_of_every_bf16():
+    """SiLU of all 65,536 bf16 values (silu_mul with up = 1): the float64 value correctly rounded down to x = -88.5 (its
+    fp32 error, about 2 ulp, never crosses a bf16 rounding boundary there), past which 1 + e^-x leaves fp32's range and
+    the result is 0 or the value, both under 1e-35; infinities and NaN as x / (1 + e^-x) gives them."""
+    from hs_guard.engine.kernels import silu_mul
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    out = silu_mul(x.to("cuda:0"), torch.ones_like(x, device="cuda:0")).cpu()
+    ref = x.double() / (1 + torch.exp(-x.double()))
+    normal = torch.isfinite(x) & (x > -88.5)
+    assert torch.equal(out[normal], ref[normal].to(torch.bfloat16))
+    low = torch.isfinite(x) & (x <= -88.5)
+    assert bool((out[low].float().abs() < 1e-35).all())
+    assert torch.equal(out[~torch.isfinite(x)].isnan(), ~(x[~torch.isfinite(x)] == torch.inf))
+    assert float(out[x == torch.inf]) == torch.inf
