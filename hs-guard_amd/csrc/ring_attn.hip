@@ -326,7 +326,7 @@ __device__ __forceinline__ void attend_group(const RingParams& p, const Row& ro,
     for (int t = 0; t < D / 16; ++t) {
       float y[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(O[t][i] / l_run) : 0.f;
+      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(quotient(O[t][i], l_run)) : 0.f;
       if (gsrc) {
         float gt[4];
         unpack2(gw[t][0], gt[0], gt[1]);
@@ -588,7 +588,7 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
     for (int t = 0; t < 4; ++t) {
       float y[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(o[t][i] / l_tot) : 0.f;
+      for (int i = 0; i < 4; ++i) y[i] = valid ? rbf(quotient(o[t][i], l_tot)) : 0.f;
       if (ro.grow) {
         float gt[4];
         unpack2(gw[t][0], gt[0], gt[1]);

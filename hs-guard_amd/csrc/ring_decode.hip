@@ -429,7 +429,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecParams p) 
     }
     float y[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = l > 0.f ? rbf(o[i] / l) : 0.f;
+    for (int i = 0; i < 4; ++i) y[i] = l > 0.f ? rbf(quotient(o[i], l)) : 0.f;
     if (grow) {
       float gt[4];
       load4_bf16(grow + g * p.g_sg + d, gt);
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(256) void decode_fused_kernel(const DecParams p) {
         for (int w = 0; w < NWV; ++w) l += lsum_s[w][g];
         float y[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = l > 0.f ? rbf(acc[g][e] / l) : 0.f;
+        for (int e = 0; e < 4; ++e) y[e] = l > 0.f ? rbf(quotient(acc[g][e], l)) : 0.f;
         if (grow) {
           float gt[4];
           unpack2(gw[g].x, gt[0], gt[1]);
