@@ -79,7 +79,8 @@ __device__ __forceinline__ void store4_bf16(uint16_t* p, const float* x) {
 // 900 tokens of ring attention 93.8 us (88.5); a one-token step of 24 layers 792 us (765). The SiLU of every bf16 value
 // rounds to the same bf16 as before. The attention outputs' division by the
 // softmax sum takes quotient too: 72 padded rows of 2 to 64 steps 93.3 -> 90.8 us a call, bitwise the same. ----
-__device__ __forceinline__ float quarter_one_plus_exp_neg(float x) {   // (1 + e^-x) / 4
+// (1 + e^-x) / 4. The clamp is a median, which takes -200 for a NaN: the callers' numerators carry the NaN.
+__device__ __forceinline__ float quarter_one_plus_exp_neg(float x) {
   constexpr float LOG2E = 1.44269502f, LOG2E_LO = 1.92596303e-8f, LN2_4 = 0.173286795f;
   const float y = __builtin_amdgcn_fmed3f(x, -200.f, 200.f);   // keeps lo finite
   const float hi = y * -LOG2E;
@@ -91,7 +92,7 @@ __device__ __forceinline__ float quotient(float a, float b) {   // a / b, 1 / b 
   const float q = a * r;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-b, q, a), r, q), b, a);
 }
-__device__ __forceinline__ float sigmoidf_(float x) { return quotient(0.25f, quarter_one_plus_exp_neg(x)); }
+__device__ __forceinline__ float sigmoidf_(float x) { return quotient(x == x ? 0.25f : x, quarter_one_plus_exp_neg(x)); }
 __device__ __forceinline__ float siluf_(float x) { return quotient(0.25f * x, quarter_one_plus_exp_neg(x)); }
 
 // ---- wave64 butterfly sums (every lane ends with the same bitwise value) ----

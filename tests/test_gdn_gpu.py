@@ -285,3 +285,46 @@ def test_conv_fused_step_equals_conv_then_step(state_code, burst_min):
                                           state_code, S, sl.data_ptr(), ln.data_ptr(), of.data_ptr(), N, H // 2, HV, K,
                                           K, K ** -0.5, z_ptr, stride, nwd.data_ptr(), 1e-6, out_b.data_ptr(),
                                           burst_min, st) == -3
+
+
+BETAS = [float("nan"), -float("nan"), float("inf"), -float("inf"), 3e38, -3e38, 200.0, -200.0, 100.0, -100.0, 88.5, -88.5,
+         30.0, -30.0, 17.0, -17.0, 8.0, -8.0, 3.0, -3.0, 1.0, -1.0, 0.5, -0.5, 1e-3, -1e-3, 1e-30, -1e-30, 1e-40, -1e-40, 0.0,
+         -0.0]
+
+
+@pytest.mark.parametrize("route,L", [("step", 1), ("step", 7), ("burst", 20), ("chunk", 1), ("chunk", 70), ("chunk", 1100)])
+def test_every_beta(route, L):
+    """The last token's beta = sigmoid(b) over NaN, infinities and finite b on each GDN path: a NaN reaches that token's
+    output and the whole state of its (row, head), and nothing else; every other head matches the float64 recurrence."""
+    from hs_guard.engine.kernels import gdn_chunk_prefill, gdn_slot_v8
+    print(f"[gdn] betas {route} L={L}", flush=True)
+    gen = torch.Generator().manual_seed(9)
+    K, H = 128, 8
+    N = len(BETAS) // H if L < 1000 else 1
+    packed = torch.randn(N, L, 3 * H * K, generator=gen).to(torch.bfloat16)
+    a, b = (torch.randn(N, L, H, generator=gen).to(torch.bfloat16) for _ in range(2))
+    b[:, L - 1] = torch.tensor(BETAS[:N * H]).to(torch.bfloat16).view(N, H)
+    A_log, dt = (torch.randn(H, generator=gen).to(torch.bfloat16) for _ in range(2))
+    state0 = torch.randn(N + 1, H, K, K, generator=gen) * 0.05
+    lens = torch.full((N,), L)
+    dev = torch.device("cuda:0")
+    state = state0.to(dev)
+    args = (packed.to(dev), H * K, H, K, H, K, a.to(dev), b.to(dev), A_log.to(dev), dt.to(dev), state,
+            torch.arange(N, device=dev), lens.to(dev))
+    o = gdn_chunk_prefill(*args)[0] if route == "chunk" else gdn_slot_v8(*args, burst_min=8 if route == "burst" else 0)[0]
+    nan = b[:, L - 1].isnan()
+    finite = torch.where(b.isnan(), torch.zeros_like(b), b)
+    o_ref, _, st_ref = ogdn.gdn_slot_step(_np(packed), H * K, H, K, H, K, _np(a), _np(finite), _np(A_log), _np(dt),
+                                          _np(state0), np.arange(N), lens.numpy())
+    got, st = _np(o).reshape(N, L, H, K), _np(state)
+    o_ref = np.asarray(o_ref).reshape(N, L, H, K)
+    for n in range(N):
+        for h in range(H):
+            if nan[n, h]:
+                assert np.isnan(got[n, L - 1, h]).all() and np.isnan(st[n, h]).all()
+                continue
+            bad, worst = _out_close(got[n, :, h], o_ref[n, :, h])
+            assert bad == 0, f"row {n} head {h}: {bad} outputs off (max diff {worst})"
+            rel, mx = _state_err(st[n, h], st_ref[n, h])
+            assert rel <= STATE_TOL and mx <= STATE_TOL, f"row {n} head {h}: {rel:.2e} {mx:.2e}"
+    np.testing.assert_array_equal(st[N], _np(state0[N]))

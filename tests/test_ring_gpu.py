@@ -531,3 +531,34 @@ def test_ring_prefill_of_long_rows(W, G, lens, starts):
     assert lib().hsg_ring_pos_update(d[6].data_ptr(), S, W, d[7].data_ptr(), d[8].data_ptr(), d[9].data_ptr(), N,
                                      max(lens), None) == 0
     assert torch.equal(d[6].cpu(), want_pos)
+
+
+@pytest.mark.parametrize("N,Lb,Hkv,G,split_k", [(16, 1, 4, 4, True), (8, 1, 2, 16, True), (8, 3, 4, 4, False),
+                                                 (1, 33, 4, 4, False)])
+def test_every_gate_value(N, Lb, Hkv, G, split_k):
+    """The sigmoid of every bf16 gate, NaN and infinities included, on each path (fused decode, split decode, tiles whose
+    keys the waves split, groups of tiles). Queries are 0 and values 1, so each output is bf16(sigmoid(gate)) but for one
+    rounding (the fp32 sigmoid's error of about 2 ulp may cross a boundary); past 1 + e^-x = 2^128 it may be 0."""
+    from hs_guard.engine.kernels import ring_attention_v8
+    print(f"[ring] gates N={N} Lb={Lb} G={G}", flush=True)
+    D, W, per = 256, 64, N * Lb * Hkv * G * 256
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = x.repeat(-(-per // 65536) + 1)[:-(-65536 // per) * per]
+    gen = torch.Generator().manual_seed(1)
+    dev = torch.device("cuda:0")
+    ring = [torch.randn(N, Hkv, W + 1, D, generator=gen).to(torch.bfloat16).to(dev) for _ in range(2)]
+    new_k = torch.randn(N, Hkv, Lb, D, generator=gen).to(torch.bfloat16).to(dev)
+    pos = torch.full((N, W + 1), -1, dtype=torch.long, device=dev)
+    args = (pos, torch.arange(N, device=dev), torch.zeros(N, dtype=torch.long, device=dev),
+            torch.full((N,), Lb, device=dev), D ** -0.5, W, False)
+    q = torch.zeros(N, Hkv, G * Lb, D, dtype=torch.bfloat16, device=dev)
+    value = torch.ones(N, Lb, Hkv * D, dtype=torch.bfloat16, device=dev)
+    for part in x.view(-1, per):
+        gate = torch.zeros(N, Lb, Hkv * G, 2, D, dtype=torch.bfloat16)
+        gate[..., 1, :] = part.view(N, Lb, Hkv * G, D)
+        out = ring_attention_v8(q, *ring, new_k, value, gate.view(N, Lb, -1).to(dev), *args, split_k=split_k).cpu().view(-1)
+        assert torch.equal(out.isnan(), part.isnan())
+        got, gd = out.double(), part.double()
+        ref = torch.sigmoid(gd)
+        live = ~part.isnan()
+        assert bool(((got - ref).abs() <= 2.0 ** -8 * ref + 1e-35)[live].all())
