@@ -420,7 +420,7 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
       for (int ks = 0; ks < D / 32; ++ks) ka[kt][ks] = *reinterpret_cast<const u32x4*>(src + 32 * ks);
     }
   };
-  // V: load u covers rows 2 u, 2 u + 1 whole (a key past the last valid one repeats it; its probability is zero)
+  // V: load u covers rows 2 u, 2 u + 1 whole (a key past the last valid one repeats it; it is zeroed when staged)
   auto load_values = [&](int i, u32x4 (&va)[KV_LOADS]) __attribute__((always_inline)) {
     int64_t st;
     int last;
@@ -506,8 +506,15 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
     for (int t = 0; t < D / 16; ++t) O[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = FIRST; i < SLOTS; ++i) {
-      // V of block i from registers into LDS, the next block's loads behind it
+      // V of block i from registers into LDS, the next block's loads behind it. Rows past the row's last key are zeros
+      // there: their probability is zero, but 0 x an infinite value of that key would be NaN
       const int lv = lane_per_site(lane);
+      const int last = wave + NW * i < RB ? KB - 1 : len - 1 - (cb0 + wave + NW * i - RB) * KB;
+      if ((seen >> i & 1u) && last < KB - 1) {
+#pragma unroll
+        for (int u = 0; u < KV_LOADS; ++u)
+          if (2 * u + (lv >> 5) > last) va[u] = (u32x4){0u, 0u, 0u, 0u};
+      }
 #pragma unroll
       for (int u = 0; u < KV_LOADS; ++u)
         *reinterpret_cast<u32x4*>(vlds + piece_at(2 * u + (lv >> 5), lv & 31)) = va[u];

@@ -562,3 +562,39 @@ def test_every_gate_value(N, Lb, Hkv, G, split_k):
         ref = torch.sigmoid(gd)
         live = ~part.isnan()
         assert bool(((got - ref).abs() <= 2.0 ** -8 * ref + 1e-35)[live].all())
+
+
+@pytest.mark.parametrize("G,Hkv,lens,starts", [(4, 2, [1, 3, 17, 33], [0, 200, 5, 64]), (1, 2, [1, 9, 40, 64], [70, 0, 3, 200]),
+                                               (16, 1, [1, 2, 5, 31], [64, 0, 129, 1])])
+def test_infinite_value_of_the_last_key(G, Hkv, lens, starts):
+    """An infinity among the values of a row's last key reaches the last step's output as that infinity (keys past the
+    row's end weigh nothing, and add no 0 x inf), and no other dim of it. The row's end falls in a block of 32 keys that a
+    lone tile takes (rows of up to 16 / G steps, or a last tile) or a group of tiles."""
+    from hs_guard.engine.kernels import ring_attention_v8
+    print(f"[ring] infinite last value G={G}", flush=True)
+    gen = torch.Generator().manual_seed(80 + G)
+    N, D, W, Lb = len(lens), 256, 64, max(lens)
+    q = torch.randn(N, Hkv, G * Lb, D, generator=gen).to(torch.bfloat16)
+    ring_k, ring_v = (torch.randn(N, Hkv, W + 1, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    new_k = torch.randn(N, Hkv, Lb, D, generator=gen).to(torch.bfloat16)
+    value = torch.randn(N, Lb, Hkv, D, generator=gen).to(torch.bfloat16)
+    gate = torch.randn(N, Lb, Hkv * G * 2 * D, generator=gen).to(torch.bfloat16)
+    slots, starts, lens_t = torch.arange(N), torch.tensor(starts), torch.tensor(lens)
+    ring_pos = torch.full((N, W + 1), -1, dtype=torch.long)
+    for s, st in enumerate(starts.tolist()):
+        for p_ in range(max(0, st - W), st):
+            ring_pos[s, p_ % W] = p_
+    ref, _, _, _ = oring.ring_attention_v8(_np(q), _np(ring_k), _np(ring_v), _np(new_k), _np(value.reshape(N, Lb, -1)),
+                                           _np(gate), ring_pos.numpy(), slots.numpy(), starts.numpy(), lens_t.numpy(),
+                                           D ** -0.5, W, False)
+    for n, k in enumerate(lens):
+        value[n, k - 1, :, 3], value[n, k - 1, :, 250] = float("inf"), -float("inf")
+    dev = torch.device("cuda:0")
+    out = ring_attention_v8(q.to(dev), ring_k.to(dev), ring_v.to(dev), new_k.to(dev), value.reshape(N, Lb, -1).to(dev),
+                            gate.to(dev), ring_pos.to(dev), slots.to(dev), starts.to(dev), lens_t.to(dev), D ** -0.5, W,
+                            False, split_k=False)
+    got, ref = _np(out).reshape(N, Lb, Hkv * G, D), np.asarray(ref).reshape(N, Lb, Hkv * G, D)
+    rest = [d for d in range(D) if d not in (3, 250)]
+    for n, k in enumerate(lens):
+        assert (got[n, k - 1, :, 3] == np.inf).all() and (got[n, k - 1, :, 250] == -np.inf).all(), f"row {n}"
+        _check(got[n, k - 1][:, rest], ref[n, k - 1][:, rest])
