@@ -63,6 +63,8 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* hidden, const ui
 // write the row's last 3 raw rows back, so no other block reads or writes it. The SiLU
 // and the 4 bytes per value bound it about equally: one 8,000-token row of 6,144 channels 40.6 us (4.84 TB/s; 54.8 as
 // 64-token segments of one channel per thread, 49.5 with expf and an IEEE divide), one of 311 tokens 6.3 us (12.0).
+// WALK (out is qkv): a thread takes its channels through the whole row, reading each raw value once, before its output
+// takes the place, and keeping the last window in registers.
 // ---------------------------------------------------------------------------------------------------
 constexpr int KS = 4;
 constexpr int CONV_TB = 16;
@@ -91,7 +93,7 @@ __device__ __forceinline__ void store_ch(uint16_t* p, const ChannelVec<VEC>& v) 
   else *p = v.x[0];
 }
 
-template <int VEC>
+template <int VEC, bool WALK>
 __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int64_t qkv_stride, uint16_t* pool,
                                                         int64_t pool_rows, const uint16_t* weight,
                                                         const int64_t* slots, const int64_t* lens,
@@ -108,7 +110,7 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int
   if (padded && len > L) len = L;
   const int64_t steps = padded ? L : len;
   const int64_t tok0 = padded ? (int64_t)n * L : offsets[n];
-  if ((int64_t)blockIdx.z * CONV_TB >= steps) return;
+  if (WALK ? steps == 0 : (int64_t)blockIdx.z * CONV_TB >= steps) return;
   float w[VEC][KS];
 #pragma unroll
   for (int v = 0; v < VEC; ++v)
@@ -117,36 +119,31 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int
   const uint16_t* const row = qkv + tok0 * qkv_stride + c;
   const bool history = pool && slot_ok;
   uint16_t* const prow = history ? pool + slot * (KS - 1) * (int64_t)C + c : nullptr;
-  ChannelVec<VEC> e[KS - 1], first[KS - 1];
-  for (int64_t t0 = (int64_t)blockIdx.z * CONV_TB; t0 < steps; t0 += (int64_t)gridDim.z * CONV_TB) {
+  ChannelVec<VEC> e[KS - 1], keep[KS - 1];   // the window; WALK: that after the last real token, else that before the first
+  auto step = [&](int64_t t, ChannelVec<VEC> x) __attribute__((always_inline)) {
+    ChannelVec<VEC> y;
 #pragma unroll
-    for (int i = 0; i < KS - 1; ++i) {
-      if (t0 > 0) e[i] = load_ch<VEC>(row + (t0 + i - (KS - 1)) * qkv_stride);
-      else if (history) e[i] = load_ch<VEC>(prow + i * (int64_t)C);
-      else e[i] = ChannelVec<VEC>{};
-      if (t0 == 0) first[i] = e[i];
+    for (int v = 0; v < VEC; ++v) {
+      float acc = 0.f;
+      acc = fmaf(w[v][0], bf2f(e[0].x[v]), acc);
+      acc = fmaf(w[v][1], bf2f(e[1].x[v]), acc);
+      acc = fmaf(w[v][2], bf2f(e[2].x[v]), acc);
+      acc = fmaf(w[v][3], bf2f(x.x[v]), acc);
+      y.x[v] = f2bf(siluf_(rbf(acc)));
     }
-    auto step = [&](int64_t t, ChannelVec<VEC> x) {
-      ChannelVec<VEC> y;
+    store_ch<VEC>(out + (tok0 + t) * out_stride + c, y);
+    e[0] = e[1];
+    e[1] = e[2];
+    e[2] = x;
+    if (WALK && t == len - 1) {
 #pragma unroll
-      for (int v = 0; v < VEC; ++v) {
-        float acc = 0.f;
-        acc = fmaf(w[v][0], bf2f(e[0].x[v]), acc);
-        acc = fmaf(w[v][1], bf2f(e[1].x[v]), acc);
-        acc = fmaf(w[v][2], bf2f(e[2].x[v]), acc);
-        acc = fmaf(w[v][3], bf2f(x.x[v]), acc);
-        y.x[v] = f2bf(siluf_(rbf(acc)));
-      }
-      store_ch<VEC>(out + (tok0 + t) * out_stride + c, y);
-      e[0] = e[1];
-      e[1] = e[2];
-      e[2] = x;
-    };
-    // Whole batches of TB tokens load together (one memory round trip per batch instead of per token); the
-    // remainder, which is all of a single-token row, goes one load at a time.
+      for (int i = 0; i < KS - 1; ++i) keep[i] = e[i];
+    }
+  };
+  // Whole batches of TB tokens load together (one memory round trip per batch instead of per token); the
+  // remainder, which is all of a single-token row, goes one load at a time.
+  auto run = [&](int64_t t, int64_t t1) __attribute__((always_inline)) {
     constexpr int TB = 8;
-    const int64_t t1 = min(t0 + CONV_TB, steps);
-    int64_t t = t0;
     for (; t + TB <= t1; t += TB) {
       ChannelVec<VEC> xs[TB];
 #pragma unroll
@@ -155,14 +152,34 @@ __global__ __launch_bounds__(256) void conv_silu_kernel(const uint16_t* qkv, int
       for (int i = 0; i < TB; ++i) step(t + i, xs[i]);
     }
     for (; t < t1; ++t) step(t, load_ch<VEC>(row + t * qkv_stride));
-  }
-  if (blockIdx.z == 0 && history && len > 0) {
-    ChannelVec<VEC> keep[KS - 1];   // the window after the last real token = ext[len .. len+2]
+  };
 #pragma unroll
-    for (int i = 0; i < KS - 1; ++i) {
-      const int64_t t = len - (KS - 1) + i;
-      if (t >= 0) keep[i] = load_ch<VEC>(row + t * qkv_stride);
-      else keep[i] = t == -3 ? first[0] : t == -2 ? first[1] : first[2];
+  for (int i = 0; i < KS - 1; ++i) {
+    keep[i] = history && (WALK || blockIdx.z == 0) ? load_ch<VEC>(prow + i * (int64_t)C) : ChannelVec<VEC>{};
+    e[i] = keep[i];
+  }
+  if constexpr (WALK) {
+    run(0, steps);
+  } else {
+    for (int64_t t0 = (int64_t)blockIdx.z * CONV_TB; t0 < steps; t0 += (int64_t)gridDim.z * CONV_TB) {
+      if (t0 > 0) {
+#pragma unroll
+        for (int i = 0; i < KS - 1; ++i) e[i] = load_ch<VEC>(row + (t0 + i - (KS - 1)) * qkv_stride);
+      }
+      run(t0, min(t0 + CONV_TB, steps));
+    }
+  }
+  if ((WALK || blockIdx.z == 0) && history && len > 0) {
+    if constexpr (!WALK) {   // the window after the last real token = ext[len .. len+2]
+      ChannelVec<VEC> tail[KS - 1];
+#pragma unroll
+      for (int i = 0; i < KS - 1; ++i) {
+        const int64_t t = len - (KS - 1) + i;
+        if (t >= 0) tail[i] = load_ch<VEC>(row + t * qkv_stride);
+        else tail[i] = t == -3 ? keep[0] : t == -2 ? keep[1] : keep[2];
+      }
+#pragma unroll
+      for (int i = 0; i < KS - 1; ++i) keep[i] = tail[i];
     }
 #pragma unroll
     for (int i = 0; i < KS - 1; ++i) store_ch<VEC>(prow + i * (int64_t)C, keep[i]);
@@ -431,8 +448,9 @@ extern "C" int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* p
   if (!qkv || !weight || (pool && !slots) || !lens || !out || (!offsets && L <= 0)) return HSG_ERR_ARG;
   const bool pairs = channels % 2 == 0 && qkv_stride % 2 == 0 && out_stride % 2 == 0 && aligned(qkv, 4) &&
                      aligned(out, 4) && (!pool || aligned(pool, 4));
+  const bool in_place = out == qkv;   // (in parallel, a block could read a neighbour's outputs)
   // token blocks of a row in parallel, up to the grid's z limit (a row with more walks them)
-  const int blocks = L > 0 ? min((L - 1) / CONV_TB + 1, 65535) : 1;
+  const int blocks = L > 0 && !in_place ? min((L - 1) / CONV_TB + 1, 65535) : 1;
   const int cols = pairs ? channels / 2 : channels;
   const dim3 grid((cols + 255) / 256, n_rows, blocks);
   const auto launch = [&](auto kernel) {
@@ -441,8 +459,13 @@ extern "C" int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* p
                        static_cast<const uint16_t*>(weight), slots, lens, offsets, L, channels,
                        static_cast<uint16_t*>(out), out_stride);
   };
-  if (pairs) launch(conv_silu_kernel<2>);
-  else launch(conv_silu_kernel<1>);
+  if (in_place) {
+    if (pairs) launch(conv_silu_kernel<2, true>);
+    else launch(conv_silu_kernel<1, true>);
+  } else {
+    if (pairs) launch(conv_silu_kernel<2, false>);
+    else launch(conv_silu_kernel<1, false>);
+  }
   return launch_status();
 }
 

@@ -330,6 +330,7 @@ int hsg_gated_rmsnorm(const void* x, int64_t x_stride, const void* z, int64_t z_
  *   out [tokens, out_stride] bf16. Padded layout computes all L positions of every row like the reference. Packed
  *   layout: rows of any length; L (0: unknown) is their usual largest length, by which a row's tokens are spread over
  *   workgroups. pool NULL: rows start from a zero history, and none is kept (slots is not read).
+ *   out may be qkv itself with the same stride; otherwise the two must not overlap.
  * Supported: kernel_size == 4.
  */
 int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* pool, int64_t pool_rows, const void* weight,

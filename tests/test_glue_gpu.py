@@ -280,6 +280,31 @@ def test_conv_token_blocks(lens, L, C, history):
         np.testing.assert_array_equal(_np(pool_d), ref_pool)
 
 
+@pytest.mark.parametrize("packed,lens,L,C", [(True, [40, 1, 16, 17, 0, 2], 40, 6144), (True, [33, 70], 0, 258),
+                                             (True, [19, 3], 19, 77), (False, [21, 2, 0, 9, 21], 21, 512)])
+def test_conv_in_place(packed, lens, L, C):
+    """hsg_conv_silu_update with out = qkv: the same outputs and history, bit for bit, as into another buffer."""
+    from hs_guard._lib import lib
+    print(f"[glue] conv in place packed={packed} {lens} C={C}", flush=True)
+    gen = torch.Generator().manual_seed(8)
+    N, S = len(lens), len(lens) + 1
+    lens_t, slots = torch.tensor(lens), torch.randperm(S, generator=gen)[:N]
+    offs = torch.cumsum(lens_t, 0) - lens_t
+    T = int(lens_t.sum()) if packed else N * L
+    qkv, pool, w = (torch.randn(*s, generator=gen).to(torch.bfloat16) for s in ((T, C + 6), (S, 3, C), (C, 4)))
+    w_d, sl_d, ln_d, of_d = (t.to(DEV) for t in (w, slots, lens_t, offs))
+    got = []
+    for same in (False, True):
+        q_d, p_d = qkv.to(DEV), pool.to(DEV)
+        out = q_d if same else q_d.clone()
+        assert lib().hsg_conv_silu_update(q_d.data_ptr(), C + 6, p_d.data_ptr(), S, w_d.data_ptr(), 4, sl_d.data_ptr(),
+                                          ln_d.data_ptr(), of_d.data_ptr() if packed else None, N, L, C, out.data_ptr(),
+                                          C + 6, _stream()) == 0
+        got.append((out.cpu(), p_d.cpu()))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    assert not torch.equal(got[1][0][:, :C], qkv[:, :C]) and torch.equal(got[1][0][:, C:], qkv[:, C:])
+
+
 def test_silu_of_every_bf16():
     """SiLU of all 65,536 bf16 values (silu_mul with up = 1): the float64 value correctly rounded down to x = -88.5 (its
     fp32 error, about 2 ulp, never crosses a bf16 rounding boundary there), past which 1 + e^-x leaves fp32's range and
