@@ -63,11 +63,15 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(uint16_t* hidden, const ui
 // write the row's last 3 raw rows back, so no other block reads or writes it. The SiLU
 // and the 4 bytes per value bound it about equally: one 8,000-token row of 6,144 channels 40.6 us (4.84 TB/s; 54.8 as
 // 64-token segments of one channel per thread, 49.5 with expf and an IEEE divide), one of 311 tokens 6.3 us (12.0).
-// WALK (out is qkv): a thread takes its channels through the whole row, reading each raw value once, before its output
-// takes the place, and keeping the last window in registers.
+// WALK (one workgroup a row and column block): a thread takes its channels through the whole row, reading each raw value
+// once, so that its output may take the value's place, and keeping the last window in registers.
 // ---------------------------------------------------------------------------------------------------
 constexpr int KS = 4;
 constexpr int CONV_TB = 16;
+// Workgroups up to which a row's blocks are spread. 352 rows of one token 7.0 us as one workgroup a row (10.9 in blocks);
+// rows of 1 to 64 tokens, 352 of them: 13.7 (19.9 at 4 blocks a row); a stated length of 22,528 for rows of 4 tokens cost
+// 1.8 ms of empty workgroups. 16 rows of 8,000 tokens take 620 us at 500 blocks a row and 657 at the 42 of this rule.
+constexpr int CONV_GRID = 8192;
 
 template <int VEC>
 struct ChannelVec {
@@ -448,18 +452,20 @@ extern "C" int hsg_conv_silu_update(const void* qkv, int64_t qkv_stride, void* p
   if (!qkv || !weight || (pool && !slots) || !lens || !out || (!offsets && L <= 0)) return HSG_ERR_ARG;
   const bool pairs = channels % 2 == 0 && qkv_stride % 2 == 0 && out_stride % 2 == 0 && aligned(qkv, 4) &&
                      aligned(out, 4) && (!pool || aligned(pool, 4));
-  const bool in_place = out == qkv;   // (in parallel, a block could read a neighbour's outputs)
-  // token blocks of a row in parallel, up to the grid's z limit (a row with more walks them)
-  const int blocks = L > 0 && !in_place ? min((L - 1) / CONV_TB + 1, 65535) : 1;
-  const int cols = pairs ? channels / 2 : channels;
-  const dim3 grid((cols + 255) / 256, n_rows, blocks);
+  const int cols = ((pairs ? channels / 2 : channels) + 255) / 256;
+  // Token blocks of a row in parallel (rows of unknown length: those of 64 tokens), as far as the column blocks of all rows
+  // leave the chip short of workgroups; a row with more blocks walks them. In place, a block could read a neighbour's
+  // outputs.
+  const int64_t want = ((L > 0 ? L : 64) - 1) / CONV_TB + 1, room = CONV_GRID / ((int64_t)cols * n_rows);
+  const int blocks = out == qkv ? 1 : (int)(want < room ? want : room > 1 ? room : 1);
+  const dim3 grid(cols, n_rows, blocks);
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, reinterpret_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(qkv), qkv_stride, static_cast<uint16_t*>(pool), pool_rows,
                        static_cast<const uint16_t*>(weight), slots, lens, offsets, L, channels,
                        static_cast<uint16_t*>(out), out_stride);
   };
-  if (in_place) {
+  if (blocks == 1) {
     if (pairs) launch(conv_silu_kernel<2, true>);
     else launch(conv_silu_kernel<1, true>);
   } else {

@@ -305,6 +305,34 @@ def test_conv_in_place(packed, lens, L, C):
     assert not torch.equal(got[1][0][:, :C], qkv[:, :C]) and torch.equal(got[1][0][:, C:], qkv[:, C:])
 
 
+@pytest.mark.parametrize("lens,C", [([200, 1, 65, 0, 16], 6144), ([3, 64, 1, 17] * 176, 6144), ([1, 2, 3] * 120, 6145)])
+def test_conv_grid(lens, C):
+    """hsg_conv_silu_update at every stated row length (0: unknown; below, at and far above the rows') and row count, spread
+    over workgroups or walked by one: the same outputs and history, bit for bit."""
+    from hs_guard._lib import lib
+    print(f"[glue] conv grid {len(lens)} rows C={C}", flush=True)
+    gen = torch.Generator().manual_seed(9)
+    N, lens_t = len(lens), torch.tensor(lens)
+    offs = torch.cumsum(lens_t, 0) - lens_t
+    T = int(lens_t.sum())
+    qkv, pool, w = (torch.randn(*s, generator=gen).to(torch.bfloat16).to(DEV) for s in ((T, C), (N, 3, C), (C, 4)))
+    sl_d, ln_d, of_d = torch.randperm(N, generator=gen).to(DEV), lens_t.to(DEV), offs.to(DEV)
+    got = []
+    for L in (max(lens), 0, 1, 40, 1 << 30):
+        p_d, out = pool.clone(), torch.zeros_like(qkv)
+        assert lib().hsg_conv_silu_update(qkv.data_ptr(), C, p_d.data_ptr(), N, w.data_ptr(), 4, sl_d.data_ptr(),
+                                          ln_d.data_ptr(), of_d.data_ptr(), N, L, C, out.data_ptr(), C, _stream()) == 0
+        got.append((out, p_d))
+    assert all(torch.equal(got[0][0], o) and torch.equal(got[0][1], p) for o, p in got[1:])
+    n = max(range(N), key=lambda i: lens[i])
+    x = qkv[int(offs[n]):int(offs[n]) + lens[n]]
+    ref, ref_pool = oglue.conv_silu_update(_np(x)[None], _np(pool), _np(w), np.array([int(sl_d[n])]), np.array([lens[n]]))
+    # the bound of test_conv_silu_update
+    atol = 4 * 2.0 ** -24 * float(w.abs().max()) * float(max(qkv.abs().max(), pool.abs().max())) * 4
+    _close(_np(got[0][0][int(offs[n]):int(offs[n]) + lens[n]]), ref[0], "conv row", atol=atol, ulps=2)
+    np.testing.assert_array_equal(_np(got[0][1][sl_d[n]]), ref_pool[int(sl_d[n])])
+
+
 def test_silu_of_every_bf16():
     """SiLU of all 65,536 bf16 values (silu_mul with up = 1): the float64 value correctly rounded down to x = -88.5 (its
     fp32 error, about 2 ulp, never crosses a bf16 rounding boundary there), past which 1 + e^-x leaves fp32's range and
