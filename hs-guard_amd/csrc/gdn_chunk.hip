@@ -368,7 +368,7 @@ __global__ __launch_bounds__(256, 4) void gdn_chunk_prep_kernel(const ChunkParam
       const float A = expf(bf2f(A_raw));
       const float x = bf2f(pa) + bf2f(dt_raw);
       g_s[st_t] = ok ? -A * (x > 20.0f ? x : logf(1.0f + expf(x))) : 0.f;
-      b_s[st_t] = ok ? sigmoidf_(bf2f(pb)) : 0.f;
+      b_s[st_t] = ok ? sigmoid_f32(bf2f(pb)) : 0.f;
     }
   }
   lds_barrier();

@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void gdn_step_kernel(const GdnParams p) {
       const float x = bf2f((uint16_t)pa) + bf2f((uint16_t)dh);
       const float g = -expf(bf2f((uint16_t)al)) * (x > 20.0f ? x : logf(1.0f + expf(x)));
       sdec_[tid] = expf(g);
-      sbe_[tid] = sigmoidf_(bf2f(pb));
+      sbe_[tid] = sigmoid_f32(bf2f(pb));
     }
   };
   auto stage = [&](int nt, bool first) __attribute__((always_inline)) {
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(256) void gdn_step_kernel(const GdnParams p) {
       const float x = bf2f((uint16_t)pa) + bf2f((uint16_t)dh);
       const float g = -expf(bf2f((uint16_t)al)) * (x > 20.0f ? x : logf(1.0f + expf(x)));
       sdec_[tid] = expf(g);
-      sbe_[tid] = sigmoidf_(bf2f(pb));
+      sbe_[tid] = sigmoid_f32(bf2f(pb));
     }
   };
   // gated RMSNorm of the burst's outputs (so_, bf16-rounded o), stored to `out`: 32 threads per token, 4 value

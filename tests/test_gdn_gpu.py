@@ -328,3 +328,27 @@ def test_every_beta(route, L):
             rel, mx = _state_err(st[n, h], st_ref[n, h])
             assert rel <= STATE_TOL and mx <= STATE_TOL, f"row {n} head {h}: {rel:.2e} {mx:.2e}"
     np.testing.assert_array_equal(st[N], _np(state0[N]))
+
+
+def test_beta_rounding():
+    """A state written with beta alone (zero state, k = e_0, v = 1: S[0] = k beta, k = 1 / sqrt(1 + 1e-6)) over every bf16 b
+    of 2^-4 <= |b| < 8 against float64: its rms error is that of 1 / (1 + exp(-b)) in fp32 on the CPU (5.48e-8, five
+    roundings), but for the device's exp, up to an ulp off where the CPU's is not: 4 %."""
+    from hs_guard.engine.kernels import gdn_slot_v8
+    K, H = 128, 16
+    b = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    b = b[(b.float().abs() >= 2.0 ** -4) & (b.float().abs() < 8)]
+    b = b.view(-1, 1, H)
+    N = len(b)
+    packed = torch.zeros(N, 1, 3 * H * K, dtype=torch.bfloat16)
+    packed[..., H * K:2 * H * K:K] = 1
+    packed[..., 2 * H * K:] = 1
+    dev = torch.device("cuda:0")
+    state, zero = torch.zeros(N + 1, H, K, K, device=dev), torch.zeros(H, dtype=torch.bfloat16, device=dev)
+    gdn_slot_v8(packed.to(dev), H * K, H, K, H, K, torch.zeros_like(b, device=dev), b.to(dev), zero, zero, state,
+                torch.arange(N, device=dev), torch.ones(N, dtype=torch.long, device=dev))
+    exact = torch.sigmoid(b[:, 0].double()) / (1 + 1e-6) ** 0.5
+    fp32 = 1 / (1 + torch.exp(-b[:, 0].float())) * (1 / torch.sqrt(torch.tensor(1 + 1e-6)))
+    rms, bar = (float(((x.double() / exact - 1) ** 2).mean().sqrt()) for x in (state[:N, :, 0, 0].cpu(), fp32))
+    print(f"[gdn] beta rms relative error {rms:.3e}, fp32 on the CPU {bar:.3e}", flush=True)
+    assert rms <= 1.04 * bar
