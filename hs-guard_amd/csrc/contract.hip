@@ -7,7 +7,8 @@
 //
 // Every kernel here is element-wise once the per-row variance is given, so each thread owns VEC consecutive
 // elements of one row: the most of 8 (16-byte bf16 loads), 4 and 1 that the row width and every pointer and stride
-// allow, so rows of any width and count work. The vector forms need a flat index of 31 bits (a cheap division).
+// allow, so rows of any width and count work. Flat indices take 32 bits up to 2^31 elements (a cheap division), 64 beyond:
+// SiLU-mul of 2^31 elements 1,345 us just below and above (4,350 with one element per thread).
 // They move each byte once and are bound by that and, below ~10 MB, by the launch. At 1,473 tokens norm_rope over 16
 // query and 4 key heads (two launches) takes 14.9 us, 38.5 with one element per thread; the others, cache-resident at
 // that size, gain up to a fifth from 8 elements over 4 (rms_finish 4.2 -> 3.5 us) or stay (silu_mul 8.2).
@@ -69,24 +70,20 @@ __device__ __forceinline__ void load_f32(const float* p, float* x) {
   }
 }
 
-// flat indices: 32-bit in the vector forms
-template <int VEC>
-using index_t = std::conditional_t<VEC == 1, int64_t, uint32_t>;
-
 // the thread's first element, n when it has none
-template <int VEC>
-__device__ __forceinline__ index_t<VEC> first_element(int64_t n) {
-  const index_t<VEC> i = ((index_t<VEC>)blockIdx.x * CT_THREADS + threadIdx.x) * VEC;
-  return i < (index_t<VEC>)n ? i : (index_t<VEC>)n;
+template <int VEC, typename I>
+__device__ __forceinline__ I first_element(int64_t n) {
+  const I i = ((I)blockIdx.x * CT_THREADS + threadIdx.x) * VEC;
+  return i < (I)n ? i : (I)n;
 }
 
 // add_square (src/hs_guard/engine/fused_kernels.py:30-52): h = bf16(res + mix) with a plain fp32 add (no
 // contraction), stored when mix is given; sq = h^2 in fp32 (of res when mix is NULL).
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void add_square_kernel(const uint16_t* res, const uint16_t* mix,
                                                                 uint16_t* out, float* sq, int64_t n) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
   float h[VEC];
   load_bf<VEC>(res + i, h);
   if (mix) {
@@ -102,13 +99,13 @@ __global__ __launch_bounds__(CT_THREADS) void add_square_kernel(const uint16_t* 
 }
 
 // rms_finish (fused_kernels.py:56-72): out = bf16((x * rsqrt(var[row] + eps)) * w1[col]).
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void rms_finish_kernel(const uint16_t* x, const float* var, const float* w1,
                                                                 float eps, uint16_t* out, int64_t n, int width) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
-  const index_t<VEC> row = i / (index_t<VEC>)width;
-  const int col = (int)(i - row * (index_t<VEC>)width);
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
+  const I row = i / (I)width;
+  const int col = (int)(i - row * (I)width);
   float h[VEC], wv[VEC];
   load_bf<VEC>(x + i, h);
   load_f32<VEC>(w1 + col, wv);
@@ -119,11 +116,11 @@ __global__ __launch_bounds__(CT_THREADS) void rms_finish_kernel(const uint16_t* 
 }
 
 // silu_mul (fused_kernels.py:76-90): out = bf16(bf16(silu(gate)) * up) over two tensors of n elements.
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void silu_mul_pair_kernel(const uint16_t* gate, const uint16_t* up,
                                                                    uint16_t* out, int64_t n) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
   float g[VEC], u[VEC];
   load_bf<VEC>(gate + i, g);
   load_bf<VEC>(up + i, u);
@@ -133,14 +130,14 @@ __global__ __launch_bounds__(CT_THREADS) void silu_mul_pair_kernel(const uint16_
 }
 
 // gated_finish (fused_kernels.py:215-233): out = bf16(bf16(w[col] * bf16(x * rsqrt(var[row] + eps))) * silu(z)).
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void gated_finish_kernel(const uint16_t* x, const float* var,
                                                                   const uint16_t* w, const uint16_t* z, float eps,
                                                                   uint16_t* out, int64_t n, int width) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
-  const index_t<VEC> row = i / (index_t<VEC>)width;
-  const int col = (int)(i - row * (index_t<VEC>)width);
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
+  const I row = i / (I)width;
+  const int col = (int)(i - row * (I)width);
   float h[VEC], g[VEC], wv[VEC];
   load_bf<VEC>(x + i, h);
   load_bf<VEC>(z + i, g);
@@ -153,15 +150,15 @@ __global__ __launch_bounds__(CT_THREADS) void gated_finish_kernel(const uint16_t
 
 // square_rows (fused_kernels.py:237-249): sq[r, c] = x^2 of head r % heads of token r / heads, read from the
 // strided projection rows; sq is [tokens * heads, dim] fp32.
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void square_rows_kernel(const uint16_t* src, float* sq, int heads,
                                                                  int64_t row_stride, int64_t head_stride, int dim,
                                                                  int64_t n) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
-  const index_t<VEC> r = i / (index_t<VEC>)dim;
-  const int c = (int)(i - r * (index_t<VEC>)dim);
-  const int64_t token = r / (index_t<VEC>)heads;
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
+  const I r = i / (I)dim;
+  const int c = (int)(i - r * (I)dim);
+  const int64_t token = r / (I)heads;
   const int j = (int)(r - token * heads);
   float x[VEC];
   load_bf<VEC>(src + token * row_stride + j * head_stride + c, x);
@@ -177,19 +174,19 @@ __global__ __launch_bounds__(CT_THREADS) void square_rows_kernel(const uint16_t*
 // written at out + n*out_n + (j / groups)*out_h + ((j % groups)*lb + l)*out_row + d for head j of token n*lb + l.
 // A thread's VEC elements lie in one half of the rotary dims (or beyond them); their partners are a second (cached) load
 // of the same row.
-template <int VEC>
+template <int VEC, typename I>
 __global__ __launch_bounds__(CT_THREADS) void norm_rope_grouped_kernel(
     const uint16_t* src, const float* var, const float* w1, const uint16_t* cosv, const uint16_t* sinv, int rot,
     float eps, int heads, int lb, int groups, int64_t row_stride, int64_t head_stride, int dim, uint16_t* out,
     int64_t out_n, int64_t out_h, int64_t out_row, int64_t n) {
-  const index_t<VEC> i = first_element<VEC>(n);
-  if (i == (index_t<VEC>)n) return;
-  const index_t<VEC> r = i / (index_t<VEC>)dim;
-  const int d = (int)(i - r * (index_t<VEC>)dim);
-  const index_t<VEC> token = r / (index_t<VEC>)heads;
-  const int j = (int)(r - token * (index_t<VEC>)heads);
-  const index_t<VEC> nn = token / (index_t<VEC>)lb;
-  const int l = (int)(token - nn * (index_t<VEC>)lb);
+  const I i = first_element<VEC, I>(n);
+  if (i == (I)n) return;
+  const I r = i / (I)dim;
+  const int d = (int)(i - r * (I)dim);
+  const I token = r / (I)heads;
+  const int j = (int)(r - token * (I)heads);
+  const I nn = token / (I)lb;
+  const int l = (int)(token - nn * (I)lb);
   const int half = rot / 2;
   const int partner = d < half ? d + half : (d < rot ? d - half : d);
   const float rr = rsqrtf(var[r] + eps);
@@ -215,11 +212,10 @@ __global__ __launch_bounds__(CT_THREADS) void norm_rope_grouped_kernel(
   store_bf<VEC>(out + (int64_t)nn * out_n + (j / groups) * out_h + ((int64_t)(j % groups) * lb + l) * out_row + d, x);
 }
 
-// Elements per thread of a call over n elements in rows of `width`, given its bf16 and fp32 pointers and its strides: bf16
-// pieces of VEC elements and fp32 pieces of 4 are aligned to their size.
-int vec_of(int64_t n, int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32,
+// Elements per thread of a call in rows of `width`, given its bf16 and fp32 pointers and its strides: bf16 pieces of VEC
+// elements and fp32 pieces of 4 are aligned to their size.
+int vec_of(int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32,
            std::initializer_list<int64_t> strides = {}) {
-  if (n >= (1ll << 31)) return 1;
   for (const void* p : f32)
     if (p && !aligned(p, 16)) return 1;
   for (int vec : {8, 4}) {
@@ -231,13 +227,23 @@ int vec_of(int64_t n, int64_t width, std::initializer_list<const void*> bf, std:
   return 1;
 }
 
-// launch(vec constant, grid) for the chosen vector width
+// Elements per thread and the type of flat indices: 32 bits (a cheap division) up to 2^31 elements
+template <int VEC, typename I>
+struct Form {
+  static constexpr int vec = VEC;
+  using index = I;
+};
+
+// launch(form, grid) for the chosen vector width over n elements
 template <typename Launch>
 int launch_vec(int vec, int64_t n, Launch launch) {
-  const dim3 grid((unsigned)((n / vec + CT_THREADS - 1) / CT_THREADS));
-  if (vec == 8) launch(std::integral_constant<int, 8>{}, grid);
-  else if (vec == 4) launch(std::integral_constant<int, 4>{}, grid);
-  else launch(std::integral_constant<int, 1>{}, grid);
+  const int64_t blocks = (n / vec + CT_THREADS - 1) / CT_THREADS;
+  if (blocks >= (1 << 24)) return HSG_ERR_SHAPE;   // a launch holds less than 2^32 threads
+  const dim3 grid((unsigned)blocks);
+  const bool wide = n >= (1ll << 31);
+  if (vec == 8) wide ? launch(Form<8, int64_t>{}, grid) : launch(Form<8, uint32_t>{}, grid);
+  else if (vec == 4) wide ? launch(Form<4, int64_t>{}, grid) : launch(Form<4, uint32_t>{}, grid);
+  else launch(Form<1, int64_t>{}, grid);
   return launch_status();
 }
 
@@ -256,8 +262,9 @@ extern "C" int hsg_add_square(const void* residual, const void* mixed, void* out
   const auto* r = static_cast<const uint16_t*>(residual);
   const auto* m = static_cast<const uint16_t*>(mixed);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(n, width, {residual, mixed, out}, {sq}), n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(add_square_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, r, m, o, sq, n);
+  return launch_vec(vec_of(width, {residual, mixed, out}, {sq}), n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((add_square_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, r, m, o, sq, n);
   });
 }
 
@@ -270,8 +277,9 @@ extern "C" int hsg_rms_finish(const void* x, const float* var, const float* w1, 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* xi = static_cast<const uint16_t*>(x);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(n, width, {x, out}, {w1}), n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(rms_finish_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n, width);
+  return launch_vec(vec_of(width, {x, out}, {w1}), n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((rms_finish_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n, width);
   });
 }
 
@@ -283,8 +291,9 @@ extern "C" int hsg_silu_mul_pair(const void* gate, const void* up, void* out, in
   const auto* g = static_cast<const uint16_t*>(gate);
   const auto* u = static_cast<const uint16_t*>(up);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(n, n, {gate, up, out}, {}), n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(silu_mul_pair_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, g, u, o, n);
+  return launch_vec(vec_of(n, {gate, up, out}, {}), n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((silu_mul_pair_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, g, u, o, n);
   });
 }
 
@@ -299,8 +308,9 @@ extern "C" int hsg_gated_finish(const void* x, const float* var, const void* wei
   const auto* w = static_cast<const uint16_t*>(weight);
   const auto* zi = static_cast<const uint16_t*>(z);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(n, width, {x, weight, z, out}, {}), n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(gated_finish_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o, n, width);
+  return launch_vec(vec_of(width, {x, weight, z, out}, {}), n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((gated_finish_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o, n, width);
   });
 }
 
@@ -312,8 +322,9 @@ extern "C" int hsg_square_rows(const void* src, float* sq, int64_t tokens, int32
   const int64_t n = tokens * heads * dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* x = static_cast<const uint16_t*>(src);
-  return launch_vec(vec_of(n, dim, {src}, {sq}, {row_stride, head_stride}), n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(square_rows_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s, x, sq, heads, row_stride, head_stride, dim, n);
+  return launch_vec(vec_of(dim, {src}, {sq}, {row_stride, head_stride}), n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((square_rows_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, x, sq, heads, row_stride, head_stride, dim, n);
   });
 }
 
@@ -328,9 +339,10 @@ extern "C" int hsg_norm_rope_grouped(const void* src, const float* var, const fl
   if (!src || !var || !w1 || !cos || !sin || !out) return HSG_ERR_ARG;
   const int64_t n = (int64_t)n_rows * lb * heads * dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return launch_vec(vec_of(n, dim, {src, cos, sin, out}, {w1}, {rot / 2, row_stride, head_stride, out_n, out_h, out_row}),
-                    n, [&](auto vec, dim3 grid) {
-    hipLaunchKernelGGL(norm_rope_grouped_kernel<vec.value>, grid, dim3(CT_THREADS), 0, s,
+  return launch_vec(vec_of(dim, {src, cos, sin, out}, {w1}, {rot / 2, row_stride, head_stride, out_n, out_h, out_row}),
+                    n, [&](auto form, dim3 grid) {
+    using F = decltype(form);
+    hipLaunchKernelGGL((norm_rope_grouped_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s,
                        static_cast<const uint16_t*>(src), var, w1, static_cast<const uint16_t*>(cos),
                        static_cast<const uint16_t*>(sin), rot, eps, heads, lb, groups, row_stride, head_stride, dim,
                        static_cast<uint16_t*>(out), out_n, out_h, out_row, n);

@@ -393,3 +393,31 @@ def test_norm_rope_vector_widths(dim, rot, shift):
     ref = oglue.norm_rope_given(x, var[..., None], w1, 1e-6, cos, sin)
     ref = ref.reshape(n, lb, heads // groups, groups, dim).transpose(0, 2, 3, 1, 4).reshape(n, heads // groups, groups * lb, dim)
     _close(_np(got), ref, "norm_rope")
+
+
+@pytest.mark.parametrize("rows,width", [(2049, 1 << 20), (4097, 1 << 20), (4097, (1 << 20) + 4)])
+def test_beyond_32_bit_indices(rows, width):
+    """The element-wise kernels past 2^31 and 2^32 elements, 8 and 4 elements per thread: rows on both sides of those bounds
+    and the last one are bitwise a call on the row alone."""
+    from hs_guard.engine.kernels import add_square, gated_finish, rms_finish, silu_mul, square_rows
+    print(f"[contract] {rows} x {width}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    row = torch.randn(width, generator=gen, device=DEV).to(torch.bfloat16)
+    x = torch.empty(rows, width, dtype=torch.bfloat16, device=DEV)
+    scale = 1 + torch.arange(rows, device=DEV) % 7
+    for r in range(rows):                      # every row its own
+        torch.mul(row, scale[r].to(torch.bfloat16), out=x[r])
+    w1 = torch.rand(width, generator=gen, device=DEV) + 0.5
+    w = w1.to(torch.bfloat16)
+    var = torch.rand(rows, 1, generator=gen, device=DEV) + 0.5
+    at = [r for r in (0, 2047, 2048, 4095, 4096, rows - 1) if r < rows]
+    for name, f in (("rms_finish", lambda t, v: rms_finish(t, v, w1, 1e-6)), ("silu_mul", lambda t, v: silu_mul(t, t)),
+                    ("gated_finish", lambda t, v: gated_finish(t, v, w, t, 1e-6)),
+                    ("add_square", lambda t, v: add_square(t, t)[0]), ("squares", lambda t, v: add_square(t)[1]),
+                    ("square_rows", lambda t, v: square_rows(t.view(-1), len(t), 1, width, width, width).view(t.shape))):
+        out = f(x, var)
+        for r in at:
+            assert torch.equal(out[r], f(x[r:r + 1].clone(), var[r:r + 1].clone())[0]), f"{name} row {r}"
+        out.fill_(float("nan"))                # the next call's output starts from this, not from the right values
+        del out
+    torch.cuda.empty_cache()
