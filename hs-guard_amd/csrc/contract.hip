@@ -56,14 +56,16 @@ __device__ __forceinline__ void store_f32(float* p, const float* x) {
   }
 }
 
+// (at any 4-byte address: a weight may start anywhere in a buffer)
 template <int VEC>
 __device__ __forceinline__ void load_f32(const float* p, float* x) {
   if constexpr (VEC == 1) {
     x[0] = p[0];
   } else {
+    typedef f32x4_n __attribute__((aligned(4))) f32x4_any;
 #pragma unroll
     for (int e = 0; e < VEC; e += 4) {
-      const f32x4_n v = *reinterpret_cast<const f32x4_n*>(p + e);
+      const f32x4_n v = *reinterpret_cast<const f32x4_any*>(p + e);
 #pragma unroll
       for (int k = 0; k < 4; ++k) x[e + k] = v[k];
     }
@@ -277,7 +279,7 @@ extern "C" int hsg_rms_finish(const void* x, const float* var, const float* w1, 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* xi = static_cast<const uint16_t*>(x);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(width, {x, out}, {w1}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(width, {x, out}, {}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((rms_finish_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n, width);
   });

@@ -421,3 +421,14 @@ def test_beyond_32_bit_indices(rows, width):
         out.fill_(float("nan"))                # the next call's output starts from this, not from the right values
         del out
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("width,shift", [(1024, 1), (1028, 2), (256, 3), (1024, 4), (10, 1)])
+def test_rms_finish_weight_at_any_address(width, shift):
+    """rms_finish with w1 at every 4-byte alignment: bitwise the result with an aligned copy."""
+    from hs_guard.engine.kernels import rms_finish
+    gen = torch.Generator().manual_seed(width + shift)
+    x = torch.randn(37, width, generator=gen).to(torch.bfloat16).to(DEV)
+    var = torch.rand(37, 1, generator=gen).to(DEV) + 0.5
+    buf = (torch.rand(width + shift, generator=gen) + 0.5).to(DEV)
+    assert torch.equal(rms_finish(x, var, buf[shift:], 1e-6), rms_finish(x, var, buf[shift:].clone(), 1e-6))
