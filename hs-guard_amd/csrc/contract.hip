@@ -214,9 +214,10 @@ __global__ __launch_bounds__(CT_THREADS) void norm_rope_grouped_kernel(
   store_bf<VEC>(out + (int64_t)nn * out_n + (j / groups) * out_h + ((int64_t)(j % groups) * lb + l) * out_row + d, x);
 }
 
-// Elements per thread of a call in rows of `width`, given its bf16 and fp32 pointers and its strides: bf16 pieces of VEC
-// elements and fp32 pieces of 4 are aligned to their size.
-int vec_of(int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32,
+// Elements per thread (8 at most, or 4) of a call in rows of `width`, given its bf16 and fp32 pointers and its strides: bf16
+// pieces of VEC elements and fp32 pieces of 4 are aligned to their size. 4 for the kernels that write fp32 squares: at 8 a
+// wave's 16-byte stores leave gaps that its second store fills (add_square of 8,000 x 4,096 60.2 us against 56.5).
+int vec_of(int most, int64_t width, std::initializer_list<const void*> bf, std::initializer_list<const void*> f32,
            std::initializer_list<int64_t> strides = {}) {
   for (const void* p : f32)
     if (p && !aligned(p, 16)) return 1;
@@ -224,7 +225,7 @@ int vec_of(int64_t width, std::initializer_list<const void*> bf, std::initialize
     bool ok = width % vec == 0;
     for (const void* p : bf) ok = ok && (!p || aligned(p, 2 * vec));
     for (int64_t s : strides) ok = ok && s % vec == 0;
-    if (ok) return vec;
+    if (ok && vec <= most) return vec;
   }
   return 1;
 }
@@ -264,7 +265,7 @@ extern "C" int hsg_add_square(const void* residual, const void* mixed, void* out
   const auto* r = static_cast<const uint16_t*>(residual);
   const auto* m = static_cast<const uint16_t*>(mixed);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(width, {residual, mixed, out}, {sq}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(4, width, {residual, mixed, out}, {sq}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((add_square_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, r, m, o, sq, n);
   });
@@ -279,7 +280,7 @@ extern "C" int hsg_rms_finish(const void* x, const float* var, const float* w1, 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* xi = static_cast<const uint16_t*>(x);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(width, {x, out}, {}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(8, width, {x, out}, {}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((rms_finish_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, xi, var, w1, eps, o, n, width);
   });
@@ -293,7 +294,7 @@ extern "C" int hsg_silu_mul_pair(const void* gate, const void* up, void* out, in
   const auto* g = static_cast<const uint16_t*>(gate);
   const auto* u = static_cast<const uint16_t*>(up);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(n, {gate, up, out}, {}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(8, n, {gate, up, out}, {}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((silu_mul_pair_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, g, u, o, n);
   });
@@ -310,7 +311,7 @@ extern "C" int hsg_gated_finish(const void* x, const float* var, const void* wei
   const auto* w = static_cast<const uint16_t*>(weight);
   const auto* zi = static_cast<const uint16_t*>(z);
   auto* o = static_cast<uint16_t*>(out);
-  return launch_vec(vec_of(width, {x, weight, z, out}, {}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(8, width, {x, weight, z, out}, {}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((gated_finish_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, xi, var, w, zi, eps, o, n, width);
   });
@@ -324,7 +325,7 @@ extern "C" int hsg_square_rows(const void* src, float* sq, int64_t tokens, int32
   const int64_t n = tokens * heads * dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const auto* x = static_cast<const uint16_t*>(src);
-  return launch_vec(vec_of(dim, {src}, {sq}, {row_stride, head_stride}), n, [&](auto form, dim3 grid) {
+  return launch_vec(vec_of(4, dim, {src}, {sq}, {row_stride, head_stride}), n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((square_rows_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s, x, sq, heads, row_stride, head_stride, dim, n);
   });
@@ -341,7 +342,7 @@ extern "C" int hsg_norm_rope_grouped(const void* src, const float* var, const fl
   if (!src || !var || !w1 || !cos || !sin || !out) return HSG_ERR_ARG;
   const int64_t n = (int64_t)n_rows * lb * heads * dim;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  return launch_vec(vec_of(dim, {src, cos, sin, out}, {w1}, {rot / 2, row_stride, head_stride, out_n, out_h, out_row}),
+  return launch_vec(vec_of(8, dim, {src, cos, sin, out}, {w1}, {rot / 2, row_stride, head_stride, out_n, out_h, out_row}),
                     n, [&](auto form, dim3 grid) {
     using F = decltype(form);
     hipLaunchKernelGGL((norm_rope_grouped_kernel<F::vec, typename F::index>), grid, dim3(CT_THREADS), 0, s,
