@@ -433,19 +433,20 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
   for (int e = tid; e < TQ * NW * SLOTS; e += NW * 64) (&bm_s[0][0])[e] = -INFINITY;
   lds_barrier();   // kp_s and the empty block maxima are in LDS
 
-  // ---- phase 1: scores of blocks FIRST .. SLOTS - 1 and their maxima; phase 2: probabilities and P.V ----
+  // ---- phase 1: scores of the blocks and their maxima; phase 2: probabilities and P.V ----
   float m_last = -INFINITY, m_fin = -INFINITY, l_run = 0.f;   // l_run: this lane's keys only
   f32x4 O[D / 16];
-  auto attend = [&](auto first) __attribute__((always_inline)) {
-    constexpr int FIRST = decltype(first)::value;
+  auto attend = [&](auto first, auto step) __attribute__((always_inline)) {   // blocks FIRST, FIRST + STEP, ...
+    constexpr int FIRST = decltype(first)::value, STEP = decltype(step)::value;
     float s[SLOTS][8];
     u32x4 va[KV_LOADS];
     {
       u32x4 ka[2][2][D / 32];
-      load_keys(FIRST, ka[FIRST & 1]);
+      load_keys(FIRST, ka[0]);
 #pragma unroll
-      for (int i = FIRST; i < SLOTS; ++i) {
-        if (i + 1 < SLOTS) load_keys(i + 1, ka[(i + 1) & 1]);
+      for (int i = FIRST; i < SLOTS; i += STEP) {
+        const int buf = (i - FIRST) / STEP & 1;
+        if (i + STEP < SLOTS) load_keys(i + STEP, ka[buf ^ 1]);
         else load_values(FIRST, va);
         if (seen >> i & 1u) {
           f32x4 S[2];
@@ -454,7 +455,7 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int ks = 0; ks < D / 32; ++ks)
-              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[i & 1][kt][ks]), qb[ks], acc, 0, 0, 0);
+              acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(ka[buf][kt][ks]), qb[ks], acc, 0, 0, 0);
             S[kt] = acc;
           }
           // scale and mask the lane's 8 keys 4 q4 + e and 16 + 4 q4 + e
@@ -505,7 +506,7 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
 #pragma unroll
     for (int t = 0; t < D / 16; ++t) O[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int i = FIRST; i < SLOTS; ++i) {
+    for (int i = FIRST; i < SLOTS; i += STEP) {
       // V of block i from registers into LDS, the next block's loads behind it. Rows past the row's last key are zeros
       // there: their probability is zero, but 0 x an infinite value of that key would be NaN
       const int lv = lane_per_site(lane);
@@ -518,7 +519,7 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
 #pragma unroll
       for (int u = 0; u < KV_LOADS; ++u)
         *reinterpret_cast<u32x4*>(vlds + piece_at(2 * u + (lv >> 5), lv & 31)) = va[u];
-      if (i + 1 < SLOTS) load_values(i + 1, va);
+      if (i + STEP < SLOTS) load_values(i + STEP, va);
       if (!(seen >> i & 1u)) continue;
       const float m = mb[i] == -INFINITY ? 0.f : mb[i];
       const float alpha = m_last == mb[i] ? 1.f : exp_fast(m_last - m);   // exp(-inf) = 0: nothing added so far
@@ -553,10 +554,14 @@ __device__ __forceinline__ void attend_tile(const RingParams& p, const Row& ro, 
       }
     }
   };
-  // a wave that sees none of its first SLOTS - 1 blocks (a row without history) skips their loads. The barrier count
-  // is the same either way.
-  if (seen & ((1u << (SLOTS - 1)) - 1)) attend(std::integral_constant<int, 0>{});
-  else attend(std::integral_constant<int, SLOTS - 1>{});
+  // A wave that sees none of its first SLOTS - 1 blocks (a row without history), or only its first and last (a history of up
+  // to NW blocks), skips the others' loads: 72 rows of 4 steps over 100 keys 26.0 -> 19.1 us. The barrier
+  // count is the same.
+  using Slot = std::integral_constant<int, 1>;
+  using Ends = std::integral_constant<int, SLOTS - 1>;
+  if (seen & ((1u << (SLOTS - 1)) - 2)) attend(std::integral_constant<int, 0>{}, Slot{});
+  else if (seen & 1u) attend(std::integral_constant<int, 0>{}, Ends{});
+  else attend(Ends{}, Slot{});
 
   // ---- combine the waves: each leaves its weighted O (lane-linear 16-byte pieces) in its own Vs and takes dims
   // 64 w + 16 t + 4 q4 + i (t < 4) of every row ----

@@ -598,3 +598,30 @@ def test_infinite_value_of_the_last_key(G, Hkv, lens, starts):
     for n, k in enumerate(lens):
         assert (got[n, k - 1, :, 3] == np.inf).all() and (got[n, k - 1, :, 250] == -np.inf).all(), f"row {n}"
         _check(got[n, k - 1][:, rest], ref[n, k - 1][:, rest])
+
+
+@pytest.mark.parametrize("G", [1, 4])
+def test_short_histories(G):
+    """Rows of one query tile over histories from 0 keys to past the first four blocks of 32, whose waves see no block, their
+    first, their first and last, or more of their blocks: against the oracle."""
+    from hs_guard.engine.kernels import ring_attention_v8
+    gen = torch.Generator().manual_seed(90 + G)
+    starts = torch.tensor([0, 1, 31, 32, 33, 64, 96, 100, 127, 128, 129, 160, 400, 512, 513, 1000])
+    N, Hkv, D, W, Lb = len(starts), 2, 256, 512, 16 // G
+    q = torch.randn(N, Hkv, G * Lb, D, generator=gen).to(torch.bfloat16)
+    ring_k, ring_v = (torch.randn(N, Hkv, W + 1, D, generator=gen).to(torch.bfloat16) for _ in range(2))
+    new_k = torch.randn(N, Hkv, Lb, D, generator=gen).to(torch.bfloat16)
+    value = torch.randn(N, Lb, Hkv * D, generator=gen).to(torch.bfloat16)
+    gate = torch.randn(N, Lb, Hkv * G * 2 * D, generator=gen).to(torch.bfloat16)
+    ring_pos = torch.full((N, W + 1), -1, dtype=torch.long)
+    for s, st in enumerate(starts.tolist()):
+        for p_ in range(max(0, st - W), st):
+            ring_pos[s, p_ % W] = p_
+    slots, lens = torch.arange(N), torch.tensor([Lb - n % 3 for n in range(N)])
+    dev = torch.device("cuda:0")
+    out = ring_attention_v8(*(t.to(dev) for t in (q, ring_k, ring_v, new_k, value, gate, ring_pos, slots, starts, lens)),
+                            D ** -0.5, W, False, split_k=False)
+    ref, _, _, _ = oring.ring_attention_v8(_np(q), _np(ring_k), _np(ring_v), _np(new_k), _np(value), _np(gate),
+                                           ring_pos.numpy(), slots.numpy(), starts.numpy(), lens.numpy(), D ** -0.5, W,
+                                           False)
+    _check(_np(out), ref)
