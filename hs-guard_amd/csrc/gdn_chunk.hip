@@ -692,20 +692,25 @@ __global__ __launch_bounds__(TRANS ? 256 : 512) void gdn_chunk_state_kernel(cons
   const int64_t srow = (int64_t)(4 * g4) * VD + vcol;   // this lane's first element of a [KD][VD] matrix
   f32x4 S[8];
   if (chain) {
+    // (a loop per source: with the choice inside, the fp16 state's loads were waited for one by one)
     const bool from_state = TRANS ? seg == 0 : sg.n_segs == 1;
-    const float* const bound = p.bound + (from_state ? 0 : matrix_at(p, n, hv, seg)) + srow;
+    if (from_state) {
 #pragma unroll
-    for (int mt = 0; mt < 8; ++mt)
+      for (int mt = 0; mt < 8; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t at = (int64_t)(16 * mt + r) * VD;
-        if (TRANS && !from_state)
-          S[mt][r] = identity && 16 * mt + 4 * g4 + r == vcol ? 1.f : 0.f;
-        else if (from_state)
-          S[mt][r] = load_state<ST>(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD);
-        else
-          S[mt][r] = bound[at];
-      }
+        for (int r = 0; r < 4; ++r) S[mt][r] = load_state<ST>(sbase + (int64_t)(16 * mt + 4 * g4 + r) * VD);
+    } else if constexpr (TRANS) {
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[mt][r] = identity && 16 * mt + 4 * g4 + r == vcol ? 1.f : 0.f;
+    } else {
+      const float* const bound = p.bound + matrix_at(p, n, hv, seg) + srow;
+#pragma unroll
+      for (int mt = 0; mt < 8; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[mt][r] = bound[(int64_t)(16 * mt + r) * VD];
+    }
     if (TRANS && seg == 0) {   // the output pass's start of segment 0: its last segment overwrites the row's state
       float* const start = p.bound + matrix_at(p, n, hv, 0) + srow;
 #pragma unroll
