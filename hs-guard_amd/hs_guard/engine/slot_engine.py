@@ -666,12 +666,16 @@ class SlotStreamEngine(PreparedWeights):
         piece = LONG_TOKENS // rows // 64 * 64
         return piece if piece >= 128 else 0
 
-    def _long_scratch(self, rows, piece):
-        """(activations, chunk workspace) of a long piece, or None where the card has no room for them (the step then
-        runs in ticks). Taken from the caching allocator for the length of the piece: an engine that only streams
-        keeps none."""
+    def _long_scratch(self, lens, piece):
+        """(activations, chunk workspace) of a long piece of rows of up to ``piece`` of ``lens`` tokens, or None where the
+        card has no room for them (the step then runs in ticks). Taken from the caching allocator for the length of the
+        piece, at its own size: an engine that only streams keeps none."""
+        take = [min(n, piece) for n in lens]
+        rows = min(len(take), self.max_rows)
+        total = max(sum(take[i:i + rows]) for i in range(0, len(take), rows))
         try:
-            return self._activations(LONG_TOKENS, rows), self._chunk_workspace(rows, piece)
+            return (self._activations(bucket(total, token_buckets(LONG_TOKENS)), rows),
+                    self._chunk_workspace(rows, max(take)))
         except torch.OutOfMemoryError:
             return None
 
@@ -805,9 +809,9 @@ class SlotStreamEngine(PreparedWeights):
         results = {role: [[] for _ in requests] for role in self.roles}
         pending = [(i, s, list(ids)) for i, (s, ids) in enumerate(requests)]
         while pending:
-            n = min(len(pending), rows)
-            piece = self._long_piece(n, max(len(ids) for _, _, ids in pending))
-            scratch = self._long_scratch(n, piece) if piece else None
+            lens = [len(ids) for _, _, ids in pending]
+            piece = self._long_piece(min(len(pending), rows), max(lens))
+            scratch = self._long_scratch(lens, piece) if piece else None
             take = piece if scratch else largest
             batch = [(i, s, ids[:take]) for i, s, ids in pending]
             for start in range(0, len(batch), rows):

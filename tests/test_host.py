@@ -274,3 +274,33 @@ def test_native_host_packing_matches_numpy_route():
     with pytest.raises(ValueError):
         _hostpack.scatter_padded(np.zeros((2, 4, 3), np.float32), 2, 4, np.array([3], np.int64),
                                  np.array([2], np.int64), 4, np.zeros((2, 1, 4, 3), np.float32))
+
+
+def test_long_piece_scratch_fits_its_piece():
+    """A long piece's scratch is sized by its rows' tokens (those of 4,096 for one row of 65 would be 50 times as much), and
+    holds every part of up to max_rows rows that the step cuts its pending rows into."""
+    import torch
+    from hs_guard._lib import lib
+    from hs_guard.engine.slot_engine import LONG_TOKENS, ROLES, SlotStreamEngine, bucket, gdn_proj_width, token_buckets
+    from hs_guard.model import GuardConfig
+    eng = SlotStreamEngine.__new__(SlotStreamEngine)
+    cfg = eng.cfg = GuardConfig.baseline()
+    eng.device, eng.roles, eng.chunk_min_tokens, eng.max_rows = torch.device("cpu"), ROLES, 16, 4
+    eng.gdn_in = gdn_proj_width(cfg)
+    eng.att_in = cfg.num_attention_heads * 2 * cfg.head_dim + 2 * cfg.num_key_value_heads * cfg.head_dim
+
+    def size(lens, piece):
+        buf, ws = eng._long_scratch(lens, piece)
+        take = [min(n, piece) for n in lens]
+        for i in range(0, len(take), eng.max_rows):
+            part = take[i:i + eng.max_rows]
+            tb = bucket(sum(part), token_buckets(LONG_TOKENS))
+            assert buf["hidden"].numel() >= tb * cfg.hidden_size and buf["proj"].numel() >= tb * eng.gdn_in
+            assert buf["inputs"].numel() >= 2 * tb + 4 * len(part) and buf["probs"].numel() >= len(ROLES) * tb * 3
+            assert ws.numel() >= lib().hsg_gdn_chunk_workspace_bytes(len(part), max(part), cfg.linear_num_value_heads)
+        return ws.numel() + sum(t.numel() * t.element_size() for t in buf.values())
+
+    full = size([9000], LONG_TOKENS)
+    assert size([65], LONG_TOKENS) * 25 <= full
+    assert size([900] * 3, 1344) < full and size([70, 3, 65, 1, 2000, 9], 1024) < full
+    assert size([LONG_TOKENS // 4] * 4, 1024) >= 100 << 20
