@@ -111,3 +111,39 @@ def oracle_whole(weights, cfg, ids, gemm=None, roles=("user", "assistant")):
                                           w[f"heads.{r}.projection.0.bias"], w[f"heads.{r}.projection.1.weight"],
                                           w[f"heads.{r}.projection.1.bias"], w[f"heads.{r}.risk.weight"],
                                           w[f"heads.{r}.risk.bias"], cfg.layer_norm_eps) for r in roles])
+
+
+# Pools of an engine whose contexts ran in long pieces against one that cut them into ticks, per slot and layer, as a
+# relative error (2-norm). The two differ by fp32 rounding and by the bf16 values that it makes round the other way: one in a
+# thousand of them is sqrt(1e-3) 2^-8 = 1e-4 of a bf16 pool, about half of it measured for the rings (whose inputs passed a GDN
+# layer; 2.5e-4 at most), 0 to 3e-9 for the conv history of layer 0 and 8e-6 for the fp32 states.
+POOL_BARS = {"conv": 2e-4, "rec": 1e-4, "ring_k": 8e-4, "ring_v": 8e-4}
+
+
+def pool_errors(got, ref, slots, window):
+    """Largest relative error over layers and ``slots`` of each pool of two engines (or oracles)."""
+    out = {}
+    for name in POOL_BARS:
+        a, b = (getattr(e, name) for e in (got, ref))
+        a, b = (x.double().cpu().numpy() if torch.is_tensor(x) else np.asarray(x, np.float64) for x in (a, b))
+        if name.startswith("ring"):
+            a, b = a[..., :window, :], b[..., :window, :]
+        out[name] = max(np.linalg.norm(a[i, s] - b[i, s]) / np.linalg.norm(b[i, s]) for i in range(len(a)) for s in slots)
+    return out
+
+
+LONG_PIECES = [[65], [900, 130, 1], [200] + [64] * 3 + [5] * 28]
+
+
+def long_piece_case(sizes):
+    """The 2-layer model and the three steps of the long-piece tests: contexts of ``sizes`` tokens, one more token each, a
+    second context of 70 tokens on slot 0 beside the others'. Returns (cfg, model on the CPU, steps)."""
+    from hs_guard.model import GuardConfig, GuardModel
+    cfg = GuardConfig(vocab_size=1000, hidden_size=1024, num_hidden_layers=2,
+                      layer_types=["linear_attention", "full_attention"], intermediate_size=1024,
+                      linear_num_key_heads=2, linear_num_value_heads=4, num_attention_heads=8,
+                      num_key_value_heads=2, window_tokens=96)
+    model = GuardModel.random(cfg, seed=1, device="cpu", std=0.005)
+    rng = np.random.default_rng(len(sizes))
+    return cfg, model, [[(s, rng.integers(0, cfg.vocab_size, n).tolist()) for s, n in enumerate(lens)]
+                        for lens in (sizes, [1] * len(sizes), [70] + sizes[1:])]

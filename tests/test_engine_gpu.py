@@ -20,6 +20,7 @@ kernel alone is held to 1e-3 in test_gdn_gpu.py).
 import numpy as np
 import pytest
 import torch
+from parity_helpers import LONG_PIECES, POOL_BARS, long_piece_case, pool_errors
 from parity_helpers import matched_gemm as _matched_gemm
 from parity_helpers import max_diff as _max_diff
 
@@ -474,24 +475,22 @@ def test_matched_engine_pools_match_oracle(setup2):
         assert rel < 1e-3, f"slot {s} state rel err {rel:.2e}"
 
 
-@pytest.mark.parametrize("sizes", [[65], [900, 130, 1], [200] + [64] * 3 + [5] * 28])
+@pytest.mark.parametrize("sizes", LONG_PIECES)
 def test_long_pieces_match_ticks(sizes):
     """Contexts in long pieces against the same engine cut into 64-token ticks, past the window, then one more tick and
     a second context on the live sessions. The two paths round their products and softmax blocks differently, so the
     probabilities agree to PROB_TOL at the weight scale where rounding alone moves them by 5e-4 (setup_small); lengths
-    and ring positions are equal."""
+    and ring positions are equal. After every step the sessions' pools agree within POOL_BARS, which a dropped row, a wrong
+    conv history, segment state or GDN output exceeds many times (tests/test_oracle_backbone.py), where the probabilities
+    move by less than PROB_TOL."""
     from hs_guard.engine.slot_engine import SlotStreamEngine
-    from hs_guard.model import GuardConfig, GuardModel
-    cfg = GuardConfig(vocab_size=1000, hidden_size=1024, num_hidden_layers=2,
-                      layer_types=["linear_attention", "full_attention"], intermediate_size=1024,
-                      linear_num_key_heads=2, linear_num_value_heads=4, num_attention_heads=8,
-                      num_key_value_heads=2, window_tokens=96)
-    model = GuardModel.random(cfg, seed=1, device="cpu", std=0.005).to("cuda:0")
+    cfg, model, steps = long_piece_case(sizes)
+    model = model.to("cuda:0")
     long, ticks = SlotStreamEngine(model, len(sizes) + 1), SlotStreamEngine(model, len(sizes) + 1)
     ticks._long_scratch = lambda rows, piece: None      # as on a card without room for the scratch
-    rng = np.random.default_rng(len(sizes))
-    for lens in (sizes, [1] * len(sizes), [70] + sizes[1:]):
-        reqs = [(s, rng.integers(0, cfg.vocab_size, n).tolist()) for s, n in enumerate(lens)]
+    slots = range(len(sizes))
+    for reqs in steps:
+        lens = [len(ids) for _, ids in reqs]
         before = long.stats["eager_steps"]
         a, b = long.step(reqs), ticks.step(reqs)
         assert (long.stats["eager_steps"] > before) == (max(lens) > 64)
@@ -499,6 +498,9 @@ def test_long_pieces_match_ticks(sizes):
             for x, y, n in zip(a[role], b[role], lens):
                 assert x.shape == y.shape == (n, 3)
                 assert float((x - y).abs().max()) <= PROB_TOL
+        errs = pool_errors(long, ticks, slots, cfg.window_tokens)
+        print("[engine] long piece pools", {k: f"{v:.1e}" for k, v in errs.items()}, flush=True)
+        assert all(errs[k] <= bar for k, bar in POOL_BARS.items()), errs
     assert ticks.stats["eager_steps"] == 0
     np.testing.assert_array_equal(long.length, ticks.length)
     assert torch.equal(long.ring_pos[:len(sizes)], ticks.ring_pos[:len(sizes)])

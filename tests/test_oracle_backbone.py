@@ -16,6 +16,8 @@ from oracle.bf16 import exact
 
 torch = pytest.importorskip("torch")
 
+from parity_helpers import LONG_PIECES, POOL_BARS, long_piece_case, pool_errors  # noqa: E402
+
 
 def _tiny_cfg():
     from hs_guard.model import GuardConfig
@@ -168,3 +170,39 @@ def test_noise_floor_scales_with_weights():
           f"(std 0.0025)")
     assert f2_small < 1e-3 and f24_small < 1e-3
     assert f2 > 2 * f2_small
+
+
+@pytest.mark.parametrize("sizes", LONG_PIECES)
+def test_long_piece_bars_see_planted_mistakes(sizes, monkeypatch):
+    """The pool bars of the long-piece tests (tests/test_engine_gpu.py) against mistakes planted in the oracle's first step:
+    GDN outputs of zero, a state, conv history or short row lost. Each exceeds a bar five times after that step or the
+    next."""
+    import oracle.gdn as ogdn
+    cfg, model, steps = long_piece_case(sizes)
+    w = {k: v.float().numpy() for k, v in model.weights.items()}
+    slots = range(len(sizes))
+
+    def run(change=None, first=steps[0]):
+        orc, pools = StreamOracle(w, cfg, len(sizes) + 1), []
+        for i, reqs in enumerate((first, steps[1])):
+            orc.step(reqs)
+            if i == 0 and change:
+                change(orc)
+            pools.append(StreamOracle.__new__(StreamOracle))
+            for name in POOL_BARS:
+                setattr(pools[-1], name, getattr(orc, name).copy())
+        return pools
+
+    def seen(pools):
+        errs = [pool_errors(a, b, slots, cfg.window_tokens) for a, b in zip(pools, right)]
+        return max(e[k] / POOL_BARS[k] for e in errs for k in POOL_BARS)
+
+    right = run()
+    assert seen(right) == 0
+    assert seen(run(lambda o: o.rec.fill(0))) > 5
+    assert seen(run(lambda o: o.conv.fill(0))) > 5
+    last = steps[0][-1]
+    assert seen(run(first=steps[0][:-1] + [(last[0], [(i + 1) % 1000 for i in last[1]])])) > 5   # the last row's own tokens lost
+    step = ogdn.gdn_slot_step
+    monkeypatch.setattr(ogdn, "gdn_slot_step", lambda *a, **k: (lambda o, sq, st: (o * 0, sq * 0, st))(*step(*a, **k)))
+    assert seen(run()) > 5
