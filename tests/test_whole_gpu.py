@@ -70,7 +70,7 @@ def test_whole_sequence_matched_gemms():
 
 
 def test_attention_segment_batches_agree(setup, monkeypatch):
-    """Splitting the attention's segments over several launches (as sequences longer than 8192 tokens do) gives
+    """Splitting the attention's segments over several launches (as sequences longer than 8,388,608 tokens do) gives
     the same result as one launch."""
     import hs_guard.engine.whole as whole
     cfg, model, _ = setup
