@@ -1034,7 +1034,9 @@ __global__ __launch_bounds__(TRANS ? 256 : 512) void gdn_chunk_state_kernel(cons
 // The states at the starts of a row's segments 2 on: bound[g + 1] holds B_g and becomes A_g bound[g] + B_g. One workgroup
 // per (row, head, 16 value columns); wave w owns rows 32 w .. 32 w + 31 of S, which the waves exchange through LDS. fp32
 // MFMA; the k order of a product is lane group g4's own four floats 16 j + 4 g4 + u, so A is read 16 bytes a lane. The
-// latency of each step's operands bounds it (20 us for the 6 steps of 8 segments; fetched a step ahead: 22 us).
+// latency of each step's operands bounds it (20 us for the 6 steps of 8 segments; fetched a step ahead: 22 us). Eight short
+// chains summed in pairs, not one of 32 products: the state of one row of 2,000 tokens (8 heads, slow decay) ends 1.798e-7 from
+// float64, 1.896e-7 with one chain, 1.800e-7 walked whole.
 constexpr int CS = 20;             // row stride (fp32) of S in LDS: rows 4 apart are 16 banks apart
 __global__ __launch_bounds__(256) void gdn_chunk_combine_kernel(const ChunkParams p) {
   __shared__ __align__(16) float Ss[2][KD * CS];
@@ -1071,15 +1073,19 @@ __global__ __launch_bounds__(256) void gdn_chunk_combine_kernel(const ChunkParam
     fetch(g);
     lds_barrier();   // S_g is in Ss[g & 1], and the reads of S_{g - 1} are done
     const float* const S = Ss[g & 1];
-    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    f32x4 part[2][8];   // eight chains of four products each, summed in pairs
 #pragma unroll
     for (int j = 0; j < 8; ++j)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const float sv = S[(16 * j + 4 * g4 + u) * CS + m16];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) acc[t] = mmf4(a[t][j][u], sv, acc[t]);
+        for (int t = 0; t < 2; ++t) part[t][j] = mmf4(a[t][j][u], sv, u ? part[t][j] : (f32x4){0.f, 0.f, 0.f, 0.f});
       }
+    f32x4 acc[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      acc[t] = ((part[t][0] + part[t][1]) + (part[t][2] + part[t][3])) + ((part[t][4] + part[t][5]) + (part[t][6] + part[t][7]));
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll

@@ -362,3 +362,44 @@ def test_segments_match_whole_rows(HV, lens, state_dtype, padded):
         assert errs[0][0] <= 1.5 * errs[1][0] + 1e-6
     unused = [s for s in range(N + 1) if s not in slots.tolist()]
     np.testing.assert_array_equal(got[0][1][unused], _np(state0[unused]))
+
+
+def _recurrence_f64(packed, a, b, A_log, dt, S0, H, K):
+    """Final state of one row in float64 on the GPU (H value heads, each with its own key head), token by token."""
+    x = packed.double()
+    k, v = (x[:, i * H * K:(i + 1) * H * K].view(-1, H, K) for i in (1, 2))
+    k = k / torch.sqrt((k * k).sum(-1, keepdim=True) + 1e-6)
+    decay = torch.exp(-torch.exp(A_log.double()) * torch.nn.functional.softplus(a.double() + dt.double(), threshold=100))
+    beta = torch.sigmoid(b.double())
+    S = S0.double().clone()
+    for t in range(len(x)):
+        S *= decay[t][:, None, None]
+        kv = torch.bmm(k[t][:, None], S)[:, 0]
+        S += k[t][:, :, None] * (beta[t][:, None] * (v[t] - kv))[:, None]
+    return S
+
+
+@pytest.mark.parametrize("T,H,A_mean,dt_mean", [(2000, 8, -3.0, -3.0), (1100, 16, -3.0, -3.0), (2000, 8, -0.5, 0.0)])
+def test_segments_lose_no_precision(T, H, A_mean, dt_mean):
+    """Rows in segments end no further from the float64 recurrence than walked whole: the state's error over four seeds
+    (about 1.8e-7 where decay is slow and segments matter most; a seed's moves by 1 %) to 2 %."""
+    from hs_guard._lib import lib
+    from hs_guard.engine.kernels import gdn_chunk_prefill
+    dev, K = torch.device("cuda:0"), 128
+    base = lib().hsg_gdn_chunk_workspace_bytes(1, T, H)
+    assert lib().hsg_gdn_chunk_segment_workspace_bytes(1, T, H) > base
+    err = [0.0, 0.0]
+    for seed in range(4):
+        gen = torch.Generator(device=dev).manual_seed(seed)
+        packed, a, b, A_log, dt = (torch.randn(*n, generator=gen, device=dev) for n in ((T, 3 * H * K), (T, H), (T, H), (H,), (H,)))
+        packed, a, b = (t.to(torch.bfloat16) for t in (packed, a, b))
+        A_log, dt = (A_log * 0.3 + A_mean).to(torch.bfloat16), (dt * 0.3 + dt_mean).to(torch.bfloat16)
+        state0 = torch.randn(1, H, K, K, generator=gen, device=dev) * 0.05
+        ref = _recurrence_f64(packed, a, b, A_log, dt, state0[0], H, K)
+        for i, ws in enumerate((None, torch.empty(base, dtype=torch.uint8, device=dev))):
+            state = state0.clone()
+            gdn_chunk_prefill(packed, H * K, H, K, H, K, a, b, A_log, dt, state, torch.zeros(1, dtype=torch.long, device=dev),
+                              torch.tensor([T], device=dev), torch.zeros(1, dtype=torch.long, device=dev), workspace=ws)
+            err[i] += float((state[0].double() - ref).norm() / ref.norm()) / 4
+    print(f"[chunk] T={T} H={H}: state error segments {err[0]:.4e} whole {err[1]:.4e}", flush=True)
+    assert err[0] <= 1.02 * err[1]
