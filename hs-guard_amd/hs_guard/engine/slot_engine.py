@@ -30,6 +30,7 @@ from .._lib import HSG_ERR_SHAPE, HSG_GDN_BURST_MIN_DEFAULT, HSG_GEMM_SKINNY_M_M
 from ..model import ROLES, GuardModel
 from .gemm_plan import WORKSPACE_BYTES as GEMM_WORKSPACE_BYTES
 from .gemm_plan import GemmPlans
+from .kernels import _stream
 
 SESSION_BUCKETS = (1, 2, 4, 8, 16, 32, 48, 64, 96, 128, 160, 192, 224, 256, 320, 352, 384, 448, 512)
 STATE_DTYPES = {"float32": torch.float32, "float16": torch.float16}
@@ -303,7 +304,7 @@ class SlotStreamEngine(PreparedWeights):
         N = w.shape[0]
         if w.shape[1] != K or out.shape != (M, N) or x.stride(1) != 1 or w.stride(1) != 1 or out.stride(1) != 1:
             raise ValueError("mm: shapes or strides do not match D[M, N] = A[M, K] . W[N, K]^T")
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = _stream(x)
         if self._skinny(x, w, K):
             check(calls().hsg_gemm_bf16_skinny(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(),
                                                out.stride(0), M, N, K, stream), "hsg_gemm_bf16_skinny")
@@ -335,7 +336,7 @@ class SlotStreamEngine(PreparedWeights):
         M, I = gu.shape[0], gu.shape[1] // 2
         if w.shape[1] != I or out.shape != (M, w.shape[0]) or gu.stride(1) != 1 or out.stride(1) != 1:
             raise ValueError("mm_silu: shapes or strides do not match")
-        stream = torch.cuda.current_stream(self.device).cuda_stream
+        stream = _stream(gu)
         if self._skinny(gu, w, I) and w.stride(1) == 1:
             check(calls().hsg_gemm_bf16_skinny_silu(gu.data_ptr(), gu.stride(0), w.data_ptr(), w.stride(0),
                                                     out.data_ptr(), out.stride(0), M, w.shape[0], I, stream),
@@ -411,7 +412,7 @@ class SlotStreamEngine(PreparedWeights):
             return self._view_of(buf, name, *shape)
 
         cfg = self.cfg
-        st = torch.cuda.current_stream(self.device).cuda_stream
+        st = _stream(self.emb)
         H, W = cfg.hidden_size, self.window
         S = self.max_slots + 1
         eps = cfg.rms_norm_eps
