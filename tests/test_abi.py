@@ -152,3 +152,12 @@ def test_native_calls_take_the_same_arguments():
         calls().hsg_add_square(None, None, None, None, 1, 1 << 40, None)
     with pytest.raises(TypeError):
         calls().hsg_add_square(None, None, None, None, 1, "4", None)
+
+
+def test_contract_glue_refuses_more_threads_than_a_launch_holds():
+    """2^32 elements at one per thread (an unaligned pointer) are refused on the host, before a launch (placeholder pointers,
+    never read)."""
+    from hs_guard._lib import HSG_ERR_SHAPE, lib
+    L = lib()
+    assert L.hsg_silu_mul_pair(2, 2, 2, 1 << 32, None) == HSG_ERR_SHAPE
+    assert L.hsg_add_square(2, 2, 2, 4, 1 << 20, 1 << 12, None) == HSG_ERR_SHAPE
